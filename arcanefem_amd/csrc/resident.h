@@ -1,0 +1,85 @@
+// resident.h -- conjugate gradients of scalar systems in one launch: the
+// vectors live in registers and LDS, the matrix in a pair layout read by wide
+// loads, and the workgroups meet at barriers in device memory.
+#pragma once
+
+#include "common.h"
+
+namespace afem {
+namespace resident {
+
+// Pair layout of a scalar matrix: slices of 64 rows; the off-diagonal entries
+// of a row, in CSR order, fill pairs, and pair q of lane l of slice s is at
+// (poff[s] + q) * 64 + l (values as two consecutive numbers, column offsets
+// col - row as two consecutive 16- or 32-bit integers; padding: value 0,
+// offset 0).  The diagonal entries are an array of their own.  Slices start
+// at the first row of every segment.
+struct Pack
+{
+  int32_t n = 0, nslice = 0, max_len = 0;
+  int64_t npair = 0;
+  bool idx16 = false;
+  bool all_diag = false;            // every non-empty row has its diagonal entry
+  std::vector<int32_t> seg_rows;    // row offsets of the segments
+  std::vector<int32_t> seg_slices;  // first slice of each segment (nb_seg + 1)
+  DBuf<int32_t> slice_row;          // per slice its first row, then the end row of its segment
+  DBuf<int32_t> poff;               // nslice + 1
+  DBuf<int32_t> idx;                // 64 * npair (16-bit offsets) or 128 * npair words
+  DBuf<double> v64, diag64, dinv64; // 128 * npair values; n
+  DBuf<float> v32, diag32, dinv32;  // difference form: off-diagonal entries rounded, diag32 the row sum
+  bool valid64 = false, valid32 = false;
+};
+
+// Offsets of a pattern (rows rp, columns ci) cut into segments.  False: the
+// segments do not fit the device at once, or the layout pads too much.
+bool pack_pattern(Pack& p, int32_t n, int64_t nnz, const int32_t* rp, const int32_t* ci,
+                  const std::vector<int32_t>& seg_rows);
+// Values of the pattern's matrix: FP64, and with want32 the FP32 difference form too.
+void pack_values(Pack& p, const int32_t* rp, const int32_t* ci, const double* v, bool want32);
+
+struct Status // of one segment
+{
+  double rtol2, atol2, delta2;      // in
+  int max_iter, active;             // in; active 0: the segment is left alone
+  double bb, tol2, rr_out, rr_true, rho, rr_ref, beta;
+  int iter, done, converged, breakdown, nb_ru;
+  unsigned epoch;                   // barriers taken since the slots were cleared
+};
+
+struct Options
+{
+  bool mixed = false;   // FP32 vectors and products, FP64 x and reliable updates
+  bool precond = true;  // Jacobi
+  int norm = 0;         // stopping norm of afem_solver_options
+  long long spin_limit = 0;
+};
+
+// Work arrays kept by a solver: published vector, saved vectors, barrier slots.
+struct Work
+{
+  DBuf<double> u;          // published vector (FP64, or FP32 in the same storage)
+  DBuf<double> keep;       // r, p, s between launches
+  DBuf<uint64_t> slots;
+  DBuf<int32_t> team;      // layout of the launch
+  DBuf<Status> st;         // one per segment, then the abort flag
+  Status* host = nullptr;  // pinned, nb_seg + 1
+  int nseg = 0;
+  unsigned epoch = 0;      // largest epoch in the slots
+  std::vector<int32_t> layout_rows;
+  int grid = 0, rows_per_wave = 0;
+  ~Work()
+  {
+    if (host)
+      (void)hipHostFree(host);
+  }
+};
+
+// Runs the segments of w.host (inputs set, x the starting point) to their end;
+// w.host holds the results.  False: a barrier wait gave up (x is then some
+// iterate of each segment).
+bool solve(const Pack& p, Work& w, const Options& o, double* x, const double* b);
+// Makes room for the statuses of nseg segments.
+void reserve(Work& w, int nseg);
+
+} // namespace resident
+} // namespace afem

@@ -1,0 +1,422 @@
+// resident.hip -- set-up and host side of the resident conjugate gradients
+// (resident_kernel.h): the pair layout of a matrix and the launch layout.
+//
+// Why one launch: with three kernels an iteration of a system that fits the
+// caches is bound by launches and by the latencies at each kernel's start
+// (state, partial sums, vectors from memory), about 5 us a kernel whatever it
+// does; larger systems move every vector through memory 11 times an
+// iteration.  Here an iteration is two barriers of 2-3 us and the matrix.
+// FP64 Jacobi-PCG, MI355X, three kernels -> resident: 256 x 256 quads of two
+// triangles (66049 rows) 16.3 -> 6.9 us an iteration; 48 x 52 x 45 nodes of
+// tetrahedra numbered at random (112 thousand rows) 22 -> 15.5 us.
+#include "resident_kernel.h"
+
+#include <algorithm>
+#include <cmath>
+
+namespace afem {
+namespace resident {
+
+// ---- pair layout --------------------------------------------------------------------------------
+//
+// One wave per slice.  The slice's rows are one contiguous range of the CSR
+// arrays: it is read coalesced into LDS and each lane walks its row there
+// (ranges that exceed the LDS space are walked in place).
+
+constexpr int kStageMax = 4096; // entries of a slice staged in LDS
+
+__device__ __forceinline__ void slice_rows(const int32_t* __restrict__ slice_row, int32_t nslice, int32_t s,
+                                           const int32_t* __restrict__ rp, int lane, int32_t& row, bool& live,
+                                           int32_t& b, int32_t& e, int32_t& e0, int32_t& e1)
+{
+  const int32_t r0 = slice_row[s], r1 = min(slice_row[nslice + s], r0 + 64);
+  row = r0 + lane;
+  live = row < r1;
+  e0 = rp[r0];
+  e1 = rp[r1];
+  b = live ? rp[row] : e1;
+  e = live ? rp[row + 1] : e1;
+}
+
+// Pairs of every slice, and over the matrix: the longest row, the largest
+// |column - row|, whether a non-empty row lacks its diagonal entry.
+__global__ void __launch_bounds__(64)
+k_pair_count(int32_t nslice, const int32_t* __restrict__ slice_row, const int32_t* __restrict__ rp,
+             const int32_t* __restrict__ ci, int32_t* __restrict__ width, int32_t* __restrict__ stats)
+{
+  __shared__ int32_t s_col[kStageMax];
+  const int32_t s = blockIdx.x;
+  const int lane = threadIdx.x;
+  int32_t row, b, e, e0, e1;
+  bool live;
+  slice_rows(slice_row, nslice, s, rp, lane, row, live, b, e, e0, e1);
+  const bool staged = e1 - e0 <= kStageMax;
+  if (staged) {
+    for (int32_t k = e0 + lane; k < e1; k += 64)
+      s_col[k - e0] = ci[k];
+    __syncthreads();
+  }
+  int32_t off = 0, far = 0;
+  for (int32_t k = b; k < e; ++k) {
+    const int32_t c = staged ? s_col[k - e0] : ci[k];
+    off += c != row ? 1 : 0;
+    far = max(far, abs(c - row));
+  }
+  int32_t pairs = (off + 1) / 2, len = e - b, lacks = (e > b && off == e - b) ? 1 : 0;
+#pragma unroll
+  for (int o = 32; o; o >>= 1) {
+    pairs = max(pairs, __shfl_xor(pairs, o, 64));
+    len = max(len, __shfl_xor(len, o, 64));
+    far = max(far, __shfl_xor(far, o, 64));
+    lacks = max(lacks, __shfl_xor(lacks, o, 64));
+  }
+  if (lane == 0) {
+    width[s] = pairs;
+    // a look first: almost every slice leaves the maxima as they are
+    if (len > __hip_atomic_load(stats, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(stats, len);
+    if (far > __hip_atomic_load(stats + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(stats + 1, far);
+    if (lacks)
+      atomicMax(stats + 2, 1);
+  }
+}
+
+template <class I>
+__global__ void __launch_bounds__(64)
+k_pair_index(int32_t nslice, const int32_t* __restrict__ slice_row, const int32_t* __restrict__ rp,
+             const int32_t* __restrict__ ci, const int32_t* __restrict__ poff, I* __restrict__ idx)
+{
+  typedef I I2 __attribute__((ext_vector_type(2)));
+  __shared__ int32_t s_col[kStageMax];
+  const int32_t s = blockIdx.x;
+  const int lane = threadIdx.x;
+  int32_t row, b, e, e0, e1;
+  bool live;
+  slice_rows(slice_row, nslice, s, rp, lane, row, live, b, e, e0, e1);
+  const bool staged = e1 - e0 <= kStageMax;
+  if (staged) {
+    for (int32_t k = e0 + lane; k < e1; k += 64)
+      s_col[k - e0] = ci[k];
+    __syncthreads();
+  }
+  int32_t k = b;
+  auto next = [&]() -> I { // offset of the row's next off-diagonal entry, 0 past the end
+    while (k < e) {
+      const int32_t c = staged ? s_col[k - e0] : ci[k];
+      ++k;
+      if (c != row)
+        return (I)(c - row);
+    }
+    return (I)0;
+  };
+  I2* out = reinterpret_cast<I2*>(idx) + (int64_t)poff[s] * 64 + lane;
+  const int w = poff[s + 1] - poff[s];
+  for (int q = 0; q < w; ++q) {
+    I2 d;
+    d.x = next();
+    d.y = next();
+    out[(int64_t)q * 64] = d;
+  }
+}
+
+// FP64 pairs, diagonal and its inverse, and (WANT32) the FP32 difference
+// form: off-diagonal entries rounded, diag32 the row sum taken in FP64, so
+// that y_i = diag32_i x_i + sum a_ij (x_j - x_i) has no rounded diagonal
+// cancelling the other terms on smooth vectors.
+template <bool WANT32>
+__global__ void __launch_bounds__(64)
+k_pair_values(int32_t nslice, const int32_t* __restrict__ slice_row, const int32_t* __restrict__ rp,
+              const int32_t* __restrict__ ci, const double* __restrict__ v, const int32_t* __restrict__ poff,
+              int stage, double* __restrict__ v64, double* __restrict__ diag64, double* __restrict__ dinv64,
+              float* __restrict__ v32, float* __restrict__ diag32, float* __restrict__ dinv32)
+{
+  typedef double d2 __attribute__((ext_vector_type(2)));
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  extern __shared__ __align__(16) unsigned char smem[]; // stage values, then stage columns
+  double* s_val = reinterpret_cast<double*>(smem);
+  int32_t* s_col = reinterpret_cast<int32_t*>(s_val + stage);
+  const int32_t s = blockIdx.x;
+  const int lane = threadIdx.x;
+  int32_t row, b, e, e0, e1;
+  bool live;
+  slice_rows(slice_row, nslice, s, rp, lane, row, live, b, e, e0, e1);
+  const bool staged = e1 - e0 <= stage;
+  if (staged) {
+    for (int32_t k = e0 + lane; k < e1; k += 64) {
+      s_val[k - e0] = v[k];
+      s_col[k - e0] = ci[k];
+    }
+    __syncthreads();
+  }
+  double diag = 0.0, sum = 0.0;
+  int32_t k = b;
+  auto next = [&]() -> double {
+    while (k < e) {
+      const int32_t c = staged ? s_col[k - e0] : ci[k];
+      const double a = staged ? s_val[k - e0] : v[k];
+      ++k;
+      sum += a;
+      if (c != row)
+        return a;
+      diag += a;
+    }
+    return 0.0;
+  };
+  const int64_t at = (int64_t)poff[s] * 64 + lane;
+  const int w = poff[s + 1] - poff[s];
+  for (int q = 0; q < w; ++q) {
+    d2 m;
+    m.x = next();
+    m.y = next();
+    reinterpret_cast<d2*>(v64)[at + (int64_t)q * 64] = m;
+    if constexpr (WANT32)
+      reinterpret_cast<f2*>(v32)[at + (int64_t)q * 64] = f2{ (float)m.x, (float)m.y };
+  }
+  (void)next(); // a diagonal entry after the last off-diagonal one
+  if (live) {
+    const double inv = diag != 0.0 ? 1.0 / diag : 1.0;
+    diag64[row] = diag;
+    dinv64[row] = inv;
+    if constexpr (WANT32) {
+      diag32[row] = (float)sum;
+      dinv32[row] = (float)inv;
+    }
+  }
+}
+
+// ---- launch layout ------------------------------------------------------------------------------
+
+constexpr int kMaxRows = kRowSteps[3];
+constexpr int kLaunchIterations = 8192; // iterations of one launch: a second or less at any size
+
+// Workgroups per segment: at least as many as its slices need with kMaxRows
+// per wave, at most one slice per wave, else in proportion to rows^1.5 (the
+// work of an iteration times the growth of the iteration count).  Empty: the
+// segments do not fit the device together.
+static std::vector<int32_t> team_sizes(const Pack& p, int budget)
+{
+  const int ns = (int)p.seg_rows.size() - 1;
+  std::vector<int32_t> least(ns), most(ns), m(ns);
+  std::vector<double> w(ns);
+  int64_t need = 0;
+  double wsum = 0.0;
+  for (int k = 0; k < ns; ++k) {
+    const int32_t sl = p.seg_slices[k + 1] - p.seg_slices[k];
+    least[k] = (sl + kWaves * kMaxRows - 1) / (kWaves * kMaxRows);
+    most[k] = (sl + kWaves - 1) / kWaves;
+    w[k] = std::pow((double)(p.seg_rows[k + 1] - p.seg_rows[k]), 1.5);
+    wsum += w[k];
+    need += least[k];
+  }
+  if (need > budget)
+    return {};
+  for (double scale = budget;; scale *= 0.97) {
+    int64_t total = 0;
+    for (int k = 0; k < ns; ++k) {
+      m[k] = std::max(least[k], std::min<int32_t>(most[k], (int32_t)std::floor(scale * w[k] / wsum)));
+      total += m[k];
+    }
+    if (total <= budget)
+      return m;
+  }
+}
+
+// ---- building the pair layout -------------------------------------------------------------------
+
+bool pack_pattern(Pack& p, int32_t n, int64_t nnz, const int32_t* rp, const int32_t* ci,
+                  const std::vector<int32_t>& seg_rows)
+{
+  p.n = n;
+  p.valid64 = p.valid32 = false;
+  p.seg_rows = seg_rows;
+  const int nseg = (int)seg_rows.size() - 1;
+  p.seg_slices.assign(nseg + 1, 0);
+  for (int k = 0; k < nseg; ++k)
+    p.seg_slices[k + 1] = p.seg_slices[k] + (seg_rows[k + 1] - seg_rows[k] + 63) / 64;
+  p.nslice = p.seg_slices[nseg];
+  if (team_sizes(p, rt().num_cu).empty())
+    return false;
+  std::vector<int32_t> sr((size_t)2 * p.nslice);
+  for (int k = 0; k < nseg; ++k)
+    for (int32_t s = p.seg_slices[k]; s < p.seg_slices[k + 1]; ++s) {
+      sr[s] = seg_rows[k] + 64 * (s - p.seg_slices[k]);
+      sr[(size_t)p.nslice + s] = seg_rows[k + 1];
+    }
+  p.slice_row.reserve(sr.size());
+  p.slice_row.upload(sr.data(), sr.size());
+  DBuf<int32_t> width((size_t)p.nslice), stats(3);
+  stats.zero();
+  hipLaunchKernelGGL(k_pair_count, dim3(p.nslice), dim3(64), 0, stream(), p.nslice, p.slice_row.p, rp, ci, width.p,
+                     stats.p);
+  check_launch("pair_count");
+  p.poff.reserve((size_t)p.nslice + 1);
+  p.npair = exclusive_scan_i32(width.p, p.poff.p, p.nslice);
+  int32_t h[3];
+  stats.download(h, 3);
+  // a few long rows would pad their slices many times over, and the kernel's
+  // stream offsets are 31 bits wide
+  if (p.npair * 128 > 4 * nnz + 65536 || p.npair * (kWave * 16) >= (1LL << 31))
+    return false;
+  p.max_len = h[0];
+  p.idx16 = h[1] <= 32767;
+  p.all_diag = h[2] == 0;
+  p.idx.reserve((size_t)p.npair * (p.idx16 ? 64 : 128));
+  p.v64.reserve((size_t)p.npair * 128);
+  p.diag64.reserve((size_t)n);
+  p.dinv64.reserve((size_t)n);
+  if (p.npair > 0) {
+    if (p.idx16)
+      hipLaunchKernelGGL(k_pair_index<int16_t>, dim3(p.nslice), dim3(64), 0, stream(), p.nslice, p.slice_row.p, rp,
+                         ci, p.poff.p, reinterpret_cast<int16_t*>(p.idx.p));
+    else
+      hipLaunchKernelGGL(k_pair_index<int32_t>, dim3(p.nslice), dim3(64), 0, stream(), p.nslice, p.slice_row.p, rp,
+                         ci, p.poff.p, p.idx.p);
+    check_launch("pair_index");
+  }
+  return true;
+}
+
+void pack_values(Pack& p, const int32_t* rp, const int32_t* ci, const double* v, bool want32)
+{
+  if (p.valid64 && (p.valid32 || !want32))
+    return;
+  if (want32) {
+    p.v32.reserve((size_t)p.npair * 128);
+    p.diag32.reserve((size_t)p.n);
+    p.dinv32.reserve((size_t)p.n);
+  }
+  const int stage = std::min(kStageMax, std::max(1, p.max_len) * 64);
+  const size_t lds = (size_t)stage * 12;
+  if (want32)
+    hipLaunchKernelGGL(k_pair_values<true>, dim3(p.nslice), dim3(64), lds, stream(), p.nslice, p.slice_row.p, rp, ci,
+                       v, p.poff.p, stage, p.v64.p, p.diag64.p, p.dinv64.p, p.v32.p, p.diag32.p, p.dinv32.p);
+  else
+    hipLaunchKernelGGL(k_pair_values<false>, dim3(p.nslice), dim3(64), lds, stream(), p.nslice, p.slice_row.p, rp, ci,
+                       v, p.poff.p, stage, p.v64.p, p.diag64.p, p.dinv64.p, (float*)nullptr, (float*)nullptr,
+                       (float*)nullptr);
+  check_launch("pair_values");
+  p.valid64 = true;
+  p.valid32 = p.valid32 || want32;
+}
+
+void reserve(Work& w, int nseg)
+{
+  if (w.nseg >= nseg && w.host)
+    return;
+  if (w.host)
+    AFEM_HIP(hipHostFree(w.host));
+  w.host = nullptr;
+  AFEM_HIP(hipHostMalloc(reinterpret_cast<void**>(&w.host), sizeof(Status) * ((size_t)nseg + 1),
+                         hipHostMallocDefault));
+  w.st.alloc((size_t)nseg + 1);
+  w.nseg = nseg;
+}
+
+__global__ void k_clear_slots(int64_t n, uint64_t* __restrict__ slots)
+{
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+    slots[i] = 0;
+}
+
+static void layout(const Pack& p, Work& w)
+{
+  if (w.grid > 0 && w.layout_rows == p.seg_rows)
+    return;
+  const std::vector<int32_t> m = team_sizes(p, rt().num_cu);
+  AFEM_REQUIRE(!m.empty(), AFEM_ERR_CAPACITY, "the systems do not fit the device at once");
+  const int ns = (int)m.size();
+  std::vector<int32_t> out;
+  int grid = 0, rows = 1;
+  for (int k = 0; k < ns; ++k) {
+    const int32_t sl = p.seg_slices[k + 1] - p.seg_slices[k];
+    const TeamDesc t{ p.seg_rows[k], p.seg_rows[k + 1], p.seg_slices[k], sl, grid, m[k], k, 0 };
+    const int32_t* q = reinterpret_cast<const int32_t*>(&t);
+    out.insert(out.end(), q, q + sizeof(TeamDesc) / sizeof(int32_t));
+    const int per_wg = (sl + m[k] - 1) / m[k];
+    rows = std::max(rows, (per_wg + kWaves - 1) / kWaves);
+    grid += m[k];
+  }
+  for (int k = 0; k < ns; ++k)
+    out.insert(out.end(), (size_t)m[k], k);
+  w.team.reserve(out.size());
+  w.team.upload(out.data(), out.size());
+  w.grid = grid;
+  w.rows_per_wave = *std::find_if(std::begin(kRowSteps), std::end(kRowSteps), [&](int r) { return r >= rows; });
+  w.layout_rows = p.seg_rows;
+}
+
+bool solve(const Pack& p, Work& w, const Options& o, double* x, const double* b)
+{
+  const int ns = (int)p.seg_rows.size() - 1;
+  layout(p, w);
+  w.u.reserve((size_t)p.n);
+  w.keep.reserve((size_t)3 * p.n);
+  const size_t slot_words = (size_t)2 * w.grid * kSlotWords;
+  if (w.slots.n < slot_words || w.epoch > 0x40000000u) {
+    w.slots.reserve(slot_words);
+    hipLaunchKernelGGL(k_clear_slots, dim3(64), dim3(256), 0, stream(), (int64_t)w.slots.n, w.slots.p);
+    check_launch("resident_clear");
+    w.epoch = 0;
+  }
+  Args a{};
+  a.team = reinterpret_cast<const TeamDesc*>(w.team.p);
+  a.team_of = w.team.p + (size_t)ns * (sizeof(TeamDesc) / sizeof(int32_t));
+  a.poff = p.poff.p;
+  a.idx = p.idx.p;
+  a.v = o.mixed ? (const void*)p.v32.p : (const void*)p.v64.p;
+  a.diag = o.mixed ? (const void*)p.diag32.p : (const void*)p.diag64.p;
+  a.dinv = o.mixed ? (const void*)p.dinv32.p : (const void*)p.dinv64.p;
+  a.v64 = p.v64.p;
+  a.diag64 = p.diag64.p;
+  a.x = x;
+  a.b = b;
+  a.u = w.u.p;
+  a.keep = w.keep.p;
+  a.n = p.n;
+  a.slots = w.slots.p;
+  a.st = w.st.p;
+  a.abort_flag = &w.st.p[ns].done;
+  a.spin_limit = o.spin_limit > 0 ? o.spin_limit : (1LL << 22);
+  a.precond = o.precond ? 1 : 0;
+  a.norm = o.norm;
+  a.max_launch_iter = kLaunchIterations;
+  const size_t lds = (size_t)w.rows_per_wave * kBS * 16; // x, and D^-1 (FP64) or p (mixed)
+  for (int k = 0; k < ns; ++k) {
+    Status& s = w.host[k];
+    s.iter = s.done = s.converged = s.breakdown = s.nb_ru = 0;
+    s.bb = s.rr_out = s.rr_true = s.rho = s.rr_ref = s.beta = 0.0;
+  }
+  for (;;) {
+    w.host[ns] = Status{};
+    for (int k = 0; k < ns; ++k)
+      w.host[k].epoch = w.epoch;
+    AFEM_HIP(hipMemcpyAsync(w.st.p, w.host, sizeof(Status) * ((size_t)ns + 1), hipMemcpyHostToDevice, stream()));
+    {
+      ProfScope prof(o.mixed ? "resident_cg_mixed" : "resident_cg_fp64");
+      launch_f64(a, w.rows_per_wave, p.idx16, w.grid, lds);
+    }
+    AFEM_HIP(hipMemcpyAsync(w.host, w.st.p, sizeof(Status) * ((size_t)ns + 1), hipMemcpyDeviceToHost, stream()));
+    AFEM_HIP(hipStreamSynchronize(stream()));
+    if (w.host[ns].done) { // a wait gave up: slots of unknown epochs
+      w.slots.release();
+      return false;
+    }
+    bool all = true;
+    for (int k = 0; k < ns; ++k) {
+      w.epoch = std::max(w.epoch, w.host[k].epoch);
+      all = all && (!w.host[k].active || w.host[k].done);
+    }
+    if (all)
+      return true;
+    a.resume = 1;
+  }
+}
+
+void launch_f64(const Args& a, int rows, bool idx16, int grid, size_t lds)
+{
+  launch_kernel<double>(a, rows, idx16, grid, lds);
+}
+
+} // namespace resident
+} // namespace afem

@@ -20,6 +20,9 @@
 // in FP64; only the FP64 residual of a reliable update can declare
 // convergence.  Dots are accumulated in FP64.
 //
+// Scalar FP64 solves without a pinned SpMV format run in one launch instead
+// (resident.hip) when the system fits the chip.
+//
 // SpMV formats: CSR with G lanes per row (wavefront-group row reductions) and
 // SELL-64 (slices of 64 rows stored column-major, one lane per row, fully
 // coalesced value/column streams), scalar or with 3x3 blocks.  The first
@@ -27,6 +30,7 @@
 #include "common.h"
 #include "device_utils.h"
 #include "linsys.h"
+#include "resident.h"
 
 #include <chrono>
 #include <type_traits>
@@ -1416,6 +1420,11 @@ struct afem_solver_ws
   bool has_spai = false;
   bool spai_sell_valid = false;
   bool spai_bf16_valid = false;
+  // resident solves (resident.hip): their own copy of the matrix
+  afem::resident::Pack pack;
+  afem::resident::Work rwork;
+  bool pack_valid = false;  // the pattern's layout is built
+  bool pack_usable = false; // and the resident kernel takes it
   ~afem_solver_ws()
   {
     if (host_st)
@@ -1479,6 +1488,7 @@ static afem_solver_ws* workspace(afem_system* s)
     w->unr32 = 0;
     w->has_spai = false;
     w->spai_sell_valid = false;
+    w->pack_valid = false;
   }
   if (!w->parts.p) {
     w->parts.alloc((size_t)9 * kMaxBlocks);
@@ -1498,9 +1508,11 @@ static afem_solver_ws* workspace(afem_system* s)
     w->unr32 = 0;
     w->has_spai = false;
     w->spai_sell_valid = false;
+    w->pack_valid = false;
   }
   if (s->matrix_changed) {
     w->values_valid = false;
+    w->pack.valid64 = w->pack.valid32 = false;
     s->matrix_changed = false;
   }
   return w;
@@ -2042,7 +2054,57 @@ static void launch_flex_iteration(afem_system* s, afem_solver_ws* w, int k, cons
   }
 }
 
-static int solve(afem_system* s, const afem_solver_options& o, afem_solve_result* res)
+// The resident kernel runs scalar FP64 CG and Jacobi-PCG on systems
+// whose vectors fit the device's registers and LDS (2.2 million rows on 256
+// CUs), unless the caller pinned an SpMV format.
+static bool resident_usable(afem_system* s, afem_solver_ws* w, const afem_solver_options& o)
+{
+  if (s->block != 1 || (o.method != AFEM_SOLVER_PCG_FP64 && o.method != AFEM_SOLVER_CG_FP64) || o.spmv_lanes != 0 || w->forced_format)
+    return false;
+  if (!w->pack_valid) {
+    w->pack_usable = resident::pack_pattern(w->pack, s->nb_dof, s->nnz, s->row_index, s->columns, { 0, s->nb_dof });
+    w->pack_valid = true;
+  }
+  return w->pack_usable;
+}
+
+// False: a barrier wait gave up (x is some iterate).
+static bool solve_resident(afem_system* s, afem_solver_ws* w, const afem_solver_options& o, afem_solve_result& res)
+{
+  const bool mixed = o.method == AFEM_SOLVER_PCG_MIXED;
+  const double delta = o.reliable_delta > 0.0 ? o.reliable_delta : 0.1;
+  resident::pack_values(w->pack, s->row_index, s->columns, s->values, mixed);
+  resident::Options ro;
+  ro.mixed = mixed;
+  ro.precond = o.method != AFEM_SOLVER_CG_FP64 && o.preconditioner != AFEM_PRECOND_NONE;
+  ro.norm = o.norm;
+  resident::reserve(w->rwork, 1);
+  resident::Status& st = w->rwork.host[0];
+  for (int restarts = 0;; ++restarts) {
+    st.rtol2 = o.rtol * o.rtol;
+    st.atol2 = o.atol * o.atol;
+    st.delta2 = delta * delta;
+    st.max_iter = o.max_iter - res.iterations;
+    st.active = 1;
+    if (!resident::solve(w->pack, w->rwork, ro, s->x.p, s->rhs.p))
+      return false;
+    res.iterations += st.iter;
+    res.reliable_updates += st.nb_ru;
+    const double bnorm = std::sqrt(st.bb), rnorm = std::sqrt(o.norm == 2 ? st.rr_out : st.rr_true);
+    res.relres = bnorm > 0.0 ? rnorm / bnorm : rnorm;
+    if (o.norm != 0) { // these tests have no true-residual restart
+      res.converged = st.converged && std::isfinite(res.relres);
+      return true;
+    }
+    res.converged = res.relres <= o.rtol || rnorm <= o.atol;
+    // restarted from the current iterate when the recursive residual met the
+    // tolerance but the true one does not
+    if (res.converged || res.iterations >= o.max_iter || restarts >= 8 || !std::isfinite(res.relres) || st.iter == 0)
+      return true;
+  }
+}
+
+static int solve(afem_system* s, const afem_solver_options& o, afem_solve_result* res, bool resident_ok = true)
 {
   AFEM_REQUIRE(o.method == AFEM_SOLVER_PCG_FP64 || o.method == AFEM_SOLVER_PCG_MIXED ||
                  o.method == AFEM_SOLVER_CG_FP64 || o.method == AFEM_SOLVER_FPCG_SPAI,
@@ -2069,6 +2131,25 @@ static int solve(afem_system* s, const afem_solver_options& o, afem_solve_result
     AFEM_REQUIRE(s->block == 1, AFEM_ERR_NOT_IMPLEMENTED, "the sparse preconditioner is for scalar systems");
     AFEM_REQUIRE(w->has_spai, AFEM_ERR_STATE,
                  "no preconditioner values: call afem_system_set_spai or afem_spai_apply after the matrix transformation");
+  }
+  if (resident_ok && resident_usable(s, w, o)) {
+    if (!o.use_initial_guess) {
+      hipLaunchKernelGGL(k_initial_guess, dim3(grid_for(s->nb_dof, 256)), dim3(256), 0, stream(), s->nb_dof,
+                         s->elim_info.p, s->elim_value.p, s->x.p);
+      check_launch("initial_guess");
+    }
+    afem_solve_result r{};
+    if (solve_resident(s, w, o, r)) {
+      r.solve_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_start).count();
+      if (res)
+        *res = r;
+      return r.converged ? AFEM_OK : AFEM_ERR_NOT_CONVERGED;
+    }
+    // the device could not hold every workgroup at once (another process on
+    // it, say): finish with the kernels that wait for nothing
+    afem_solver_options go = o;
+    go.use_initial_guess = 1;
+    return solve(s, go, res, false);
   }
   const bool mixed = o.method == AFEM_SOLVER_PCG_MIXED || flex;
   const int precond = (o.method == AFEM_SOLVER_CG_FP64 || o.preconditioner == AFEM_PRECOND_NONE) ? 0 : 1;
@@ -2510,7 +2591,9 @@ AFEM_API int afem_system_spmv_format(afem_system_t sys, int* format, int* lanes)
   AFEM_GUARD_BEGIN
   AFEM_REQUIRE(sys && format && lanes, AFEM_ERR_ARGUMENT, "null argument");
   afem_solver_ws* w = sys->ws;
-  *format = w ? w->format : -1;
+  // a resident solve alone has tuned nothing: its layout is SELL-64 in pairs
+  const bool pairs = w && w->format < 0 && w->pack.valid64;
+  *format = pairs ? (w->pack.idx16 ? kFmtSell16 : kFmtSell) : w ? w->format : -1;
   *lanes = w ? w->lanes : 0;
   AFEM_GUARD_END
 }

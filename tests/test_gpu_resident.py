@@ -1,0 +1,201 @@
+"""Solves whose vectors stay on the chip (one launch per solve) against host
+references and against the kernels that keep every vector in memory (a
+pinned SpMV format selects those).
+
+Both run the same recurrences, so iteration counts agree up to rounding in
+the dot products: within max(3, 5 %).  Residuals are checked on the host
+with the stated tolerance (1.01 x for the host's own rounding of b - A x).
+"""
+
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+pytestmark = pytest.mark.gpu
+
+METHODS = {"fp64": 0, "cg": 2}
+
+
+def device_system(A, M):
+    M = M.tocsr()
+    M.sort_indices()
+    d = [A.DeviceArray.from_numpy(a) for a in (M.indptr.astype(np.int32)[:-1], M.indices.astype(np.int32), M.data)]
+    s = A.DoFLinearSystem(M.shape[0])
+    s.set_csr_values(*d)
+    return s, d
+
+
+def band(n, offsets, shift=0.05, seed=0):
+    """Symmetric diagonally dominant matrix with random couplings at the offsets."""
+    rng = np.random.default_rng(seed)
+    rows, cols, vals = [], [], []
+    for o in offsets:
+        if o >= n:
+            continue
+        v = -rng.uniform(0.5, 1.5, n - o)
+        i = np.arange(n - o)
+        rows += [i, i + o]
+        cols += [i + o, i]
+        vals += [v, v]
+    if rows:
+        M = sp.csr_matrix((np.concatenate(vals), (np.concatenate(rows), np.concatenate(cols))), shape=(n, n))
+    else:
+        M = sp.csr_matrix((n, n))
+    d = -np.asarray(M.sum(axis=1)).ravel() * (1 + shift) + shift
+    return (M + sp.diags(d)).tocsr()
+
+
+def check(A, M, method, rtol, norm=0, max_iter=20000):
+    rng = np.random.default_rng(1)
+    b = rng.normal(size=M.shape[0])
+    out = {}
+    for lanes in (0, -1):
+        s, keep = device_system(A, M)
+        s.rhs().upload(b)
+        r = s.solve(method=METHODS[method], rtol=rtol, norm=norm, max_iter=max_iter, spmv_lanes=lanes)
+        x = s.solution().numpy()
+        assert r.converged
+        if norm == 0:
+            assert np.linalg.norm(b - M @ x) <= 1.01 * rtol * np.linalg.norm(b), (lanes, r.relres)
+            assert r.relres <= rtol
+        out[lanes] = (r.iterations, x)
+    a, g = out[0][0], out[-1][0]
+    assert abs(a - g) <= max(3, 0.05 * g), (a, g)
+    return out
+
+
+# rows around one slice, one workgroup (8 slices), one slice per wave on 256
+# CUs (131072 rows), and the first rows that need 4, 9 and 17 slices per wave
+SIZES = [1, 2, 63, 64, 65, 511, 512, 513, 4097, 131072, 131073, 524289, 1179649]
+
+
+@pytest.mark.parametrize("method", ["fp64"])
+@pytest.mark.parametrize("n", SIZES)
+def test_sizes(afem_gpu, n, method):
+    print(f"[case] resident n={n} {method}", flush=True)
+    check(afem_gpu, band(n, [1, 2, 70], shift=0.3), method, 1e-9)
+
+
+# pairs per row from none to more than two chunks, odd counts, and offsets
+# that need 32 bits
+PATTERNS = {"diagonal": (300, []), "one": (1000, [1]), "three_pairs": (1000, [1, 5, 31]),
+            "seven_pairs": (5000, [1, 2, 3, 40, 41, 700, 701]), "nine_pairs": (3000, list(range(1, 10))),
+            "twenty_pairs": (3000, list(range(1, 21))), "far": (70001, [1, 33000, 40001])}
+
+
+@pytest.mark.parametrize("method", ["fp64", "cg"])
+@pytest.mark.parametrize("name", PATTERNS)
+def test_patterns(afem_gpu, name, method):
+    n, offsets = PATTERNS[name]
+    print(f"[case] resident pattern {name} {method}", flush=True)
+    check(afem_gpu, band(n, offsets, shift=0.2), method, 1e-9)
+
+
+@pytest.mark.parametrize("norm", [1, 2])
+def test_norms(afem_gpu, norm):
+    print(f"[case] resident norm {norm}", flush=True)
+    M = band(20000, [1, 2, 150], shift=0.01)
+    out = check(afem_gpu, M, "fp64", 1e-10, norm=norm)
+    x, y = out[0][1], out[-1][1]
+    assert np.linalg.norm(x - y) <= 1e-7 * np.linalg.norm(y)
+
+
+def test_one_long_row_takes_the_general_kernels(afem_gpu):
+    """A dense row would pad its slice's pairs 3000 times over."""
+    print("[case] resident long row", flush=True)
+    n = 6000
+    M = band(n, [1], shift=0.5).tolil()
+    M[0, :] = -1e-3
+    M[:, 0] = -1e-3
+    M[0, 0] = 50.0
+    check(afem_gpu, M.tocsr(), "fp64", 1e-10)
+
+
+def test_more_iterations_than_one_launch(afem_gpu):
+    """8192 iterations end a launch: the vectors are kept and the next one goes
+    on.  The 1D Laplacian needs about n / 2 iterations; x reaches n^2 / 8 =
+    5e7, so b - A x carries up to eps * 4 * 5e7 = 4e-8 of rounding against
+    b = 1: the tolerance is 1e-6."""
+    print("[case] resident relaunch", flush=True)
+    A = afem_gpu
+    n = 20000
+    M = sp.diags([np.full(n, 2.0), -np.ones(n - 1), -np.ones(n - 1)], [0, 1, -1]).tocsr()
+    s, keep = device_system(A, M)
+    b = np.ones(n)
+    s.rhs().upload(b)
+    r = s.solve(rtol=1e-6, max_iter=100000)
+    assert r.iterations > 8192
+    assert np.linalg.norm(b - M @ s.solution().numpy()) <= 1.1e-6 * np.linalg.norm(b)
+    t = s.solve(raise_on_failure=False, rtol=1e-6, max_iter=8200)
+    assert t.iterations == 8200 and not t.converged
+
+
+def test_iteration_limits_and_initial_guess(afem_gpu):
+    print("[case] resident limits", flush=True)
+    A = afem_gpu
+    M = band(3000, [1, 9], shift=0.02)
+    x0 = np.random.default_rng(3).normal(size=3000)
+    for method in METHODS.values():
+        s, keep = device_system(A, M)
+        s.rhs().upload(M @ x0)
+        s.solution().upload(x0)
+        r = s.solve(method=method, rtol=1e-10, use_initial_guess=1)
+        assert r.iterations == 0 and r.converged
+        assert np.array_equal(s.solution().numpy(), x0)
+        r = s.solve(raise_on_failure=False, method=method, rtol=1e-10, max_iter=0)
+        assert r.iterations == 0 and not r.converged
+        r = s.solve(raise_on_failure=False, method=method, rtol=1e-14, max_iter=5)
+        assert r.iterations == 5 and not r.converged
+        # solving twice gives the same bits
+        s.solve(method=method, rtol=1e-8)
+        x = s.solution().numpy()
+        s.solve(method=method, rtol=1e-8)
+        assert np.array_equal(x, s.solution().numpy())
+
+
+def test_indefinite_matrix_stops(afem_gpu):
+    print("[case] resident indefinite", flush=True)
+    A = afem_gpu
+    n = 500
+    M = sp.diags([np.where(np.arange(n) % 2, 1.0, -1.0)], [0]).tocsr()
+    for method in (0, 2):
+        s, keep = device_system(A, M)
+        s.rhs().upload(np.ones(n))
+        r = s.solve(raise_on_failure=False, method=method, rtol=1e-10, max_iter=50)
+        s2, keep2 = device_system(A, M)
+        s2.rhs().upload(np.ones(n))
+        g = s2.solve(raise_on_failure=False, method=method, rtol=1e-10, max_iter=50, spmv_lanes=-1)
+        assert (r.converged, r.iterations) == (g.converged, g.iterations)
+
+
+def test_changed_values_and_pattern(afem_gpu):
+    """The kept copy of the matrix follows the values and the pattern."""
+    print("[case] resident new values", flush=True)
+    A = afem_gpu
+    X, C = A.box_mesh(3, 7, 0.15, seed=2)
+    m = A.Mesh(3, X, C)
+    bsr = A.BSRFormat(m, 1, use_csr=True)
+    bsr.compute_sparsity()
+    s = A.DoFLinearSystem(X.shape[0])
+    on = np.nonzero(X[:, 2] == 0.0)[0].astype(np.int32)
+    for k, lam in enumerate((1.0, 7.0)):
+        bsr.assemble_laplace(A.DeviceArray.from_numpy(np.full(C.shape[0], lam)), 1.0, s.rhs())
+        s.set_bsr(bsr)
+        s.apply_dirichlet(A.DIRICHLET_ROW_ELIMINATION, on, 1, 0, 0.0, 0.0)
+        s.apply_matrix_transformation()
+        s.apply_rhs_transformation()
+        for method in (0, 2):
+            s.solve(method=method, rtol=1e-10)
+            row, col, val, _ = bsr.download()
+            M = sp.csr_matrix((val, col, row), shape=(X.shape[0],) * 2)
+            b = s.rhs().numpy()
+            assert np.linalg.norm(b - M @ s.solution().numpy()) <= 1.01e-10 * np.linalg.norm(b), (k, method)
+    M = band(X.shape[0], [3, 11], shift=0.1).tocsr()
+    M.sort_indices()
+    d = [A.DeviceArray.from_numpy(a) for a in (M.indptr.astype(np.int32)[:-1], M.indices.astype(np.int32), M.data)]
+    s.clear_values()
+    s.set_csr_values(*d)
+    b = np.random.default_rng(0).normal(size=X.shape[0])
+    s.rhs().upload(b)
+    s.solve(rtol=1e-10)
+    assert np.linalg.norm(b - M @ s.solution().numpy()) <= 1.01e-10 * np.linalg.norm(b)
