@@ -28,6 +28,9 @@ struct Pack
   DBuf<double> v64, diag64, dinv64; // 128 * npair values; n
   DBuf<float> v32, diag32, dinv32;  // difference form: off-diagonal entries rounded, diag32 the row sum
   bool valid64 = false, valid32 = false;
+  DBuf<uint32_t> m;                 // sparse preconditioner: 64 * npair words (BF16) or 128 * npair (FP32)
+  DBuf<float> mdiag;
+  int valid_prec = 0;               // 0, 16 or 32: the bits of the values in m
 };
 
 // Offsets of a pattern (rows rp, columns ci) cut into segments.  False: the
@@ -36,6 +39,10 @@ bool pack_pattern(Pack& p, int32_t n, int64_t nnz, const int32_t* rp, const int3
                   const std::vector<int32_t>& seg_rows);
 // Values of the pattern's matrix: FP64, and with want32 the FP32 difference form too.
 void pack_values(Pack& p, const int32_t* rp, const int32_t* ci, const double* v, bool want32);
+
+// Sparse preconditioner with the pattern's entries (v in CSR order), stored
+// with 16 (BF16) or 32 bits.
+void pack_prec(Pack& p, const int32_t* rp, const int32_t* ci, const float* v, int bits);
 
 struct Status // of one segment
 {
@@ -50,6 +57,7 @@ struct Options
 {
   bool mixed = false;   // FP32 vectors and products, FP64 x and reliable updates
   bool precond = true;  // Jacobi
+  int prec = 0;         // flexible CG with the pack's sparse preconditioner (its bits); mixed
   int norm = 0;         // stopping norm of afem_solver_options
   long long spin_limit = 0;
 };

@@ -8,7 +8,10 @@
 // iteration.  Here an iteration is two barriers of 2-3 us and the matrix.
 // FP64 Jacobi-PCG, MI355X, three kernels -> resident: 256 x 256 quads of two
 // triangles (66049 rows) 16.3 -> 6.9 us an iteration; 48 x 52 x 45 nodes of
-// tetrahedra numbered at random (112 thousand rows) 22 -> 15.5 us.
+// tetrahedra numbered at random (112 thousand rows) 22 -> 15.5 us.  Mixed
+// Jacobi-PCG on 128^3 hexes of six tetrahedra (2.15 million rows) to 1e-8
+// 84.9 -> 36.9 ms; flexible PCG with a BF16 sparse preconditioner on 0.89
+// million rows, assembly and inference included, 61.6 -> 27.8 ms.
 #include "resident_kernel.h"
 
 #include <algorithm>
@@ -185,6 +188,65 @@ k_pair_values(int32_t nslice, const int32_t* __restrict__ slice_row, const int32
   }
 }
 
+// Sparse preconditioner with the pattern of the matrix: FP32 pairs, or pairs
+// of BF16 values (round to nearest even) in one word; its diagonal in FP32
+// with the same rounding.
+template <bool BF16>
+__global__ void __launch_bounds__(64)
+k_pair_prec(int32_t nslice, const int32_t* __restrict__ slice_row, const int32_t* __restrict__ rp,
+            const int32_t* __restrict__ ci, const float* __restrict__ v, const int32_t* __restrict__ poff, int stage,
+            uint32_t* __restrict__ out, float* __restrict__ mdiag)
+{
+  extern __shared__ __align__(16) unsigned char smem[]; // stage values, then stage columns
+  float* s_val = reinterpret_cast<float*>(smem);
+  int32_t* s_col = reinterpret_cast<int32_t*>(s_val + stage);
+  const int32_t s = blockIdx.x;
+  const int lane = threadIdx.x;
+  int32_t row, b, e, e0, e1;
+  bool live;
+  slice_rows(slice_row, nslice, s, rp, lane, row, live, b, e, e0, e1);
+  const bool staged = e1 - e0 <= stage;
+  if (staged) {
+    for (int32_t k = e0 + lane; k < e1; k += 64) {
+      s_val[k - e0] = v[k];
+      s_col[k - e0] = ci[k];
+    }
+    __syncthreads();
+  }
+  auto bits = [](float f) -> uint32_t {
+    const uint32_t u = __float_as_uint(f);
+    if constexpr (BF16)
+      return (u & 0x7fffffffu) > 0x7f800000u ? 0x7fc00000u : (u + 0x7fffu + ((u >> 16) & 1u)) & 0xffff0000u;
+    else
+      return u;
+  };
+  float diag = 0.f;
+  int32_t k = b;
+  auto next = [&]() -> uint32_t {
+    while (k < e) {
+      const int32_t c = staged ? s_col[k - e0] : ci[k];
+      const uint32_t a = bits(staged ? s_val[k - e0] : v[k]);
+      ++k;
+      if (c != row)
+        return a;
+      diag += __uint_as_float(a);
+    }
+    return 0u;
+  };
+  const int64_t at = (int64_t)poff[s] * 64 + lane;
+  const int w = poff[s + 1] - poff[s];
+  for (int q = 0; q < w; ++q) {
+    const uint32_t x = next(), y = next();
+    if constexpr (BF16)
+      out[at + (int64_t)q * 64] = (x >> 16) | y;
+    else
+      reinterpret_cast<uint2*>(out)[at + (int64_t)q * 64] = make_uint2(x, y);
+  }
+  (void)next(); // a diagonal entry after the last off-diagonal one
+  if (live)
+    mdiag[row] = diag;
+}
+
 // ---- launch layout ------------------------------------------------------------------------------
 
 constexpr int kMaxRows = kRowSteps[3];
@@ -229,6 +291,7 @@ bool pack_pattern(Pack& p, int32_t n, int64_t nnz, const int32_t* rp, const int3
 {
   p.n = n;
   p.valid64 = p.valid32 = false;
+  p.valid_prec = 0;
   p.seg_rows = seg_rows;
   const int nseg = (int)seg_rows.size() - 1;
   p.seg_slices.assign(nseg + 1, 0);
@@ -367,6 +430,8 @@ bool solve(const Pack& p, Work& w, const Options& o, double* x, const double* b)
   a.v = o.mixed ? (const void*)p.v32.p : (const void*)p.v64.p;
   a.diag = o.mixed ? (const void*)p.diag32.p : (const void*)p.diag64.p;
   a.dinv = o.mixed ? (const void*)p.dinv32.p : (const void*)p.dinv64.p;
+  a.m = p.m.p;
+  a.mdiag = p.mdiag.p;
   a.v64 = p.v64.p;
   a.diag64 = p.diag64.p;
   a.x = x;
@@ -393,8 +458,13 @@ bool solve(const Pack& p, Work& w, const Options& o, double* x, const double* b)
       w.host[k].epoch = w.epoch;
     AFEM_HIP(hipMemcpyAsync(w.st.p, w.host, sizeof(Status) * ((size_t)ns + 1), hipMemcpyHostToDevice, stream()));
     {
-      ProfScope prof(o.mixed ? "resident_cg_mixed" : "resident_cg_fp64");
-      launch_f64(a, w.rows_per_wave, p.idx16, w.grid, lds);
+      ProfScope prof(o.prec ? "resident_fpcg" : o.mixed ? "resident_cg_mixed" : "resident_cg_fp64");
+      if (o.prec)
+        launch_flex(a, w.rows_per_wave, p.idx16, o.prec == 16, w.grid, lds);
+      else if (o.mixed)
+        launch_f32(a, w.rows_per_wave, p.idx16, w.grid, lds);
+      else
+        launch_f64(a, w.rows_per_wave, p.idx16, w.grid, lds);
     }
     AFEM_HIP(hipMemcpyAsync(w.host, w.st.p, sizeof(Status) * ((size_t)ns + 1), hipMemcpyDeviceToHost, stream()));
     AFEM_HIP(hipStreamSynchronize(stream()));
@@ -413,9 +483,30 @@ bool solve(const Pack& p, Work& w, const Options& o, double* x, const double* b)
   }
 }
 
+void pack_prec(Pack& p, const int32_t* rp, const int32_t* ci, const float* v, int bits)
+{
+  if (p.valid_prec == bits)
+    return;
+  p.m.reserve((size_t)p.npair * (bits == 16 ? 64 : 128));
+  p.mdiag.reserve((size_t)p.n);
+  const int stage = std::min(kStageMax, std::max(1, p.max_len) * 64);
+  const size_t lds = (size_t)stage * 8;
+  if (bits == 16)
+    hipLaunchKernelGGL(k_pair_prec<true>, dim3(p.nslice), dim3(64), lds, stream(), p.nslice, p.slice_row.p, rp, ci, v,
+                       p.poff.p, stage, p.m.p, p.mdiag.p);
+  else
+    hipLaunchKernelGGL(k_pair_prec<false>, dim3(p.nslice), dim3(64), lds, stream(), p.nslice, p.slice_row.p, rp, ci,
+                       v, p.poff.p, stage, p.m.p, p.mdiag.p);
+  check_launch("pair_prec");
+  p.valid_prec = bits;
+}
+
 void launch_f64(const Args& a, int rows, bool idx16, int grid, size_t lds)
 {
-  launch_kernel<double>(a, rows, idx16, grid, lds);
+  if (idx16)
+    launch_kernel<double, 0, true>(a, rows, grid, lds);
+  else
+    launch_kernel<double, 0, false>(a, rows, grid, lds);
 }
 
 } // namespace resident

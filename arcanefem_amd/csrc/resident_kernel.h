@@ -25,11 +25,13 @@ struct Args
   const void* v;    // pairs of the product: FP64, or FP32 in difference form
   const void* diag; // its diagonal
   const void* dinv;
+  const void* m;     // pairs of the sparse preconditioner (FP32 or BF16) and its diagonal
+  const float* mdiag;
   const double* v64; // FP64 pairs and diagonal of the residual
   const double* diag64;
   double* x;
   const double* b;
-  void* u;
+  void* u;      // published u = D r, or z then r with a sparse preconditioner
   double* keep; // r, p, s (n each)
   int32_t n;
   uint64_t* slots;
@@ -296,16 +298,30 @@ __device__ __forceinline__ IndexPair<I16> load_offsets(Rsrc r, int lane, int q)
 // the rough u, not with the smooth p, and FP32 sums would cost 5 % more
 // iterations than forming A p anew (FP64 sums take 6 % fewer).
 //
-// r, s, the diagonal and FP32's D^-1 (FP64's p) are in registers, x and FP32's
-// p (FP64's D^-1) in LDS.  The matrix is the only stream of an iteration: it is read a chunk of CP
-// pairs ahead of its use, the first chunk of the next product ahead of both
-// barriers.
-template <class T, int R, bool I16>
+// With a sparse preconditioner (PREC 32 or 16: its values FP32 or BF16) B
+// publishes r, and a third phase forms u = M r, published, and the partials
+// u.r and u.s, whose sum gives the flexible beta = -alpha u.s / rho
+// (Polak-Ribiere; u.r / rho after a reliable update).
+//
+// r, s, the diagonal, FP64's p and FP32's D^-1 (or u = M r) are in registers,
+// x, FP32's p and FP64's D^-1 in LDS.  The matrices are the only streams of an
+// iteration: read a chunk of CP pairs ahead of their use, the first chunk of
+// the next product ahead of the barriers.
+enum StreamKind
+{
+  kStreamA = 0,
+  kStreamM32 = 32,
+  kStreamM16 = 16
+};
+
+template <class T, int R, bool I16, int PREC>
 __global__ void __launch_bounds__(kBS, 2) k_cg(Args a)
 {
   using V2 = ValuePair<T>;
   using I2 = IndexPair<I16>;
   constexpr bool MIXED = sizeof(T) == 4;
+  constexpr bool FLEX = PREC != 0;
+  static_assert(!FLEX || MIXED, "the sparse preconditioner is FP32");
   constexpr bool DLDS = !MIXED; // D^-1 in LDS and p in registers, else the other way round
   constexpr int CP = MIXED ? 8 : 4;
   extern __shared__ __align__(16) unsigned char smem[];
@@ -340,20 +356,16 @@ __global__ void __launch_bounds__(kBS, 2) k_cg(Args a)
 
   const int32_t rows = team.row1 - team.row0;
   const Rsrc urs = segment_buffer(reinterpret_cast<const T*>(a.u), team.row0, rows);
+  const Rsrc rrs = segment_buffer(reinterpret_cast<const T*>(a.u) + (FLEX ? a.n : 0), team.row0, rows);
   const Rsrc xrs = segment_buffer(a.x, team.row0, rows);
   const Rsrc brs = segment_buffer(a.b, team.row0, rows);
-  const Rsrc vrs = whole_buffer(a.v), irs = whole_buffer(a.idx);
+  const Rsrc vrs = whole_buffer(a.v), irs = whole_buffer(a.idx), mrs = whole_buffer(a.m);
+  const Rsrc mds = segment_buffer(a.mdiag, team.row0, FLEX ? rows : 0);
 
   double* l_x = reinterpret_cast<double*>(smem) + threadIdx.x;
   double* l_2 = l_x + R * kBS;
-  T r[R], dg[R], di[DLDS ? 1 : R];
+  T r[R], dg[R], di[DLDS ? 1 : R]; // FLEX: di holds u
   double s[R], pr[DLDS ? R : 1];
-  auto get_d = [&](int j) -> T {
-    if constexpr (DLDS)
-      return l_2[j * kBS];
-    else
-      return di[j];
-  };
   auto get_p = [&](int j) -> double {
     if constexpr (DLDS)
       return pr[j];
@@ -366,6 +378,13 @@ __global__ void __launch_bounds__(kBS, 2) k_cg(Args a)
     else
       l_2[j * kBS] = v;
   };
+  auto get_d = [&](int j) -> T {
+    if constexpr (DLDS)
+      return l_2[j * kBS];
+    else
+      return di[j];
+  };
+  auto get_u = [&](int j) -> T { return FLEX ? di[DLDS ? 0 : j] : get_d(j) * r[j]; };
   {
     const Rsrc drs = segment_buffer(reinterpret_cast<const T*>(a.dinv), team.row0, rows);
     const Rsrc grs = segment_buffer(reinterpret_cast<const T*>(a.diag), team.row0, rows);
@@ -378,11 +397,13 @@ __global__ void __launch_bounds__(kBS, 2) k_cg(Args a)
         di[j] = (T)0;
       if (j < nsl) {
         l_x[j * kBS] = bload<double, 0>(xrs, row_of(j));
-        const T d = a.precond ? bload<T, 0>(drs, row_of(j)) : (T)1;
-        if constexpr (DLDS)
-          l_2[j * kBS] = d;
-        else
-          di[j] = d;
+        if constexpr (!FLEX) {
+          const T d = a.precond ? bload<T, 0>(drs, row_of(j)) : (T)1;
+          if constexpr (DLDS)
+            l_2[j * kBS] = d;
+          else
+            di[j] = d;
+        }
         dg[j] = bload<T, 0>(grs, row_of(j));
       }
     }
@@ -390,13 +411,13 @@ __global__ void __launch_bounds__(kBS, 2) k_cg(Args a)
 
   // b - A64 x of row j, x as published; 0 in the lanes past the segment
   auto residual = [&](int j) -> double {
-    const Rsrc mrs = whole_buffer(a.v64);
+    const Rsrc mrs64 = whole_buffer(a.v64);
     const Rsrc grs = segment_buffer(a.diag64, team.row0, rows);
     const int32_t row = row_of(j);
     double t0 = bload<double, 0>(grs, row) * l_x[j * kBS], t1 = 0.0;
     const int q1 = pair0(j + 1);
     for (int q = pair0(j); q < q1; ++q) {
-      const ValuePair<double> m = load_values<double>(mrs, lane, q);
+      const ValuePair<double> m = load_values<double>(mrs64, lane, q);
       const I2 d = load_offsets<I16>(irs, lane, q);
       t0 += m.x * bload<double, kSc1>(xrs, row + d.x());
       t1 += m.y * bload<double, kSc1>(xrs, row + d.y());
@@ -408,6 +429,94 @@ __global__ void __launch_bounds__(kBS, 2) k_cg(Args a)
     for (int j = 0; j < R; ++j)
       if (j < nsl)
         bstore<double, kSc1>(xrs, row_of(j), l_x[j * kBS]);
+  };
+
+  // the stream: the chunk whose gathers go out next
+  V2 cv[CP];
+  I2 cd[CP];
+  auto fetch = [&](auto stream, int q0, int cnt) {
+    constexpr int S = decltype(stream)::value;
+#pragma unroll
+    for (int z = 0; z < CP; ++z)
+      if (z < cnt) {
+        if constexpr (S == kStreamM16)
+          cv[z].x = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(mrs, lane * 4, (q0 + z) * (kWave * 4), 0));
+        else
+          cv[z] = load_values<T>(S == kStreamA ? vrs : mrs, lane, q0 + z);
+        cd[z] = load_offsets<I16>(irs, lane, q0 + z);
+      }
+  };
+  const int first = pair0(0), first_cnt = nsl > 0 ? pair0(1) - first : 0;
+  using StreamA = std::integral_constant<int, kStreamA>;
+  using StreamM = std::integral_constant<int, PREC>; // A's own when there is none
+  // One product: row j's sum of value * (gathered element of `src`, less
+  // `own` in difference form) is handed to finish(j, own, sum).
+  auto product = [&](auto stream, auto next, Rsrc src, auto own, auto finish) {
+    constexpr int S = decltype(stream)::value;
+    using Acc = typename std::conditional<S == kStreamA, double, float>::type;
+    constexpr bool DIFF = MIXED && S == kStreamA;
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+      if (j < nsl) {
+        const int32_t row = row_of(j);
+        const int q1 = pair0(j + 1);
+        const T uv = own(j);
+        Acc t0 = 0, t1 = 0;
+        int c = pair0(j);
+        do {
+          const int cnt = q1 - c;
+          T x0[CP], x1[CP];
+#pragma unroll
+          for (int z = 0; z < CP; ++z)
+            if (z < cnt) {
+              x0[z] = bload<T, kSc1>(src, row + cd[z].x());
+              x1[z] = bload<T, kSc1>(src, row + cd[z].y());
+            }
+          V2 m[CP];
+#pragma unroll
+          for (int z = 0; z < CP; ++z)
+            m[z] = cv[z];
+          // the next chunk's loads go out before this chunk's gathers are used
+          if (c + CP < q1)
+            fetch(stream, c + CP, cnt - CP);
+          else if (j + 1 < R && j + 1 < nsl)
+            fetch(stream, q1, pair0(j + 2) - q1);
+          else
+            fetch(next, first, first_cnt);
+#pragma unroll
+          for (int z = 0; z < CP; ++z)
+            if (z < cnt) {
+              if constexpr (S == kStreamM16) { // two BF16 values in one word
+                const uint32_t w = __float_as_uint(m[z].x);
+                t0 += __uint_as_float(w << 16) * x0[z];
+                t1 += __uint_as_float(w & 0xffff0000u) * x1[z];
+              }
+              else if constexpr (DIFF) { // padding: value 0, the row itself
+                t0 += (Acc)(m[z].x * (x0[z] - uv));
+                t1 += (Acc)(m[z].y * (x1[z] - uv));
+              }
+              else {
+                t0 += m[z].x * x0[z];
+                t1 += m[z].y * x1[z];
+              }
+            }
+          c += CP;
+        } while (c < q1);
+        finish(j, uv, t0 + t1);
+      }
+  };
+  // u = M r from the published r; partials u.r and u.s
+  auto precondition = [&](double (&v)[2]) {
+    v[0] = v[1] = 0.0;
+    product(
+      StreamM{}, StreamA{}, rrs, [&](int j) { return r[j]; },
+      [&](int j, T rv, float t) {
+        const float u = t + bload<float, 0>(mds, row_of(j)) * (float)rv;
+        di[DLDS ? 0 : j] = (T)u;
+        bstore<float, kSc1>(urs, row_of(j), u);
+        v[0] += (double)u * (double)rv;
+        v[1] += (double)u * s[j];
+      });
   };
 
   const int norm = a.norm;
@@ -425,13 +534,19 @@ __global__ void __launch_bounds__(kBS, 2) k_cg(Args a)
     for (int j = 0; j < R; ++j)
       if (j < nsl) {
         const double rd = residual(j), bd = bload<double, 0>(brs, row_of(j));
-        const T rv = (T)rd;
-        const T uv = get_d(j) * rv, mb = get_d(j) * (T)bd;
-        r[j] = rv;
-        bstore<T, kSc1>(urs, row_of(j), uv);
-        v[0] += (double)rv * (double)uv;
-        v[1] += norm == 2 ? (double)uv * (double)uv : rd * rd;
-        v[2] += norm == 2 ? (double)mb * (double)mb : bd * bd;
+        r[j] = (T)rd;
+        if constexpr (FLEX) {
+          bstore<T, kSc1>(rrs, row_of(j), r[j]);
+          v[1] += rd * rd;
+          v[2] += bd * bd;
+        }
+        else {
+          const T uv = get_u(j), mb = get_d(j) * (T)bd;
+          bstore<T, kSc1>(urs, row_of(j), uv);
+          v[0] += (double)r[j] * (double)uv;
+          v[1] += norm == 2 ? (double)uv * (double)uv : rd * rd;
+          v[2] += norm == 2 ? (double)mb * (double)mb : bd * bd;
+        }
       }
     if (!team_sum<3>(bar, v))
       return;
@@ -440,7 +555,7 @@ __global__ void __launch_bounds__(kBS, 2) k_cg(Args a)
     rr_ref = v[1];
     rr_out = v[1];
     beta = 0.0;
-    finished = (norm == 1 ? v[0] : v[1]) <= tol2 || v[0] == 0.0;
+    finished = (norm == 1 ? v[0] : v[1]) <= tol2 || (!FLEX && v[0] == 0.0);
     converged = finished ? 1 : 0;
     if (me == 0 && threadIdx.x == 0) {
       st.bb = v[2];
@@ -448,141 +563,136 @@ __global__ void __launch_bounds__(kBS, 2) k_cg(Args a)
     }
   }
   else {
-    const Rsrc rrs = segment_buffer(keep, team.row0, rows);
-    const Rsrc prs = segment_buffer(keep + a.n, team.row0, rows);
-    const Rsrc srs = segment_buffer(keep + 2 * (int64_t)a.n, team.row0, rows);
+    const Rsrc krs = segment_buffer(keep, team.row0, rows);
+    const Rsrc kps = segment_buffer(keep + a.n, team.row0, rows);
+    const Rsrc kss = segment_buffer(keep + 2 * (int64_t)a.n, team.row0, rows);
 #pragma unroll
     for (int j = 0; j < R; ++j)
       if (j < nsl) {
-        r[j] = (T)bload<double, 0>(rrs, row_of(j));
-        set_p(j, bload<double, 0>(prs, row_of(j)));
-        s[j] = bload<double, 0>(srs, row_of(j));
-        bstore<T, kSc1>(urs, row_of(j), get_d(j) * r[j]);
+        r[j] = (T)bload<double, 0>(krs, row_of(j));
+        set_p(j, bload<double, 0>(kps, row_of(j)));
+        s[j] = bload<double, 0>(kss, row_of(j));
+        bstore<T, kSc1>(FLEX ? rrs : urs, row_of(j), FLEX ? r[j] : get_u(j));
       }
     double v[1] = { 0.0 };
     if (!team_sum<1>(bar, v))
       return;
   }
   finished = finished || k >= max_iter;
-
-  V2 cv[CP];
-  I2 cd[CP];
-  auto fetch = [&](int q0, int cnt) {
-#pragma unroll
-    for (int z = 0; z < CP; ++z)
-      if (z < cnt) {
-        cv[z] = load_values<T>(vrs, lane, q0 + z);
-        cd[z] = load_offsets<I16>(irs, lane, q0 + z);
-      }
-  };
-  const int first = pair0(0), first_cnt = nsl > 0 ? pair0(1) - first : 0;
-  fetch(first, first_cnt);
+  fetch(StreamM{}, first, first_cnt); // of A without a sparse preconditioner
+  bool skip = FLEX;                   // a launch of the flexible method starts with u = M r
 
   while (!finished && k < k_end) {
-    // A
-    double v1[1] = { 0.0 };
-#pragma unroll
-    for (int j = 0; j < R; ++j)
-      if (j < nsl) {
-        const int32_t row = row_of(j);
-        const int q1 = pair0(j + 1);
-        const T uv = get_d(j) * r[j];
-        double t0 = (double)(dg[j] * uv), t1 = 0.0;
-        int c = pair0(j);
-        do {
-          const int cnt = q1 - c;
-          T x0[CP], x1[CP];
-#pragma unroll
-          for (int z = 0; z < CP; ++z)
-            if (z < cnt) {
-              x0[z] = bload<T, kSc1>(urs, row + cd[z].x());
-              x1[z] = bload<T, kSc1>(urs, row + cd[z].y());
-            }
-          V2 m[CP];
-#pragma unroll
-          for (int z = 0; z < CP; ++z)
-            m[z] = cv[z];
-          // the next chunk's loads go out before this chunk's gathers are used
-          if (c + CP < q1)
-            fetch(c + CP, cnt - CP);
-          else if (j + 1 < R && j + 1 < nsl)
-            fetch(q1, pair0(j + 2) - q1);
-          else
-            fetch(first, first_cnt);
-#pragma unroll
-          for (int z = 0; z < CP; ++z)
-            if (z < cnt) {
-              if constexpr (MIXED) { // difference form; padding: value 0, the row itself
-                t0 += (double)(m[z].x * (x0[z] - uv));
-                t1 += (double)(m[z].y * (x1[z] - uv));
-              }
-              else {
-                t0 += m[z].x * x0[z];
-                t1 += m[z].y * x1[z];
-              }
-            }
-          c += CP;
-        } while (c < q1);
-        const double pj = (double)uv + beta * get_p(j);
-        set_p(j, pj);
-        s[j] = (t0 + t1) + beta * s[j];
-        v1[0] += pj * s[j];
-      }
-    if (!team_sum<1>(bar, v1))
-      return;
-    const double ps = v1[0];
-    if (!(ps > 0.0) || !isfinite(ps)) { // the operator is not positive definite on p
-      breakdown = 1;
-      finished = true;
-      break;
-    }
-    // B
-    const double alpha = rho / ps;
+    double alpha = 0.0;
     double v2[2] = { 0.0, 0.0 };
-#pragma unroll
-    for (int j = 0; j < R; ++j)
-      if (j < nsl) {
-        r[j] = (T)((double)r[j] - alpha * s[j]);
-        const T uv = get_d(j) * r[j];
-        bstore<T, kSc1>(urs, row_of(j), uv);
-        v2[0] += (double)r[j] * (double)uv;
-        v2[1] += norm == 2 ? (double)uv * (double)uv : (double)r[j] * (double)r[j];
-        l_x[j * kBS] += alpha * get_p(j);
+    bool updated = false; // a reliable update replaced r
+    if (!skip) {
+      // A
+      double v1[1] = { 0.0 };
+      product(
+        StreamA{}, StreamM{}, urs, get_u,
+        [&](int j, T uv, double t) {
+          const double pj = (double)uv + beta * get_p(j);
+          set_p(j, pj);
+          s[j] = (double)(dg[j] * uv) + t + beta * s[j];
+          v1[0] += pj * s[j];
+        });
+      if (!team_sum<1>(bar, v1))
+        return;
+      const double ps = v1[0];
+      if (!(ps > 0.0) || !isfinite(ps) || (FLEX && !(rho > 0.0))) { // the operator is not positive definite on p
+        breakdown = 1;
+        finished = true;
+        break;
       }
-    if (!team_sum<2>(bar, v2))
-      return;
-    const double rz = v2[0], rr = v2[1];
-    beta = rho != 0.0 ? rz / rho : 0.0;
-    if constexpr (MIXED) {
-      if (rr <= delta2 * rr_ref || rr <= tol2 || k + 1 >= max_iter || !isfinite(rr)) {
-        publish_x();
-        double v[1] = { 0.0 };
-        if (!team_sum<1>(bar, v))
-          return;
-        v[0] = 0.0;
+      // B
+      alpha = rho / ps;
 #pragma unroll
-        for (int j = 0; j < R; ++j)
-          if (j < nsl) {
-            const double rd = residual(j);
-            r[j] = (T)rd;
-            v[0] += rd * rd;
+      for (int j = 0; j < R; ++j)
+        if (j < nsl) {
+          r[j] = (T)((double)r[j] - alpha * s[j]);
+          if constexpr (FLEX) {
+            bstore<T, kSc1>(rrs, row_of(j), r[j]);
+            v2[1] += (double)r[j] * (double)r[j];
           }
-        if (!team_sum<1>(bar, v))
-          return;
-        ++nb_ru;
-        rr_out = v[0];
-        if (v[0] <= tol2 || k + 1 >= max_iter || !isfinite(v[0])) {
-          converged = v[0] <= tol2 ? 1 : 0;
-          ++k;
-          finished = true;
-          break;
+          else {
+            const T uv = get_u(j);
+            bstore<T, kSc1>(urs, row_of(j), uv);
+            v2[0] += (double)r[j] * (double)uv;
+            v2[1] += norm == 2 ? (double)uv * (double)uv : (double)r[j] * (double)r[j];
+          }
+          l_x[j * kBS] += alpha * get_p(j);
         }
-        rr_ref = v[0];
-        v[0] = 0.0;
+      if (!team_sum<2>(bar, v2))
+        return;
+      const double rr = v2[1];
+      if constexpr (MIXED) {
+        if (rr <= delta2 * rr_ref || rr <= tol2 || k + 1 >= max_iter || !isfinite(rr)) {
+          updated = true;
+          publish_x();
+          double v[1] = { 0.0 };
+          if (!team_sum<1>(bar, v))
+            return;
+          v[0] = 0.0;
+#pragma unroll
+          for (int j = 0; j < R; ++j)
+            if (j < nsl) {
+              const double rd = residual(j);
+              r[j] = (T)rd;
+              if constexpr (FLEX)
+                bstore<T, kSc1>(rrs, row_of(j), r[j]);
+              v[0] += rd * rd;
+            }
+          if (!team_sum<1>(bar, v))
+            return;
+          ++nb_ru;
+          rr_out = v[0];
+          if (v[0] <= tol2 || k + 1 >= max_iter || !isfinite(v[0])) {
+            converged = v[0] <= tol2 ? 1 : 0;
+            ++k;
+            finished = true;
+            break;
+          }
+          rr_ref = v[0];
+        }
+        else
+          rr_out = rr;
+      }
+    }
+    if constexpr (FLEX) {
+      double v[2];
+      precondition(v);
+      if (!team_sum<2>(bar, v))
+        return;
+      if (skip) {
+        skip = false;
+        if (!a.resume) { // else rho and beta come from the last launch
+          rho = v[0];
+          if (rho == 0.0) {
+            finished = true;
+            converged = 1;
+          }
+        }
+        continue;
+      }
+      beta = updated ? v[0] / rho : -alpha * v[1] / rho;
+      if (!(v[0] > 0.0) || !isfinite(v[0]) || !isfinite(beta)) { // M is not positive on this residual
+        breakdown = 1;
+        ++k;
+        finished = true;
+        break;
+      }
+      rho = v[0];
+    }
+    else {
+      beta = rho != 0.0 ? v2[0] / rho : 0.0;
+      rho = v2[0];
+      if (updated) {
+        double v[1] = { 0.0 };
 #pragma unroll
         for (int j = 0; j < R; ++j)
           if (j < nsl) {
-            const T uv = get_d(j) * r[j];
+            const T uv = get_u(j);
             bstore<T, kSc1>(urs, row_of(j), uv);
             v[0] += (double)r[j] * (double)uv;
           }
@@ -590,21 +700,16 @@ __global__ void __launch_bounds__(kBS, 2) k_cg(Args a)
           return;
         rho = v[0];
       }
-      else {
-        rho = rz;
+      if constexpr (!MIXED) {
+        const double rr = v2[1], crit = norm == 1 ? rho : rr;
         rr_out = rr;
+        if (crit <= tol2 || k + 1 >= max_iter || !isfinite(rr)) {
+          converged = crit <= tol2 ? 1 : 0;
+          ++k;
+          finished = true;
+          break;
+        }
       }
-    }
-    else {
-      rr_out = rr;
-      const double crit = norm == 1 ? rz : rr;
-      if (crit <= tol2 || k + 1 >= max_iter || !isfinite(rr)) {
-        converged = crit <= tol2 ? 1 : 0;
-        ++k;
-        finished = true;
-        break;
-      }
-      rho = rz;
     }
     ++k;
   }
@@ -631,16 +736,16 @@ __global__ void __launch_bounds__(kBS, 2) k_cg(Args a)
     }
   }
   else {
-    const Rsrc rrs = segment_buffer(keep, team.row0, rows);
-    const Rsrc prs = segment_buffer(keep + a.n, team.row0, rows);
-    const Rsrc srs = segment_buffer(keep + 2 * (int64_t)a.n, team.row0, rows);
+    const Rsrc krs = segment_buffer(keep, team.row0, rows);
+    const Rsrc kps = segment_buffer(keep + a.n, team.row0, rows);
+    const Rsrc kss = segment_buffer(keep + 2 * (int64_t)a.n, team.row0, rows);
 #pragma unroll
     for (int j = 0; j < R; ++j)
       if (j < nsl) {
         bstore<double, 0>(xrs, row_of(j), l_x[j * kBS]);
-        bstore<double, 0>(rrs, row_of(j), (double)r[j]);
-        bstore<double, 0>(prs, row_of(j), get_p(j));
-        bstore<double, 0>(srs, row_of(j), s[j]);
+        bstore<double, 0>(krs, row_of(j), (double)r[j]);
+        bstore<double, 0>(kps, row_of(j), get_p(j));
+        bstore<double, 0>(kss, row_of(j), s[j]);
       }
   }
   if (lead) {
@@ -658,23 +763,18 @@ __global__ void __launch_bounds__(kBS, 2) k_cg(Args a)
 // Launches the kernel with room for `rows` slices per wave.
 void launch_f64(const Args& a, int rows, bool idx16, int grid, size_t lds);
 void launch_f32(const Args& a, int rows, bool idx16, int grid, size_t lds);
+void launch_flex(const Args& a, int rows, bool idx16, bool bf16, int grid, size_t lds);
 
 constexpr int kRowSteps[4] = { 1, 4, 9, 17 };
 
-template <class T>
-inline void launch_kernel(const Args& a, int rows, bool idx16, int grid, size_t lds)
+template <class T, int PREC, bool I16>
+inline void launch_kernel(const Args& a, int rows, int grid, size_t lds)
 {
   auto go = [&](auto tag) {
-    constexpr int R = decltype(tag)::value;
-    auto one = [&](auto kernel) {
-      AFEM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)lds));
-      hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBS), lds, stream(), a);
-    };
-    if (idx16)
-      one(k_cg<T, R, true>);
-    else
-      one(k_cg<T, R, false>);
+    auto kernel = k_cg<T, decltype(tag)::value, I16, PREC>;
+    AFEM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 (int)lds));
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBS), lds, stream(), a);
   };
   switch (rows) {
   case 1: go(std::integral_constant<int, 1>{}); break;

@@ -20,7 +20,7 @@
 // in FP64; only the FP64 residual of a reliable update can declare
 // convergence.  Dots are accumulated in FP64.
 //
-// Scalar FP64 solves without a pinned SpMV format run in one launch instead
+// Scalar solves without a pinned SpMV format run in one launch instead
 // (resident.hip) when the system fits the chip.
 //
 // SpMV formats: CSR with G lanes per row (wavefront-group row reductions) and
@@ -2054,103 +2054,75 @@ static void launch_flex_iteration(afem_system* s, afem_solver_ws* w, int k, cons
   }
 }
 
-// The resident kernel runs scalar FP64 CG and Jacobi-PCG on systems
-// whose vectors fit the device's registers and LDS (2.2 million rows on 256
-// CUs), unless the caller pinned an SpMV format.
+// The resident kernel runs scalar systems whose vectors fit the device's
+// registers and LDS (2.2 million rows on 256 CUs), unless the caller pinned an
+// SpMV format; the mixed solvers' difference form needs every diagonal entry.
 static bool resident_usable(afem_system* s, afem_solver_ws* w, const afem_solver_options& o)
 {
-  if (s->block != 1 || (o.method != AFEM_SOLVER_PCG_FP64 && o.method != AFEM_SOLVER_CG_FP64) || o.spmv_lanes != 0 || w->forced_format)
+  if (s->block != 1 || o.spmv_lanes != 0 || w->forced_format)
     return false;
   if (!w->pack_valid) {
     w->pack_usable = resident::pack_pattern(w->pack, s->nb_dof, s->nnz, s->row_index, s->columns, { 0, s->nb_dof });
     w->pack_valid = true;
   }
-  return w->pack_usable;
+  const bool fp64 = o.method == AFEM_SOLVER_PCG_FP64 || o.method == AFEM_SOLVER_CG_FP64;
+  return w->pack_usable && (fp64 || w->pack.all_diag);
 }
 
-// False: a barrier wait gave up (x is some iterate).
-static bool solve_resident(afem_system* s, afem_solver_ws* w, const afem_solver_options& o, afem_solve_result& res)
+struct SolveTotals
 {
-  const bool mixed = o.method == AFEM_SOLVER_PCG_MIXED;
+  int iterations = 0, reliable_updates = 0;
+  bool converged = false, breakdown = false;
+  double relres = 0.0;
+};
+
+// False: a barrier wait gave up (x is some iterate).
+static bool solve_resident(afem_system* s, afem_solver_ws* w, const afem_solver_options& o, SolveTotals& t)
+{
+  const bool flex = o.method == AFEM_SOLVER_FPCG_SPAI;
+  const bool mixed = o.method == AFEM_SOLVER_PCG_MIXED || flex;
   const double delta = o.reliable_delta > 0.0 ? o.reliable_delta : 0.1;
   resident::pack_values(w->pack, s->row_index, s->columns, s->values, mixed);
   resident::Options ro;
   ro.mixed = mixed;
   ro.precond = o.method != AFEM_SOLVER_CG_FP64 && o.preconditioner != AFEM_PRECOND_NONE;
   ro.norm = o.norm;
+  if (flex) { // BF16 values come with 16-bit offsets, FP32 otherwise
+    ro.prec = o.precond_bf16 && w->pack.idx16 ? 16 : 32;
+    resident::pack_prec(w->pack, s->row_index, s->columns, w->spai32.p, ro.prec);
+  }
   resident::reserve(w->rwork, 1);
   resident::Status& st = w->rwork.host[0];
   for (int restarts = 0;; ++restarts) {
     st.rtol2 = o.rtol * o.rtol;
     st.atol2 = o.atol * o.atol;
     st.delta2 = delta * delta;
-    st.max_iter = o.max_iter - res.iterations;
+    st.max_iter = o.max_iter - t.iterations;
     st.active = 1;
     if (!resident::solve(w->pack, w->rwork, ro, s->x.p, s->rhs.p))
       return false;
-    res.iterations += st.iter;
-    res.reliable_updates += st.nb_ru;
+    t.iterations += st.iter;
+    t.reliable_updates += st.nb_ru;
+    t.breakdown = st.breakdown != 0;
     const double bnorm = std::sqrt(st.bb), rnorm = std::sqrt(o.norm == 2 ? st.rr_out : st.rr_true);
-    res.relres = bnorm > 0.0 ? rnorm / bnorm : rnorm;
+    t.relres = bnorm > 0.0 ? rnorm / bnorm : rnorm;
     if (o.norm != 0) { // these tests have no true-residual restart
-      res.converged = st.converged && std::isfinite(res.relres);
+      t.converged = st.converged && std::isfinite(t.relres);
       return true;
     }
-    res.converged = res.relres <= o.rtol || rnorm <= o.atol;
+    t.converged = t.relres <= o.rtol || rnorm <= o.atol;
     // restarted from the current iterate when the recursive residual met the
     // tolerance but the true one does not
-    if (res.converged || res.iterations >= o.max_iter || restarts >= 8 || !std::isfinite(res.relres) || st.iter == 0)
+    if (t.converged || t.iterations >= o.max_iter || restarts >= 8 || !std::isfinite(t.relres) || st.iter == 0 ||
+        (flex && t.breakdown))
       return true;
   }
 }
 
-static int solve(afem_system* s, const afem_solver_options& o, afem_solve_result* res, bool resident_ok = true)
+// Every vector in memory, three to five kernels an iteration.
+static void solve_streaming(afem_system* s, afem_solver_ws* w, const afem_solver_options& o, SolveTotals& out)
 {
-  AFEM_REQUIRE(o.method == AFEM_SOLVER_PCG_FP64 || o.method == AFEM_SOLVER_PCG_MIXED ||
-                 o.method == AFEM_SOLVER_CG_FP64 || o.method == AFEM_SOLVER_FPCG_SPAI,
-               AFEM_ERR_ARGUMENT, "unknown solver method");
-  AFEM_REQUIRE(o.preconditioner == AFEM_PRECOND_JACOBI || o.preconditioner == AFEM_PRECOND_NONE, AFEM_ERR_ARGUMENT,
-               "unknown preconditioner");
-  AFEM_REQUIRE(o.rtol >= 0.0 && o.atol >= 0.0 && o.max_iter >= 0, AFEM_ERR_ARGUMENT, "bad tolerances");
-  AFEM_REQUIRE(o.norm >= 0 && o.norm <= 2, AFEM_ERR_ARGUMENT, "unknown stopping norm");
-  AFEM_REQUIRE(o.norm == 0 || (o.method != AFEM_SOLVER_PCG_MIXED && o.method != AFEM_SOLVER_FPCG_SPAI),
-               AFEM_ERR_NOT_IMPLEMENTED,
-               "the natural-norm and preconditioned-norm stopping tests are available for the FP64 solvers");
-  // The reference's row-column elimination never touches column 0
-  // (femutils/CsrDoFLinearSystemImpl.cc:111), so with DoF 0 eliminated the
-  // matrix keeps A[i,0] in every row while the RHS is lifted by A[0,i] g
-  // (femutils/DoFLinearSystemImplBase.cc:65-87): a non-symmetric system
-  // that no conjugate-gradient method solves.
-  AFEM_REQUIRE(!s->dof0_row_column, AFEM_ERR_NOT_IMPLEMENTED,
-               "DoF 0 is row-column eliminated: the transformed matrix keeps column 0 and is not symmetric, "
-               "so PCG does not apply (use RowElimination or Penalty for that DoF)");
-  auto t_start = std::chrono::steady_clock::now();
-  afem_solver_ws* w = workspace(s);
   const bool flex = o.method == AFEM_SOLVER_FPCG_SPAI;
-  if (flex) {
-    AFEM_REQUIRE(s->block == 1, AFEM_ERR_NOT_IMPLEMENTED, "the sparse preconditioner is for scalar systems");
-    AFEM_REQUIRE(w->has_spai, AFEM_ERR_STATE,
-                 "no preconditioner values: call afem_system_set_spai or afem_spai_apply after the matrix transformation");
-  }
-  if (resident_ok && resident_usable(s, w, o)) {
-    if (!o.use_initial_guess) {
-      hipLaunchKernelGGL(k_initial_guess, dim3(grid_for(s->nb_dof, 256)), dim3(256), 0, stream(), s->nb_dof,
-                         s->elim_info.p, s->elim_value.p, s->x.p);
-      check_launch("initial_guess");
-    }
-    afem_solve_result r{};
-    if (solve_resident(s, w, o, r)) {
-      r.solve_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_start).count();
-      if (res)
-        *res = r;
-      return r.converged ? AFEM_OK : AFEM_ERR_NOT_CONVERGED;
-    }
-    // the device could not hold every workgroup at once (another process on
-    // it, say): finish with the kernels that wait for nothing
-    afem_solver_options go = o;
-    go.use_initial_guess = 1;
-    return solve(s, go, res, false);
-  }
   const bool mixed = o.method == AFEM_SOLVER_PCG_MIXED || flex;
   const int precond = (o.method == AFEM_SOLVER_CG_FP64 || o.preconditioner == AFEM_PRECOND_NONE) ? 0 : 1;
   const int check_every = o.check_every > 0 ? o.check_every : 16;
@@ -2167,11 +2139,6 @@ static int solve(afem_system* s, const afem_solver_options& o, afem_solve_result
   const Parts P = parts_of(w);
   const int nblk = spmv_blocks(s);
 
-  if (!o.use_initial_guess) {
-    hipLaunchKernelGGL(k_initial_guess, dim3(grid_for(s->nb_dof, 256)), dim3(256), 0, stream(), s->nb_dof,
-                       s->elim_info.p, s->elim_value.p, s->x.p);
-    check_launch("initial_guess");
-  }
   State init{};
   init.rtol2 = o.rtol * o.rtol;
   init.atol2 = o.atol * o.atol;
@@ -2228,36 +2195,83 @@ static int solve(afem_system* s, const afem_solver_options& o, afem_solve_result
     // restart from the current iterate
     ++restarts;
   }
+  out = SolveTotals{ total_iter, nb_ru, converged, breakdown, relres };
+}
+
+static int solve(afem_system* s, const afem_solver_options& o, afem_solve_result* res, bool resident_ok = true)
+{
+  AFEM_REQUIRE(o.method == AFEM_SOLVER_PCG_FP64 || o.method == AFEM_SOLVER_PCG_MIXED ||
+                 o.method == AFEM_SOLVER_CG_FP64 || o.method == AFEM_SOLVER_FPCG_SPAI,
+               AFEM_ERR_ARGUMENT, "unknown solver method");
+  AFEM_REQUIRE(o.preconditioner == AFEM_PRECOND_JACOBI || o.preconditioner == AFEM_PRECOND_NONE, AFEM_ERR_ARGUMENT,
+               "unknown preconditioner");
+  AFEM_REQUIRE(o.rtol >= 0.0 && o.atol >= 0.0 && o.max_iter >= 0, AFEM_ERR_ARGUMENT, "bad tolerances");
+  AFEM_REQUIRE(o.norm >= 0 && o.norm <= 2, AFEM_ERR_ARGUMENT, "unknown stopping norm");
+  AFEM_REQUIRE(o.norm == 0 || (o.method != AFEM_SOLVER_PCG_MIXED && o.method != AFEM_SOLVER_FPCG_SPAI),
+               AFEM_ERR_NOT_IMPLEMENTED,
+               "the natural-norm and preconditioned-norm stopping tests are available for the FP64 solvers");
+  // The reference's row-column elimination never touches column 0
+  // (femutils/CsrDoFLinearSystemImpl.cc:111), so with DoF 0 eliminated the
+  // matrix keeps A[i,0] in every row while the RHS is lifted by A[0,i] g
+  // (femutils/DoFLinearSystemImplBase.cc:65-87): a non-symmetric system
+  // that no conjugate-gradient method solves.
+  AFEM_REQUIRE(!s->dof0_row_column, AFEM_ERR_NOT_IMPLEMENTED,
+               "DoF 0 is row-column eliminated: the transformed matrix keeps column 0 and is not symmetric, "
+               "so PCG does not apply (use RowElimination or Penalty for that DoF)");
+  auto t_start = std::chrono::steady_clock::now();
+  afem_solver_ws* w = workspace(s);
+  const bool flex = o.method == AFEM_SOLVER_FPCG_SPAI;
+  if (flex) {
+    AFEM_REQUIRE(s->block == 1, AFEM_ERR_NOT_IMPLEMENTED, "the sparse preconditioner is for scalar systems");
+    AFEM_REQUIRE(w->has_spai, AFEM_ERR_STATE,
+                 "no preconditioner values: call afem_system_set_spai or afem_spai_apply after the matrix transformation");
+  }
+  if (!o.use_initial_guess) {
+    hipLaunchKernelGGL(k_initial_guess, dim3(grid_for(s->nb_dof, 256)), dim3(256), 0, stream(), s->nb_dof,
+                       s->elim_info.p, s->elim_value.p, s->x.p);
+    check_launch("initial_guess");
+  }
+  SolveTotals t;
+  const bool on_chip = resident_ok && resident_usable(s, w, o);
+  if (on_chip && !solve_resident(s, w, o, t)) {
+    // the device could not hold every workgroup at once (another process on
+    // it, say): finish with the kernels that wait for nothing
+    afem_solver_options go = o;
+    go.use_initial_guess = 1;
+    return solve(s, go, res, false);
+  }
+  if (!on_chip)
+    solve_streaming(s, w, o, t);
   int fallback = 0;
-  if (flex && !converged && breakdown && total_iter < o.max_iter && std::isfinite(relres)) {
+  if (flex && !t.converged && t.breakdown && t.iterations < o.max_iter && std::isfinite(t.relres)) {
     // the preconditioner is not positive on some residual: finish with
     // Jacobi mixed-precision PCG from the current iterate
     afem_solver_options jo = o;
     jo.method = AFEM_SOLVER_PCG_MIXED;
     jo.preconditioner = AFEM_PRECOND_JACOBI;
     jo.use_initial_guess = 1;
-    jo.max_iter = o.max_iter - total_iter;
+    jo.max_iter = o.max_iter - t.iterations;
     afem_solve_result jr{};
-    const int rc = solve(s, jo, &jr);
+    const int rc = solve(s, jo, &jr, resident_ok);
     if (rc != AFEM_OK && rc != AFEM_ERR_NOT_CONVERGED)
       return rc;
-    total_iter += jr.iterations;
-    nb_ru += jr.reliable_updates;
-    relres = jr.relres;
-    converged = jr.converged != 0;
+    t.iterations += jr.iterations;
+    t.reliable_updates += jr.reliable_updates;
+    t.relres = jr.relres;
+    t.converged = jr.converged != 0;
     fallback = 1;
   }
   AFEM_HIP(hipStreamSynchronize(stream()));
   auto t_end = std::chrono::steady_clock::now();
   if (res) {
-    res->iterations = total_iter;
-    res->converged = converged ? 1 : 0;
-    res->reliable_updates = nb_ru;
-    res->relres = relres;
+    res->iterations = t.iterations;
+    res->converged = t.converged ? 1 : 0;
+    res->reliable_updates = t.reliable_updates;
+    res->relres = t.relres;
     res->solve_ms = std::chrono::duration<double, std::milli>(t_end - t_start).count();
     res->fallback = fallback;
   }
-  return converged ? AFEM_OK : AFEM_ERR_NOT_CONVERGED;
+  return t.converged ? AFEM_OK : AFEM_ERR_NOT_CONVERGED;
 }
 
 // ---- allocation-free FP64 PCG ---------------------------------------------------------------
@@ -2583,6 +2597,7 @@ AFEM_API int afem_system_set_spai(afem_system_t sys, const float* values)
   AFEM_HIP(hipStreamSynchronize(stream()));
   w->has_spai = true;
   w->spai_sell_valid = false;
+  w->pack.valid_prec = 0;
   AFEM_GUARD_END
 }
 

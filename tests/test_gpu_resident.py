@@ -13,7 +13,7 @@ import scipy.sparse as sp
 
 pytestmark = pytest.mark.gpu
 
-METHODS = {"fp64": 0, "cg": 2}
+METHODS = {"fp64": 0, "mixed": 1, "cg": 2}
 
 
 def device_system(A, M):
@@ -69,11 +69,11 @@ def check(A, M, method, rtol, norm=0, max_iter=20000):
 SIZES = [1, 2, 63, 64, 65, 511, 512, 513, 4097, 131072, 131073, 524289, 1179649]
 
 
-@pytest.mark.parametrize("method", ["fp64"])
+@pytest.mark.parametrize("method", ["fp64", "mixed"])
 @pytest.mark.parametrize("n", SIZES)
 def test_sizes(afem_gpu, n, method):
     print(f"[case] resident n={n} {method}", flush=True)
-    check(afem_gpu, band(n, [1, 2, 70], shift=0.3), method, 1e-9)
+    check(afem_gpu, band(n, [1, 2, 70], shift=0.3), method, 1e-9 if method == "fp64" else 1e-8)
 
 
 # pairs per row from none to more than two chunks, odd counts, and offsets
@@ -83,12 +83,12 @@ PATTERNS = {"diagonal": (300, []), "one": (1000, [1]), "three_pairs": (1000, [1,
             "twenty_pairs": (3000, list(range(1, 21))), "far": (70001, [1, 33000, 40001])}
 
 
-@pytest.mark.parametrize("method", ["fp64", "cg"])
+@pytest.mark.parametrize("method", ["fp64", "mixed", "cg"])
 @pytest.mark.parametrize("name", PATTERNS)
 def test_patterns(afem_gpu, name, method):
     n, offsets = PATTERNS[name]
     print(f"[case] resident pattern {name} {method}", flush=True)
-    check(afem_gpu, band(n, offsets, shift=0.2), method, 1e-9)
+    check(afem_gpu, band(n, offsets, shift=0.2), method, 1e-9 if method != "mixed" else 1e-8)
 
 
 @pytest.mark.parametrize("norm", [1, 2])
@@ -184,7 +184,7 @@ def test_changed_values_and_pattern(afem_gpu):
         s.apply_dirichlet(A.DIRICHLET_ROW_ELIMINATION, on, 1, 0, 0.0, 0.0)
         s.apply_matrix_transformation()
         s.apply_rhs_transformation()
-        for method in (0, 2):
+        for method in (0, 1):
             s.solve(method=method, rtol=1e-10)
             row, col, val, _ = bsr.download()
             M = sp.csr_matrix((val, col, row), shape=(X.shape[0],) * 2)
@@ -199,3 +199,53 @@ def test_changed_values_and_pattern(afem_gpu):
     s.rhs().upload(b)
     s.solve(rtol=1e-10)
     assert np.linalg.norm(b - M @ s.solution().numpy()) <= 1.01e-10 * np.linalg.norm(b)
+
+
+# the flexible method: one and four slices per wave, 16- and 32-bit offsets,
+# no off-diagonal pairs in some slices, FP32 and BF16 preconditioner values
+FLEX = {"small": (200, [1, 9]), "wave_edge": (4097, [1, 2, 64]), "rows4": (131073, [1, 2, 70]),
+        "nine_pairs": (3000, list(range(1, 10))), "far": (70001, [1, 33000, 40001]), "diagonal": (130, [])}
+
+
+@pytest.mark.parametrize("bf16", [0, 1])
+@pytest.mark.parametrize("name", FLEX)
+def test_sparse_preconditioner(afem_gpu, name, bf16):
+    """M = 2 D^-1 - D^-1 A D^-1 (positive: the spectral radius of D^-1 A is
+    below 2 for a diagonally dominant matrix); 1e-6 is above FP32's resolution
+    of the residual, where both recurrences take the same iterations."""
+    print(f"[case] resident flexible {name} bf16={bf16}", flush=True)
+    A = afem_gpu
+    n, offsets = FLEX[name]
+    M = band(n, offsets, shift=0.05)
+    M.sort_indices()
+    dinv = 1.0 / M.diagonal()
+    rid = np.repeat(np.arange(n), np.diff(M.indptr))
+    prec = np.where(M.indices == rid, dinv[rid], -M.data * dinv[rid] * dinv[M.indices]).astype(np.float32)
+    b = np.random.default_rng(1).normal(size=n)
+    its = {}
+    for lanes in (0, -2 if name != "far" else -1):
+        s, keep = device_system(A, M)
+        s.rhs().upload(b)
+        s.set_spai(A.DeviceArray.from_numpy(prec))
+        r = s.solve(method=A.SOLVER_FPCG_SPAI, rtol=1e-6, precond_bf16=bf16, spmv_lanes=lanes)
+        assert r.converged and not r.fallback
+        assert np.linalg.norm(b - M @ s.solution().numpy()) <= 1.01e-6 * np.linalg.norm(b)
+        its[lanes] = r.iterations
+    a, g = its[0], its[min(its)]
+    assert abs(a - g) <= max(3, 0.05 * g), its
+
+
+def test_sparse_preconditioner_that_is_not_positive_falls_back(afem_gpu):
+    print("[case] resident flexible fallback", flush=True)
+    A = afem_gpu
+    M = band(3000, [1, 9], shift=0.05)
+    M.sort_indices()
+    rid = np.repeat(np.arange(3000), np.diff(M.indptr))
+    prec = np.where(M.indices == rid, -1.0 / M.diagonal()[rid], 0.0).astype(np.float32)
+    b = np.random.default_rng(1).normal(size=3000)
+    s, keep = device_system(A, M)
+    s.rhs().upload(b)
+    s.set_spai(A.DeviceArray.from_numpy(prec))
+    r = s.solve(method=A.SOLVER_FPCG_SPAI, rtol=1e-8)
+    assert r.converged and r.fallback
+    assert np.linalg.norm(b - M @ s.solution().numpy()) <= 1.01e-8 * np.linalg.norm(b)
