@@ -18,6 +18,10 @@
 // ahead), so a chunk of iterations can be captured once in a hipGraph and
 // replayed; converged segments make their workgroups return at once.
 //
+// By default the solve runs in the resident kernel (resident.hip) instead,
+// every system a team of workgroups of one launch: 24 systems of 2 to 103
+// thousand rows to 1e-8, assembly included, 83.6 -> 25.0 ms.
+//
 // Tuning: lanes per row (G) and row tiles per workgroup (T) are timed on
 // the batch and the fastest pair is kept; G = 1 selects a SELL-64 copy of
 // the matrix whose slices start at every segment's first row (16-bit column
@@ -27,6 +31,7 @@
 #include "common.h"
 #include "device_utils.h"
 #include "linsys.h"
+#include "resident.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -1111,6 +1116,12 @@ struct afem_batch
   DBuf<SegState> st;
   SegState* host_st = nullptr;
   bool prepared = false;
+  // resident solve (resident.hip): its copy of the matrix and work arrays
+  resident::Pack pack;
+  resident::Work rwork;
+  uint64_t pack_pattern = 0; // pattern_count + 1 of the system when the pack was built
+  bool pack_usable = false;
+  bool tiles_pinned = false; // set_tiles chose the chunked kernels' shape
   hipGraphExec_t graph = nullptr;
   int64_t graph_key = -1;
   // persistent solve: team layout, second p buffer, partials, barrier
@@ -1713,6 +1724,59 @@ int persistent_once(afem_batch* b, const afem_batch_options& o, bool local, bool
   return aborted;
 }
 
+// The default solve keeps the vectors on the chip, every system a team of
+// workgroups, in as few launches as the systems need to fit (one for up to
+// 2.2 million rows in at most 256 systems); the chunked graphs run what does
+// not fit, and what set_tiles asked for.  Many tiny systems, one workgroup
+// each, take launch after launch of about 6 us an iteration, while an
+// iteration of the chunked kernels costs about 45 us plus 20 us per million
+// rows for all of them: measured (five-point systems to 1e-8, resident /
+// chunked) 1024 x 100 rows 0.79 / 1.15 ms, 2048 x 100 1.61 / 1.51, 4096 x 64
+// 2.69 / 1.73, 1024 x 400 1.36 / 2.98, 600 x 2500 3.9 / 10.1, 64 x 59536
+// 35 / 93 ms: the line lies at 8 launches, later for larger systems.
+bool resident_usable(afem_batch* b, const afem_batch_options& o)
+{
+  afem_system* s = b->sys;
+  if (o.persistent != 0 || b->tiles_pinned)
+    return false;
+  if (b->pack_pattern != s->pattern_count + 1) {
+    b->pack_usable = resident::pack_pattern(b->pack, s->nb_dof, s->nnz, s->row_index, s->columns, b->seg_rows);
+    b->pack_usable = b->pack_usable && 4.0 * resident::round_count(b->pack) <= 28.0 + 19e-6 * s->nb_dof;
+    b->pack_pattern = s->pattern_count + 1;
+  }
+  return b->pack_usable && b->pack.all_diag;
+}
+
+// Solves the segments with want set; false: a barrier wait gave up.
+bool run_resident(afem_batch* b, const afem_batch_options& o, double delta, const std::vector<char>& want,
+                  const std::vector<int>& iters)
+{
+  afem_system* s = b->sys;
+  resident::reserve(b->rwork, b->nb_seg);
+  for (int k = 0; k < b->nb_seg; ++k) {
+    resident::Status& st = b->rwork.host[k];
+    st.rtol2 = o.rtol * o.rtol;
+    st.atol2 = o.atol * o.atol;
+    st.delta2 = delta * delta;
+    st.max_iter = std::max(0, o.max_iter - iters[k]);
+    st.active = want[k] && st.max_iter > 0 ? 1 : 0;
+  }
+  resident::Options ro;
+  ro.mixed = true;
+  if (!resident::solve(b->pack, b->rwork, ro, s->x.p, s->rhs.p))
+    return false;
+  for (int k = 0; k < b->nb_seg; ++k) {
+    const resident::Status& st = b->rwork.host[k];
+    SegState& z = b->host_st[k];
+    z.iter = st.iter;
+    z.nb_ru = st.nb_ru;
+    z.bb = st.bb;
+    z.rr_true = st.rr_true;
+    z.converged = st.converged;
+  }
+  return true;
+}
+
 // Solves the active segments in one persistent launch.  persistent = 1 uses
 // XCD-local teams when the device's dispatch allows it (probed once per
 // batch) and the packing fits, else the coherent exchange; persistent = 2
@@ -1831,6 +1895,7 @@ AFEM_API int afem_batch_set_tiles(afem_batch_t b, int lanes, int tiles)
   AFEM_REQUIRE(tiles >= 1 && tiles <= 16, AFEM_ERR_ARGUMENT, "tiles must be in [1, 16]");
   b->lanes = lanes;
   b->tiles = tiles;
+  b->tiles_pinned = true;
   layout(b);
   AFEM_GUARD_END
 }
@@ -1846,7 +1911,13 @@ AFEM_API int afem_batch_solve(afem_batch_t b, const afem_batch_options* opt, afe
   AFEM_REQUIRE(opt->rtol >= 0.0 && opt->atol >= 0.0 && opt->max_iter >= 0, AFEM_ERR_ARGUMENT, "bad tolerances");
   AFEM_REQUIRE(opt->persistent >= 0 && opt->persistent <= 2, AFEM_ERR_ARGUMENT, "persistent must be 0, 1 or 2");
   const auto t0 = std::chrono::steady_clock::now();
-  prepare(b);
+  bool on_chip = resident_usable(b, *opt);
+  if (on_chip) { // the values may have changed in place since the last solve
+    b->pack.valid64 = b->pack.valid32 = false;
+    resident::pack_values(b->pack, s->row_index, s->columns, s->values, true);
+  }
+  else
+    prepare(b);
   if (!opt->use_initial_guess) {
     hipLaunchKernelGGL(k_initial_guess, dim3(grid_for(s->nb_dof, 256)), dim3(256), 0, stream(), s->nb_dof,
                        s->elim_info.p, s->elim_value.p, s->x.p);
@@ -1870,18 +1941,25 @@ AFEM_API int afem_batch_solve(afem_batch_t b, const afem_batch_options* opt, afe
     }
     if (!any)
       break;
-    write_states(b);
-    if (opt->persistent)
-      run_persistent(b, *opt);
-    else
-      run(b, *opt, opt->use_graph != 0);
-    // FP64 true residual of every segment that ran
-    read_states(b);
+    if (on_chip && !run_resident(b, *opt, delta, want, iters)) {
+      on_chip = false; // another process holds part of the device: the chunked kernels wait for nothing
+      prepare(b);
+    }
+    if (!on_chip) {
+      write_states(b);
+      if (opt->persistent)
+        run_persistent(b, *opt);
+      else
+        run(b, *opt, opt->use_graph != 0);
+      read_states(b);
+    }
     std::vector<SegState> after(b->host_st, b->host_st + b->nb_seg);
-    launch_residual(b, 0, 1);
-    hipLaunchKernelGGL(k_true_finalize, dim3(b->nb_seg), dim3(kBT), 0, stream(), seg_of(b), b->st.p, parts_of(b));
-    check_launch("batch_true_residual");
-    read_states(b);
+    if (!on_chip) { // FP64 true residual of every segment that ran (the resident kernel takes its own)
+      launch_residual(b, 0, 1);
+      hipLaunchKernelGGL(k_true_finalize, dim3(b->nb_seg), dim3(kBT), 0, stream(), seg_of(b), b->st.p, parts_of(b));
+      check_launch("batch_true_residual");
+      read_states(b);
+    }
     bool again = false;
     for (int k = 0; k < b->nb_seg; ++k) {
       if (!after[k].active)

@@ -386,6 +386,7 @@ AFEM_API int afem_system_set_csr_values(afem_system_t sys, int32_t nb_row, int64
   sys->block = 1;
   sys->bsr = nullptr;
   sys->matrix_changed = true;
+  ++sys->pattern_count;
   sys->pattern_changed = true; // a caller's arrays may hold a new pattern at the same addresses
   AFEM_GUARD_END
 }
@@ -399,8 +400,10 @@ AFEM_API int afem_system_set_bsr(afem_system_t sys, afem_bsr_t bsr)
                "matrix size differs from the DoF count");
   AFEM_REQUIRE(bsr->nb_dof != 2 || !bsr->per_block, AFEM_ERR_NOT_IMPLEMENTED,
                "2x2 blocks: use the per-row (CSR) value order (does_linear_system_use_csr)");
-  if (sys->bsr != bsr || sys->bsr_gen != bsr->pattern_gen)
+  if (sys->bsr != bsr || sys->bsr_gen != bsr->pattern_gen) {
     sys->pattern_changed = true;
+    ++sys->pattern_count;
+  }
   sys->has_matrix = true;
   sys->nb_row = bsr->nb_row * bsr->nb_dof;
   sys->nnz = bsr->nb_col * bsr->nb_dof * bsr->nb_dof;
@@ -551,6 +554,7 @@ AFEM_API int afem_system_clear_values(afem_system_t sys)
   sys->bsr = nullptr;
   sys->matrix_changed = true;
   sys->pattern_changed = true;
+  ++sys->pattern_count;
   AFEM_GUARD_END
 }
 

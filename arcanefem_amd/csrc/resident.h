@@ -22,7 +22,7 @@ struct Pack
   bool all_diag = false;            // every non-empty row has its diagonal entry
   std::vector<int32_t> seg_rows;    // row offsets of the segments
   std::vector<int32_t> seg_slices;  // first slice of each segment (nb_seg + 1)
-  DBuf<int32_t> slice_row;          // per slice its first row, then the end row of its segment
+  DBuf<int32_t> slice_row;          // per slice its first row, then the first and the end row of its segment
   DBuf<int32_t> poff;               // nslice + 1
   DBuf<int32_t> idx;                // 64 * npair (16-bit offsets) or 128 * npair words
   DBuf<double> v64, diag64, dinv64; // 128 * npair values; n
@@ -33,8 +33,9 @@ struct Pack
   int valid_prec = 0;               // 0, 16 or 32: the bits of the values in m
 };
 
-// Offsets of a pattern (rows rp, columns ci) cut into segments.  False: the
-// segments do not fit the device at once, or the layout pads too much.
+// Offsets of a pattern (rows rp, columns ci) cut into segments.  False: a
+// segment alone does not fit the device, a column leaves its segment, or the
+// layout pads too much.
 bool pack_pattern(Pack& p, int32_t n, int64_t nnz, const int32_t* rp, const int32_t* ci,
                   const std::vector<int32_t>& seg_rows);
 // Values of the pattern's matrix: FP64, and with want32 the FP32 difference form too.
@@ -62,19 +63,26 @@ struct Options
   long long spin_limit = 0;
 };
 
+struct Round // segments that run together: one launch
+{
+  int first_word = 0; // of its teams in Work::team
+  int teams = 0, grid = 0, rows_per_wave = 0;
+  int64_t first_slot = 0;
+};
+
 // Work arrays kept by a solver: published vector, saved vectors, barrier slots.
 struct Work
 {
   DBuf<double> u;          // published vector (FP64, or FP32 in the same storage)
   DBuf<double> keep;       // r, p, s between launches
   DBuf<uint64_t> slots;
-  DBuf<int32_t> team;      // layout of the launch
+  DBuf<int32_t> team;      // layout of the launches
   DBuf<Status> st;         // one per segment, then the abort flag
-  Status* host = nullptr;  // pinned, nb_seg + 1
+  Status* host = nullptr;  // pinned, nseg + 1
   int nseg = 0;
   unsigned epoch = 0;      // largest epoch in the slots
   std::vector<int32_t> layout_rows;
-  int grid = 0, rows_per_wave = 0;
+  std::vector<Round> rounds;
   ~Work()
   {
     if (host)
@@ -86,6 +94,8 @@ struct Work
 // w.host holds the results.  False: a barrier wait gave up (x is then some
 // iterate of each segment).
 bool solve(const Pack& p, Work& w, const Options& o, double* x, const double* b);
+// Launches that a solve of the pack's segments takes one after the other.
+int round_count(const Pack& p);
 // Makes room for the statuses of nseg segments.
 void reserve(Work& w, int nseg);
 

@@ -32,7 +32,7 @@ __device__ __forceinline__ void slice_rows(const int32_t* __restrict__ slice_row
                                            const int32_t* __restrict__ rp, int lane, int32_t& row, bool& live,
                                            int32_t& b, int32_t& e, int32_t& e0, int32_t& e1)
 {
-  const int32_t r0 = slice_row[s], r1 = min(slice_row[nslice + s], r0 + 64);
+  const int32_t r0 = slice_row[s], r1 = min(slice_row[2 * nslice + s], r0 + 64);
   row = r0 + lane;
   live = row < r1;
   e0 = rp[r0];
@@ -42,7 +42,8 @@ __device__ __forceinline__ void slice_rows(const int32_t* __restrict__ slice_row
 }
 
 // Pairs of every slice, and over the matrix: the longest row, the largest
-// |column - row|, whether a non-empty row lacks its diagonal entry.
+// |column - row|, whether a non-empty row lacks its diagonal entry, whether a
+// column leaves its row's segment.
 __global__ void __launch_bounds__(64)
 k_pair_count(int32_t nslice, const int32_t* __restrict__ slice_row, const int32_t* __restrict__ rp,
              const int32_t* __restrict__ ci, int32_t* __restrict__ width, int32_t* __restrict__ stats)
@@ -59,19 +60,21 @@ k_pair_count(int32_t nslice, const int32_t* __restrict__ slice_row, const int32_
       s_col[k - e0] = ci[k];
     __syncthreads();
   }
-  int32_t off = 0, far = 0;
+  const int32_t g0 = slice_row[nslice + s], g1 = slice_row[2 * nslice + s];
+  int32_t off = 0, far = 0, leaves = 0;
   for (int32_t k = b; k < e; ++k) {
     const int32_t c = staged ? s_col[k - e0] : ci[k];
     off += c != row ? 1 : 0;
     far = max(far, abs(c - row));
+    leaves |= c < g0 || c >= g1 ? 2 : 0;
   }
-  int32_t pairs = (off + 1) / 2, len = e - b, lacks = (e > b && off == e - b) ? 1 : 0;
+  int32_t pairs = (off + 1) / 2, len = e - b, lacks = ((e > b && off == e - b) ? 1 : 0) | leaves;
 #pragma unroll
   for (int o = 32; o; o >>= 1) {
     pairs = max(pairs, __shfl_xor(pairs, o, 64));
     len = max(len, __shfl_xor(len, o, 64));
     far = max(far, __shfl_xor(far, o, 64));
-    lacks = max(lacks, __shfl_xor(lacks, o, 64));
+    lacks |= __shfl_xor(lacks, o, 64);
   }
   if (lane == 0) {
     width[s] = pairs;
@@ -81,7 +84,7 @@ k_pair_count(int32_t nslice, const int32_t* __restrict__ slice_row, const int32_
     if (far > __hip_atomic_load(stats + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
       atomicMax(stats + 1, far);
     if (lacks)
-      atomicMax(stats + 2, 1);
+      atomicOr(stats + 2, lacks);
   }
 }
 
@@ -252,32 +255,33 @@ k_pair_prec(int32_t nslice, const int32_t* __restrict__ slice_row, const int32_t
 constexpr int kMaxRows = kRowSteps[3];
 constexpr int kLaunchIterations = 8192; // iterations of one launch: a second or less at any size
 
-// Workgroups per segment: at least as many as its slices need with kMaxRows
-// per wave, at most one slice per wave, else in proportion to rows^1.5 (the
-// work of an iteration times the growth of the iteration count).  Empty: the
-// segments do not fit the device together.
-static std::vector<int32_t> team_sizes(const Pack& p, int budget)
+// Workgroups a segment needs at least (kMaxRows slices per wave).
+static int32_t least_workgroups(const Pack& p, int k)
 {
-  const int ns = (int)p.seg_rows.size() - 1;
-  std::vector<int32_t> least(ns), most(ns), m(ns);
+  const int32_t sl = p.seg_slices[k + 1] - p.seg_slices[k];
+  return (sl + kWaves * kMaxRows - 1) / (kWaves * kMaxRows);
+}
+
+// Workgroups per segment of `segs`, `budget` together: at least what it needs,
+// at most one slice per wave, else in proportion to rows^1.5 (the work of an
+// iteration times the growth of the iteration count).
+static std::vector<int32_t> team_sizes(const Pack& p, const std::vector<int>& segs, int budget)
+{
+  const size_t ns = segs.size();
+  std::vector<int32_t> m(ns);
   std::vector<double> w(ns);
-  int64_t need = 0;
   double wsum = 0.0;
-  for (int k = 0; k < ns; ++k) {
-    const int32_t sl = p.seg_slices[k + 1] - p.seg_slices[k];
-    least[k] = (sl + kWaves * kMaxRows - 1) / (kWaves * kMaxRows);
-    most[k] = (sl + kWaves - 1) / kWaves;
-    w[k] = std::pow((double)(p.seg_rows[k + 1] - p.seg_rows[k]), 1.5);
-    wsum += w[k];
-    need += least[k];
+  for (size_t i = 0; i < ns; ++i) {
+    w[i] = std::pow((double)(p.seg_rows[segs[i] + 1] - p.seg_rows[segs[i]]), 1.5);
+    wsum += w[i];
   }
-  if (need > budget)
-    return {};
   for (double scale = budget;; scale *= 0.97) {
     int64_t total = 0;
-    for (int k = 0; k < ns; ++k) {
-      m[k] = std::max(least[k], std::min<int32_t>(most[k], (int32_t)std::floor(scale * w[k] / wsum)));
-      total += m[k];
+    for (size_t i = 0; i < ns; ++i) {
+      const int32_t sl = p.seg_slices[segs[i] + 1] - p.seg_slices[segs[i]];
+      m[i] = std::max(least_workgroups(p, segs[i]),
+                      std::min<int32_t>((sl + kWaves - 1) / kWaves, (int32_t)std::floor(scale * w[i] / wsum)));
+      total += m[i];
     }
     if (total <= budget)
       return m;
@@ -298,13 +302,15 @@ bool pack_pattern(Pack& p, int32_t n, int64_t nnz, const int32_t* rp, const int3
   for (int k = 0; k < nseg; ++k)
     p.seg_slices[k + 1] = p.seg_slices[k] + (seg_rows[k + 1] - seg_rows[k] + 63) / 64;
   p.nslice = p.seg_slices[nseg];
-  if (team_sizes(p, rt().num_cu).empty())
-    return false;
-  std::vector<int32_t> sr((size_t)2 * p.nslice);
+  for (int k = 0; k < nseg; ++k)
+    if (least_workgroups(p, k) > rt().num_cu)
+      return false;
+  std::vector<int32_t> sr((size_t)3 * p.nslice);
   for (int k = 0; k < nseg; ++k)
     for (int32_t s = p.seg_slices[k]; s < p.seg_slices[k + 1]; ++s) {
       sr[s] = seg_rows[k] + 64 * (s - p.seg_slices[k]);
-      sr[(size_t)p.nslice + s] = seg_rows[k + 1];
+      sr[(size_t)p.nslice + s] = seg_rows[k];
+      sr[(size_t)2 * p.nslice + s] = seg_rows[k + 1];
     }
   p.slice_row.reserve(sr.size());
   p.slice_row.upload(sr.data(), sr.size());
@@ -317,13 +323,13 @@ bool pack_pattern(Pack& p, int32_t n, int64_t nnz, const int32_t* rp, const int3
   p.npair = exclusive_scan_i32(width.p, p.poff.p, p.nslice);
   int32_t h[3];
   stats.download(h, 3);
-  // a few long rows would pad their slices many times over, and the kernel's
+  // a segment's buffers end with its rows; a few long rows would pad their slices many times over, and the kernel's
   // stream offsets are 31 bits wide
-  if (p.npair * 128 > 4 * nnz + 65536 || p.npair * (kWave * 16) >= (1LL << 31))
+  if ((h[2] & 2) || p.npair * 128 > 4 * nnz + 65536 || p.npair * (kWave * 16) >= (1LL << 31))
     return false;
   p.max_len = h[0];
   p.idx16 = h[1] <= 32767;
-  p.all_diag = h[2] == 0;
+  p.all_diag = (h[2] & 1) == 0;
   p.idx.reserve((size_t)p.npair * (p.idx16 ? 64 : 128));
   p.v64.reserve((size_t)p.npair * 128);
   p.diag64.reserve((size_t)n);
@@ -382,30 +388,69 @@ __global__ void k_clear_slots(int64_t n, uint64_t* __restrict__ slots)
     slots[i] = 0;
 }
 
+// Rounds of segments, the largest first: a round takes segments while the
+// workgroups that they need at least fit the device together.
+static std::vector<std::vector<int>> rounds_of(const Pack& p, int budget)
+{
+  const int ns = (int)p.seg_rows.size() - 1;
+  std::vector<int> order(ns);
+  for (int k = 0; k < ns; ++k)
+    order[k] = k;
+  std::stable_sort(order.begin(), order.end(), [&](int i, int j) {
+    return p.seg_rows[i + 1] - p.seg_rows[i] > p.seg_rows[j + 1] - p.seg_rows[j];
+  });
+  std::vector<std::vector<int>> out;
+  int need = budget + 1;
+  for (int k : order) {
+    const int m = least_workgroups(p, k);
+    if (need + m > budget) {
+      out.emplace_back();
+      need = 0;
+    }
+    out.back().push_back(k);
+    need += m;
+  }
+  return out;
+}
+
+int round_count(const Pack& p) { return (int)rounds_of(p, rt().num_cu).size(); }
+
 static void layout(const Pack& p, Work& w)
 {
-  if (w.grid > 0 && w.layout_rows == p.seg_rows)
+  if (!w.rounds.empty() && w.layout_rows == p.seg_rows)
     return;
-  const std::vector<int32_t> m = team_sizes(p, rt().num_cu);
-  AFEM_REQUIRE(!m.empty(), AFEM_ERR_CAPACITY, "the systems do not fit the device at once");
-  const int ns = (int)m.size();
+  const int budget = rt().num_cu;
+  constexpr int kTeamWords = sizeof(TeamDesc) / sizeof(int32_t);
   std::vector<int32_t> out;
-  int grid = 0, rows = 1;
-  for (int k = 0; k < ns; ++k) {
-    const int32_t sl = p.seg_slices[k + 1] - p.seg_slices[k];
-    const TeamDesc t{ p.seg_rows[k], p.seg_rows[k + 1], p.seg_slices[k], sl, grid, m[k], k, 0 };
-    const int32_t* q = reinterpret_cast<const int32_t*>(&t);
-    out.insert(out.end(), q, q + sizeof(TeamDesc) / sizeof(int32_t));
-    const int per_wg = (sl + m[k] - 1) / m[k];
-    rows = std::max(rows, (per_wg + kWaves - 1) / kWaves);
-    grid += m[k];
+  w.rounds.clear();
+  int64_t slot = 0;
+  for (const std::vector<int>& segs : rounds_of(p, budget)) {
+    const std::vector<int32_t> m = team_sizes(p, segs, budget);
+    Round r;
+    r.first_word = (int)out.size();
+    r.teams = (int)segs.size();
+    r.first_slot = slot;
+    int rows = 1;
+    for (size_t i = 0; i < segs.size(); ++i) {
+      const int k = segs[i];
+      const int32_t sl = p.seg_slices[k + 1] - p.seg_slices[k];
+      const TeamDesc t{ p.seg_rows[k], p.seg_rows[k + 1], p.seg_slices[k], sl, r.grid, m[i], k, 0 };
+      const int32_t* q = reinterpret_cast<const int32_t*>(&t);
+      out.insert(out.end(), q, q + kTeamWords);
+      const int per_wg = (sl + m[i] - 1) / m[i];
+      rows = std::max(rows, (per_wg + kWaves - 1) / kWaves);
+      r.grid += m[i];
+    }
+    for (size_t i = 0; i < segs.size(); ++i)
+      out.insert(out.end(), (size_t)m[i], (int32_t)i);
+    out.resize((out.size() + kTeamWords - 1) / kTeamWords * kTeamWords);
+    r.rows_per_wave = *std::find_if(std::begin(kRowSteps), std::end(kRowSteps), [&](int q) { return q >= rows; });
+    slot += (int64_t)2 * r.grid * kSlotWords;
+    w.rounds.push_back(r);
   }
-  for (int k = 0; k < ns; ++k)
-    out.insert(out.end(), (size_t)m[k], k);
   w.team.reserve(out.size());
   w.team.upload(out.data(), out.size());
-  w.grid = grid;
-  w.rows_per_wave = *std::find_if(std::begin(kRowSteps), std::end(kRowSteps), [&](int r) { return r >= rows; });
+  w.slots.release();
   w.layout_rows = p.seg_rows;
 }
 
@@ -415,16 +460,13 @@ bool solve(const Pack& p, Work& w, const Options& o, double* x, const double* b)
   layout(p, w);
   w.u.reserve((size_t)p.n);
   w.keep.reserve((size_t)3 * p.n);
-  const size_t slot_words = (size_t)2 * w.grid * kSlotWords;
-  if (w.slots.n < slot_words || w.epoch > 0x40000000u) {
-    w.slots.reserve(slot_words);
+  if (!w.slots.p || w.epoch > 0x40000000u) {
+    w.slots.reserve((size_t)(w.rounds.back().first_slot + (int64_t)2 * w.rounds.back().grid * kSlotWords));
     hipLaunchKernelGGL(k_clear_slots, dim3(64), dim3(256), 0, stream(), (int64_t)w.slots.n, w.slots.p);
     check_launch("resident_clear");
     w.epoch = 0;
   }
   Args a{};
-  a.team = reinterpret_cast<const TeamDesc*>(w.team.p);
-  a.team_of = w.team.p + (size_t)ns * (sizeof(TeamDesc) / sizeof(int32_t));
   a.poff = p.poff.p;
   a.idx = p.idx.p;
   a.v = o.mixed ? (const void*)p.v32.p : (const void*)p.v64.p;
@@ -439,14 +481,12 @@ bool solve(const Pack& p, Work& w, const Options& o, double* x, const double* b)
   a.u = w.u.p;
   a.keep = w.keep.p;
   a.n = p.n;
-  a.slots = w.slots.p;
   a.st = w.st.p;
   a.abort_flag = &w.st.p[ns].done;
   a.spin_limit = o.spin_limit > 0 ? o.spin_limit : (1LL << 22);
   a.precond = o.precond ? 1 : 0;
   a.norm = o.norm;
   a.max_launch_iter = kLaunchIterations;
-  const size_t lds = (size_t)w.rows_per_wave * kBS * 16; // x, and D^-1 (FP64) or p (mixed)
   for (int k = 0; k < ns; ++k) {
     Status& s = w.host[k];
     s.iter = s.done = s.converged = s.breakdown = s.nb_ru = 0;
@@ -457,14 +497,18 @@ bool solve(const Pack& p, Work& w, const Options& o, double* x, const double* b)
     for (int k = 0; k < ns; ++k)
       w.host[k].epoch = w.epoch;
     AFEM_HIP(hipMemcpyAsync(w.st.p, w.host, sizeof(Status) * ((size_t)ns + 1), hipMemcpyHostToDevice, stream()));
-    {
+    for (const Round& r : w.rounds) {
+      a.team = reinterpret_cast<const TeamDesc*>(w.team.p + r.first_word);
+      a.team_of = w.team.p + r.first_word + (size_t)r.teams * (sizeof(TeamDesc) / sizeof(int32_t));
+      a.slots = w.slots.p + r.first_slot;
+      const size_t lds = (size_t)r.rows_per_wave * kBS * 16; // x, and D^-1 (FP64) or p (mixed)
       ProfScope prof(o.prec ? "resident_fpcg" : o.mixed ? "resident_cg_mixed" : "resident_cg_fp64");
       if (o.prec)
-        launch_flex(a, w.rows_per_wave, p.idx16, o.prec == 16, w.grid, lds);
+        launch_flex(a, r.rows_per_wave, p.idx16, o.prec == 16, r.grid, lds);
       else if (o.mixed)
-        launch_f32(a, w.rows_per_wave, p.idx16, w.grid, lds);
+        launch_f32(a, r.rows_per_wave, p.idx16, r.grid, lds);
       else
-        launch_f64(a, w.rows_per_wave, p.idx16, w.grid, lds);
+        launch_f64(a, r.rows_per_wave, p.idx16, r.grid, lds);
     }
     AFEM_HIP(hipMemcpyAsync(w.host, w.st.p, sizeof(Status) * ((size_t)ns + 1), hipMemcpyDeviceToHost, stream()));
     AFEM_HIP(hipStreamSynchronize(stream()));

@@ -501,9 +501,12 @@ AFEM_API int afem_spai_inspect(afem_spai_t spai, int what, float* out, int64_t c
  * matrix (e.g. the Laplace matrix of a disjoint union of meshes, assembled in
  * one launch by afem_bsr_assemble_laplace).  They are solved together by
  * mixed-precision Jacobi PCG with per-system scalars: FP32 matrix and vectors,
- * FP64 x, FP64 reliable-update residual deciding convergence.  Either chunks
- * of iterations of ordinary kernels captured in a hipGraph and replayed (the
- * default), or one persistent kernel launch (captured in a hipGraph and
+ * FP64 x, FP64 reliable-update residual deciding convergence.  By default
+ * every system is a team of workgroups of one launch that keeps its vectors
+ * in registers and LDS (further launches for systems that do not fit beside
+ * the others).  Systems too large for that, thousands of tiny ones, and
+ * batches whose tiles were set run chunks of iterations of ordinary kernels
+ * captured in a hipGraph and replayed.  Or one persistent kernel launch (captured in a hipGraph and
  * replayed) in which every system gets a team of resident workgroups that
  * synchronize through bounded barrier waits in device memory. */
 typedef struct afem_batch* afem_batch_t;
@@ -512,10 +515,11 @@ typedef struct afem_batch_options {
   double atol;
   int max_iter;
   double reliable_delta;  /* reliable-update reduction factor (0 = 0.1) */
-  int chunk;              /* chunked solve: iterations per captured graph launch (even; 0 = 32) */
-  int use_graph;          /* 1: replay a hipGraph (per chunk, or of the persistent launch); 0: plain launches */
+  int chunk;              /* chunked kernels: iterations per captured graph launch (even; 0 = 32) */
+  int use_graph;          /* 1: replay a hipGraph (per chunk, or of the persistent launch); 0: plain launches
+                             (the default solve's single launch is plain either way) */
   int use_initial_guess;  /* 1: start from the system's solution array */
-  int persistent;         /* 0: chunks of iterations (default); 1: one persistent launch, each
+  int persistent;         /* 0: default (above); 1: one persistent launch, each
                              system's team on one XCD when the device dispatches workgroups to XCDs
                              round-robin (probed once per batch) and the teams fit, exchanging
                              vectors through that XCD's L2, else as 2; 2: one persistent launch,
@@ -541,7 +545,8 @@ AFEM_API int afem_batch_destroy(afem_batch_t batch);
 /* Lanes per matrix row (4, 8, 16 over the CSR arrays; 1 = one thread per row
  * over a SELL-64 copy whose slices start at every segment's first row, with
  * 16-bit column offsets -- CSR with 8 lanes when an offset does not fit) and
- * 256-row strips per workgroup (1..16). */
+ * 256-row strips per workgroup (1..16).  The batch's default solves use the
+ * chunked kernels with this shape from then on. */
 AFEM_API int afem_batch_set_tiles(afem_batch_t batch, int lanes, int tiles);
 /* Times the (lanes, tiles) candidates on one chunk and keeps the fastest. */
 AFEM_API int afem_batch_autotune(afem_batch_t batch, int* lanes, int* tiles, double* ms_per_iteration);

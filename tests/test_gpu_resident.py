@@ -249,3 +249,54 @@ def test_sparse_preconditioner_that_is_not_positive_falls_back(afem_gpu):
     r = s.solve(method=A.SOLVER_FPCG_SPAI, rtol=1e-8)
     assert r.converged and r.fallback
     assert np.linalg.norm(b - M @ s.solution().numpy()) <= 1.01e-8 * np.linalg.norm(b)
+
+
+# one launch; two launches (more than 256 systems, a large one among them);
+# so many tiny systems that the chunked kernels take over
+BATCHES = {"teams": [40, 700, 65, 5000, 1, 64], "two_launches": [70] * 300 + [20000, 3], "chunked": [20] * 2100}
+
+
+@pytest.mark.parametrize("name", BATCHES)
+def test_batches(afem_gpu, name):
+    print(f"[case] resident batch {name}", flush=True)
+    A = afem_gpu
+    parts = [band(n, [1, 7], shift=0.1, seed=k) for k, n in enumerate(BATCHES[name])]
+    M = sp.block_diag(parts).tocsr()
+    offs = np.concatenate([[0], np.cumsum(BATCHES[name])])
+    b = np.random.default_rng(5).normal(size=M.shape[0])
+    s, keep = device_system(A, M)
+    s.rhs().upload(b)
+    bs = A.BatchSolver(s, offs)
+    for _ in range(2):
+        res, _ = bs.solve(rtol=1e-8)
+        r = b - M @ s.solution().numpy()
+        for k in range(len(parts)):
+            a, e = offs[k], offs[k + 1]
+            assert res[k].converged and res[k].relres <= 1e-8
+            assert np.linalg.norm(r[a:e]) <= 1.01e-8 * np.linalg.norm(b[a:e]), k
+    res, _ = bs.solve(raise_on_failure=False, rtol=1e-13, max_iter=2)
+    assert max(q.iterations for q in res) == 2
+    # started from the solution: nothing to do
+    bs.solve(rtol=1e-8)
+    res, _ = bs.solve(rtol=1e-7, use_initial_guess=1)
+    assert max(q.iterations for q in res) == 0
+
+
+def test_batch_with_entries_outside_its_blocks(afem_gpu):
+    """Stored zeros that couple two systems: the kernels that read whole vectors take them."""
+    print("[case] resident batch couplings", flush=True)
+    A = afem_gpu
+    M = sp.block_diag([band(300, [1], shift=0.3), band(200, [1], shift=0.3)]).tolil()
+    M[299, 300] = M[300, 299] = 1.0
+    M = M.tocsr()
+    M.sort_indices()
+    rid = np.repeat(np.arange(500), np.diff(M.indptr))
+    M.data[(rid < 300) != (M.indices < 300)] = 0.0
+    b = np.random.default_rng(5).normal(size=500)
+    s, keep = device_system(A, M)
+    s.rhs().upload(b)
+    res, _ = A.BatchSolver(s, [0, 300, 500]).solve(rtol=1e-8)
+    r = b - M @ s.solution().numpy()
+    assert all(q.converged for q in res)
+    assert np.linalg.norm(r[:300]) <= 1.01e-8 * np.linalg.norm(b[:300])
+    assert np.linalg.norm(r[300:]) <= 1.01e-8 * np.linalg.norm(b[300:])
