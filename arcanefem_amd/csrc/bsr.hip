@@ -1315,6 +1315,7 @@ static void build_brick_plan(afem_bsr* b)
 {
   const afem_mesh& m = *b->mesh;
   auto release_all = [b]() {
+    b->border.release();
     b->bperm.release();
     b->bval_off.release();
     b->btotal.release();
@@ -1349,17 +1350,19 @@ static void build_brick_plan(afem_bsr* b)
     }
   DBuf<uint64_t> code((size_t)n), code2((size_t)n);
   DBuf<int32_t> node((size_t)n);
+  b->border.alloc((size_t)n);
   b->bperm.alloc((size_t)n);
   hipLaunchKernelGGL(k_morton, dim3(grid_for(n, 256)), dim3(256), 0, stream(), m.coords.p, n,
                      make_double3(lo[0], lo[1], lo[2]), make_double3(hi[0] - lo[0], hi[1] - lo[1], hi[2] - lo[2]),
                      code.p, node.p);
   check_launch("morton");
   size_t tmp_bytes = 0;
-  AFEM_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp_bytes, code.p, code2.p, node.p, b->bperm.p, n, 0, 63,
+  AFEM_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp_bytes, code.p, code2.p, node.p, b->border.p, n, 0, 63,
                                               stream()));
   DBuf<unsigned char> tmp(std::max<size_t>(tmp_bytes, 1));
-  AFEM_HIP(hipcub::DeviceRadixSort::SortPairs(tmp.p, tmp_bytes, code.p, code2.p, node.p, b->bperm.p, n, 0, 63,
+  AFEM_HIP(hipcub::DeviceRadixSort::SortPairs(tmp.p, tmp_bytes, code.p, code2.p, node.p, b->border.p, n, 0, 63,
                                               stream()));
+  AFEM_HIP(hipMemcpyAsync(b->bperm.p, b->border.p, sizeof(int32_t) * (size_t)n, hipMemcpyDeviceToDevice, stream()));
   const int32_t nblk = (n + kLocalRows - 1) / kLocalRows;
   hipLaunchKernelGGL(k_sort_brick_rows, dim3(nblk), dim3(kLocalRows), 0, stream(), b->bperm.p, n);
   check_launch("sort_brick_rows");

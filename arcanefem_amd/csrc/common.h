@@ -231,6 +231,7 @@ struct afem_bsr
   afem::DBuf<int32_t> lcell_sl;      // cell id of each sliced word
   afem::DBuf<int64_t> slice;         // per block of rows: first sliced word
   // brick order (Morton order of the nodes, blocks of 256 rows)
+  afem::DBuf<int32_t> border;        // rows in Morton order
   afem::DBuf<int32_t> bperm;         // rows in brick order
   afem::DBuf<int32_t> bval_off;      // LDS offset of each row within its brick
   afem::DBuf<int32_t> btotal;        // values per brick

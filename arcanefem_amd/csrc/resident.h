@@ -24,6 +24,8 @@ struct Pack
   std::vector<int32_t> seg_slices;  // first slice of each segment (nb_seg + 1)
   DBuf<int32_t> slice_row;          // per slice its first row, then the first and the end row of its segment
   DBuf<int32_t> poff;               // nslice + 1
+  DBuf<int32_t> perm, inv;          // row of the matrix at each place, and back (empty: in order)
+  DBuf<int32_t> src;                // with perm: 128 * npair positions in the CSR arrays (-1: padding)
   DBuf<int32_t> idx;                // 64 * npair (16-bit offsets) or 128 * npair words
   DBuf<double> v64, diag64, dinv64; // 128 * npair values; n
   DBuf<float> v32, diag32, dinv32;  // difference form: off-diagonal entries rounded, diag32 the row sum
@@ -35,9 +37,10 @@ struct Pack
 
 // Offsets of a pattern (rows rp, columns ci) cut into segments.  False: a
 // segment alone does not fit the device, a column leaves its segment, or the
-// layout pads too much.
+// layout pads too much.  `order` (device, may be null): a permutation of the
+// rows by locality, used when neighbouring rows have unrelated columns.
 bool pack_pattern(Pack& p, int32_t n, int64_t nnz, const int32_t* rp, const int32_t* ci,
-                  const std::vector<int32_t>& seg_rows);
+                  const std::vector<int32_t>& seg_rows, const int32_t* order = nullptr);
 // Values of the pattern's matrix: FP64, and with want32 the FP32 difference form too.
 void pack_values(Pack& p, const int32_t* rp, const int32_t* ci, const double* v, bool want32);
 
@@ -75,6 +78,7 @@ struct Work
 {
   DBuf<double> u;          // published vector (FP64, or FP32 in the same storage)
   DBuf<double> keep;       // r, p, s between launches
+  DBuf<double> xb;         // x and b in the pack's order
   DBuf<uint64_t> slots;
   DBuf<int32_t> team;      // layout of the launches
   DBuf<Status> st;         // one per segment, then the abort flag

@@ -43,7 +43,8 @@ __device__ __forceinline__ void slice_rows(const int32_t* __restrict__ slice_row
 
 // Pairs of every slice, and over the matrix: the longest row, the largest
 // |column - row|, whether a non-empty row lacks its diagonal entry, whether a
-// column leaves its row's segment.
+// column leaves its row's segment, and the number of slices in most of whose
+// entries neighbouring rows have unrelated columns.
 __global__ void __launch_bounds__(64)
 k_pair_count(int32_t nslice, const int32_t* __restrict__ slice_row, const int32_t* __restrict__ rp,
              const int32_t* __restrict__ ci, int32_t* __restrict__ width, int32_t* __restrict__ stats)
@@ -68,6 +69,13 @@ k_pair_count(int32_t nslice, const int32_t* __restrict__ slice_row, const int32_
     far = max(far, abs(c - row));
     leaves |= c < g0 || c >= g1 ? 2 : 0;
   }
+  // entry j of this row against entry j of the row before: within a cache line or not
+  const int32_t pb = __shfl_up(b, 1, 64), plen = __shfl_up(e, 1, 64) - pb;
+  int32_t near = 0, both = lane > 0 && live ? min(e - b, plen) : 0;
+  for (int32_t j = 0; j < both; ++j) {
+    const int32_t c = staged ? s_col[b + j - e0] : ci[b + j], d = staged ? s_col[pb + j - e0] : ci[pb + j];
+    near += abs(c - d) <= 8 ? 1 : 0;
+  }
   int32_t pairs = (off + 1) / 2, len = e - b, lacks = ((e > b && off == e - b) ? 1 : 0) | leaves;
 #pragma unroll
   for (int o = 32; o; o >>= 1) {
@@ -75,6 +83,8 @@ k_pair_count(int32_t nslice, const int32_t* __restrict__ slice_row, const int32_
     len = max(len, __shfl_xor(len, o, 64));
     far = max(far, __shfl_xor(far, o, 64));
     lacks |= __shfl_xor(lacks, o, 64);
+    near += __shfl_xor(near, o, 64);
+    both += __shfl_xor(both, o, 64);
   }
   if (lane == 0) {
     width[s] = pairs;
@@ -85,8 +95,189 @@ k_pair_count(int32_t nslice, const int32_t* __restrict__ slice_row, const int32_
       atomicMax(stats + 1, far);
     if (lacks)
       atomicOr(stats + 2, lacks);
+    if (2 * near < both)
+      atomicAdd(stats + 3, 1);
   }
 }
+
+// ---- the same in another order of the rows ------------------------------------------------------
+//
+// Place i holds row perm[i], and its columns are places (inv).  A row's
+// entries are taken in the order of their places, so that neighbouring rows
+// read neighbouring elements; src keeps where they came from.
+
+__global__ void k_invert(int32_t n, const int32_t* __restrict__ perm, int32_t* __restrict__ inv)
+{
+  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n)
+    inv[perm[i]] = i;
+}
+
+__global__ void __launch_bounds__(64)
+k_pairp_count(int32_t nslice, int32_t n, const int32_t* __restrict__ perm, const int32_t* __restrict__ inv,
+              const int32_t* __restrict__ rp, const int32_t* __restrict__ ci, int32_t* __restrict__ width,
+              int32_t* __restrict__ stats)
+{
+  const int32_t s = blockIdx.x;
+  const int32_t i = s * 64 + threadIdx.x;
+  const int32_t row = i < n ? perm[i] : -1;
+  const int32_t b = row >= 0 ? rp[row] : 0, e = row >= 0 ? rp[row + 1] : 0;
+  int32_t off = 0, far = 0;
+  for (int32_t k = b; k < e; ++k) {
+    const int32_t c = ci[k];
+    off += c != row ? 1 : 0;
+    far = max(far, abs(inv[c] - i));
+  }
+  int32_t pairs = (off + 1) / 2;
+#pragma unroll
+  for (int o = 32; o; o >>= 1) {
+    pairs = max(pairs, __shfl_xor(pairs, o, 64));
+    far = max(far, __shfl_xor(far, o, 64));
+  }
+  if (threadIdx.x == 0) {
+    width[s] = pairs;
+    if (far > __hip_atomic_load(stats + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(stats + 1, far);
+  }
+}
+
+template <class I>
+__global__ void __launch_bounds__(64)
+k_pairp_index(int32_t n, const int32_t* __restrict__ perm, const int32_t* __restrict__ inv,
+              const int32_t* __restrict__ rp, const int32_t* __restrict__ ci, const int32_t* __restrict__ poff,
+              I* __restrict__ idx, int32_t* __restrict__ src)
+{
+  typedef I I2 __attribute__((ext_vector_type(2)));
+  const int32_t s = blockIdx.x;
+  const int lane = threadIdx.x;
+  const int32_t i = s * 64 + lane;
+  const int32_t row = i < n ? perm[i] : -1;
+  const int32_t b = row >= 0 ? rp[row] : 0, e = row >= 0 ? rp[row + 1] : 0;
+  // (place, position) taken last: equal columns keep their CSR order
+  int32_t place = -1, pos = -1;
+  auto next = [&](int32_t& from) -> I {
+    int32_t best = 0x7fffffff, at = -1;
+    for (int32_t k = b; k < e; ++k) {
+      const int32_t c = ci[k];
+      if (c == row)
+        continue;
+      const int32_t q = inv[c];
+      if ((q > place || (q == place && k > pos)) && q < best) {
+        best = q;
+        at = k;
+      }
+    }
+    from = at;
+    if (at < 0)
+      return (I)0;
+    place = best;
+    pos = at;
+    return (I)(best - i);
+  };
+  const int64_t at = (int64_t)poff[s] * 64 + lane;
+  const int w = poff[s + 1] - poff[s];
+  for (int q = 0; q < w; ++q) {
+    int2 f;
+    I2 d;
+    d.x = next(f.x);
+    d.y = next(f.y);
+    reinterpret_cast<I2*>(idx)[at + (int64_t)q * 64] = d;
+    reinterpret_cast<int2*>(src)[at + (int64_t)q * 64] = f;
+  }
+}
+
+template <bool WANT32>
+__global__ void __launch_bounds__(64)
+k_pairp_values(int32_t n, const int32_t* __restrict__ perm, const int32_t* __restrict__ rp,
+               const int32_t* __restrict__ ci, const double* __restrict__ v, const int32_t* __restrict__ poff,
+               const int32_t* __restrict__ src, double* __restrict__ v64, double* __restrict__ diag64,
+               double* __restrict__ dinv64, float* __restrict__ v32, float* __restrict__ diag32,
+               float* __restrict__ dinv32)
+{
+  const int32_t s = blockIdx.x;
+  const int lane = threadIdx.x;
+  const int32_t i = s * 64 + lane;
+  const int64_t at = (int64_t)poff[s] * 64 + lane;
+  const int w = poff[s + 1] - poff[s];
+  for (int q = 0; q < w; ++q) {
+    const int2 f = reinterpret_cast<const int2*>(src)[at + (int64_t)q * 64];
+    const double x = f.x >= 0 ? v[f.x] : 0.0, y = f.y >= 0 ? v[f.y] : 0.0;
+    reinterpret_cast<double2*>(v64)[at + (int64_t)q * 64] = make_double2(x, y);
+    if constexpr (WANT32)
+      reinterpret_cast<float2*>(v32)[at + (int64_t)q * 64] = make_float2((float)x, (float)y);
+  }
+  if (i >= n)
+    return;
+  const int32_t row = perm[i];
+  double diag = 0.0, sum = 0.0;
+  for (int32_t k = rp[row]; k < rp[row + 1]; ++k) {
+    sum += v[k];
+    diag += ci[k] == row ? v[k] : 0.0;
+  }
+  const double inv = diag != 0.0 ? 1.0 / diag : 1.0;
+  diag64[i] = diag;
+  dinv64[i] = inv;
+  if constexpr (WANT32) {
+    diag32[i] = (float)sum;
+    dinv32[i] = (float)inv;
+  }
+}
+
+__device__ __forceinline__ uint32_t prec_bits(float f, bool bf16)
+{
+  const uint32_t u = __float_as_uint(f);
+  if (!bf16)
+    return u;
+  return (u & 0x7fffffffu) > 0x7f800000u ? 0x7fc00000u : (u + 0x7fffu + ((u >> 16) & 1u)) & 0xffff0000u;
+}
+
+template <bool BF16>
+__global__ void __launch_bounds__(64)
+k_pairp_prec(int32_t n, const int32_t* __restrict__ perm, const int32_t* __restrict__ rp,
+             const int32_t* __restrict__ ci, const float* __restrict__ v, const int32_t* __restrict__ poff,
+             const int32_t* __restrict__ src, uint32_t* __restrict__ out, float* __restrict__ mdiag)
+{
+  const int32_t s = blockIdx.x;
+  const int lane = threadIdx.x;
+  const int32_t i = s * 64 + lane;
+  const int64_t at = (int64_t)poff[s] * 64 + lane;
+  const int w = poff[s + 1] - poff[s];
+  for (int q = 0; q < w; ++q) {
+    const int2 f = reinterpret_cast<const int2*>(src)[at + (int64_t)q * 64];
+    const uint32_t x = f.x >= 0 ? prec_bits(v[f.x], BF16) : 0u, y = f.y >= 0 ? prec_bits(v[f.y], BF16) : 0u;
+    if constexpr (BF16)
+      out[at + (int64_t)q * 64] = (x >> 16) | y;
+    else
+      reinterpret_cast<uint2*>(out)[at + (int64_t)q * 64] = make_uint2(x, y);
+  }
+  if (i >= n)
+    return;
+  const int32_t row = perm[i];
+  float diag = 0.f;
+  for (int32_t k = rp[row]; k < rp[row + 1]; ++k)
+    diag += ci[k] == row ? __uint_as_float(prec_bits(v[k], BF16)) : 0.f;
+  mdiag[i] = diag;
+}
+
+__global__ void k_permute_in(int32_t n, const int32_t* __restrict__ perm, const double* __restrict__ x,
+                             const double* __restrict__ b, double* __restrict__ xp, double* __restrict__ bp)
+{
+  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) {
+    xp[i] = x[perm[i]];
+    bp[i] = b[perm[i]];
+  }
+}
+
+__global__ void k_permute_out(int32_t n, const int32_t* __restrict__ perm, const double* __restrict__ xp,
+                              double* __restrict__ x)
+{
+  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n)
+    x[perm[i]] = xp[i];
+}
+
+// ---- offsets and values in the matrix's own order -----------------------------------------------
 
 template <class I>
 __global__ void __launch_bounds__(64)
@@ -216,19 +407,12 @@ k_pair_prec(int32_t nslice, const int32_t* __restrict__ slice_row, const int32_t
     }
     __syncthreads();
   }
-  auto bits = [](float f) -> uint32_t {
-    const uint32_t u = __float_as_uint(f);
-    if constexpr (BF16)
-      return (u & 0x7fffffffu) > 0x7f800000u ? 0x7fc00000u : (u + 0x7fffu + ((u >> 16) & 1u)) & 0xffff0000u;
-    else
-      return u;
-  };
   float diag = 0.f;
   int32_t k = b;
   auto next = [&]() -> uint32_t {
     while (k < e) {
       const int32_t c = staged ? s_col[k - e0] : ci[k];
-      const uint32_t a = bits(staged ? s_val[k - e0] : v[k]);
+      const uint32_t a = prec_bits(staged ? s_val[k - e0] : v[k], BF16);
       ++k;
       if (c != row)
         return a;
@@ -253,6 +437,7 @@ k_pair_prec(int32_t nslice, const int32_t* __restrict__ slice_row, const int32_t
 // ---- launch layout ------------------------------------------------------------------------------
 
 constexpr int kMaxRows = kRowSteps[3];
+constexpr int kFewestSlices = kWaves; // per workgroup
 constexpr int kLaunchIterations = 8192; // iterations of one launch: a second or less at any size
 
 // Workgroups a segment needs at least (kMaxRows slices per wave).
@@ -280,7 +465,7 @@ static std::vector<int32_t> team_sizes(const Pack& p, const std::vector<int>& se
     for (size_t i = 0; i < ns; ++i) {
       const int32_t sl = p.seg_slices[segs[i] + 1] - p.seg_slices[segs[i]];
       m[i] = std::max(least_workgroups(p, segs[i]),
-                      std::min<int32_t>((sl + kWaves - 1) / kWaves, (int32_t)std::floor(scale * w[i] / wsum)));
+                      std::min<int32_t>((sl + kFewestSlices - 1) / kFewestSlices, (int32_t)std::floor(scale * w[i] / wsum)));
       total += m[i];
     }
     if (total <= budget)
@@ -291,7 +476,7 @@ static std::vector<int32_t> team_sizes(const Pack& p, const std::vector<int>& se
 // ---- building the pair layout -------------------------------------------------------------------
 
 bool pack_pattern(Pack& p, int32_t n, int64_t nnz, const int32_t* rp, const int32_t* ci,
-                  const std::vector<int32_t>& seg_rows)
+                  const std::vector<int32_t>& seg_rows, const int32_t* order)
 {
   p.n = n;
   p.valid64 = p.valid32 = false;
@@ -314,15 +499,34 @@ bool pack_pattern(Pack& p, int32_t n, int64_t nnz, const int32_t* rp, const int3
     }
   p.slice_row.reserve(sr.size());
   p.slice_row.upload(sr.data(), sr.size());
-  DBuf<int32_t> width((size_t)p.nslice), stats(3);
+  DBuf<int32_t> width((size_t)p.nslice), stats(4);
   stats.zero();
   hipLaunchKernelGGL(k_pair_count, dim3(p.nslice), dim3(64), 0, stream(), p.nslice, p.slice_row.p, rp, ci, width.p,
                      stats.p);
   check_launch("pair_count");
+  int32_t h[4];
+  stats.download(h, 4);
+  // Numbered at random (as a mesh generator's nodes come), a gather of 64 rows
+  // touches about 60 lines of the published vector; in Morton order of the
+  // nodes about 14, numbered along a grid 6 (tetrahedra, FP64, 118 thousand
+  // rows: 16.6 -> 9.9 us an iteration).  Numbered along a grid, the matrix
+  // keeps its order: Morton order would read more lines.
+  p.perm.release();
+  if (order && nseg == 1 && 2 * h[3] > p.nslice) {
+    p.perm.alloc((size_t)n);
+    p.inv.reserve((size_t)n);
+    AFEM_HIP(hipMemcpyAsync(p.perm.p, order, sizeof(int32_t) * (size_t)n, hipMemcpyDeviceToDevice, stream()));
+    hipLaunchKernelGGL(k_invert, dim3(grid_for(n, 256)), dim3(256), 0, stream(), n, p.perm.p, p.inv.p);
+    stats.zero();
+    hipLaunchKernelGGL(k_pairp_count, dim3(p.nslice), dim3(64), 0, stream(), p.nslice, n, p.perm.p, p.inv.p, rp, ci,
+                       width.p, stats.p);
+    check_launch("pairp_count");
+    int32_t far[2];
+    stats.download(far, 2);
+    h[1] = far[1];
+  }
   p.poff.reserve((size_t)p.nslice + 1);
   p.npair = exclusive_scan_i32(width.p, p.poff.p, p.nslice);
-  int32_t h[3];
-  stats.download(h, 3);
   // a segment's buffers end with its rows; a few long rows would pad their slices many times over, and the kernel's
   // stream offsets are 31 bits wide
   if ((h[2] & 2) || p.npair * 128 > 4 * nnz + 65536 || p.npair * (kWave * 16) >= (1LL << 31))
@@ -334,7 +538,17 @@ bool pack_pattern(Pack& p, int32_t n, int64_t nnz, const int32_t* rp, const int3
   p.v64.reserve((size_t)p.npair * 128);
   p.diag64.reserve((size_t)n);
   p.dinv64.reserve((size_t)n);
-  if (p.npair > 0) {
+  if (p.perm.p) {
+    p.src.reserve((size_t)p.npair * 128);
+    if (p.idx16)
+      hipLaunchKernelGGL(k_pairp_index<int16_t>, dim3(p.nslice), dim3(64), 0, stream(), n, p.perm.p, p.inv.p, rp, ci,
+                         p.poff.p, reinterpret_cast<int16_t*>(p.idx.p), p.src.p);
+    else
+      hipLaunchKernelGGL(k_pairp_index<int32_t>, dim3(p.nslice), dim3(64), 0, stream(), n, p.perm.p, p.inv.p, rp, ci,
+                         p.poff.p, p.idx.p, p.src.p);
+    check_launch("pairp_index");
+  }
+  else if (p.npair > 0) {
     if (p.idx16)
       hipLaunchKernelGGL(k_pair_index<int16_t>, dim3(p.nslice), dim3(64), 0, stream(), p.nslice, p.slice_row.p, rp,
                          ci, p.poff.p, reinterpret_cast<int16_t*>(p.idx.p));
@@ -357,7 +571,14 @@ void pack_values(Pack& p, const int32_t* rp, const int32_t* ci, const double* v,
   }
   const int stage = std::min(kStageMax, std::max(1, p.max_len) * 64);
   const size_t lds = (size_t)stage * 12;
-  if (want32)
+  if (p.perm.p && want32)
+    hipLaunchKernelGGL(k_pairp_values<true>, dim3(p.nslice), dim3(64), 0, stream(), p.n, p.perm.p, rp, ci, v, p.poff.p,
+                       p.src.p, p.v64.p, p.diag64.p, p.dinv64.p, p.v32.p, p.diag32.p, p.dinv32.p);
+  else if (p.perm.p)
+    hipLaunchKernelGGL(k_pairp_values<false>, dim3(p.nslice), dim3(64), 0, stream(), p.n, p.perm.p, rp, ci, v,
+                       p.poff.p, p.src.p, p.v64.p, p.diag64.p, p.dinv64.p, (float*)nullptr, (float*)nullptr,
+                       (float*)nullptr);
+  else if (want32)
     hipLaunchKernelGGL(k_pair_values<true>, dim3(p.nslice), dim3(64), lds, stream(), p.nslice, p.slice_row.p, rp, ci,
                        v, p.poff.p, stage, p.v64.p, p.diag64.p, p.dinv64.p, p.v32.p, p.diag32.p, p.dinv32.p);
   else
@@ -478,6 +699,14 @@ bool solve(const Pack& p, Work& w, const Options& o, double* x, const double* b)
   a.diag64 = p.diag64.p;
   a.x = x;
   a.b = b;
+  if (p.perm.p) {
+    w.xb.reserve((size_t)2 * p.n);
+    a.x = w.xb.p;
+    a.b = w.xb.p + p.n;
+    hipLaunchKernelGGL(k_permute_in, dim3(grid_for(p.n, 256)), dim3(256), 0, stream(), p.n, p.perm.p, x, b, w.xb.p,
+                       w.xb.p + p.n);
+    check_launch("permute_in");
+  }
   a.u = w.u.p;
   a.keep = w.keep.p;
   a.n = p.n;
@@ -510,6 +739,10 @@ bool solve(const Pack& p, Work& w, const Options& o, double* x, const double* b)
       else
         launch_f64(a, r.rows_per_wave, p.idx16, r.grid, lds);
     }
+    if (p.perm.p) {
+      hipLaunchKernelGGL(k_permute_out, dim3(grid_for(p.n, 256)), dim3(256), 0, stream(), p.n, p.perm.p, a.x, x);
+      check_launch("permute_out");
+    }
     AFEM_HIP(hipMemcpyAsync(w.host, w.st.p, sizeof(Status) * ((size_t)ns + 1), hipMemcpyDeviceToHost, stream()));
     AFEM_HIP(hipStreamSynchronize(stream()));
     if (w.host[ns].done) { // a wait gave up: slots of unknown epochs
@@ -535,7 +768,13 @@ void pack_prec(Pack& p, const int32_t* rp, const int32_t* ci, const float* v, in
   p.mdiag.reserve((size_t)p.n);
   const int stage = std::min(kStageMax, std::max(1, p.max_len) * 64);
   const size_t lds = (size_t)stage * 8;
-  if (bits == 16)
+  if (p.perm.p && bits == 16)
+    hipLaunchKernelGGL(k_pairp_prec<true>, dim3(p.nslice), dim3(64), 0, stream(), p.n, p.perm.p, rp, ci, v, p.poff.p,
+                       p.src.p, p.m.p, p.mdiag.p);
+  else if (p.perm.p)
+    hipLaunchKernelGGL(k_pairp_prec<false>, dim3(p.nslice), dim3(64), 0, stream(), p.n, p.perm.p, rp, ci, v, p.poff.p,
+                       p.src.p, p.m.p, p.mdiag.p);
+  else if (bits == 16)
     hipLaunchKernelGGL(k_pair_prec<true>, dim3(p.nslice), dim3(64), lds, stream(), p.nslice, p.slice_row.p, rp, ci, v,
                        p.poff.p, stage, p.m.p, p.mdiag.p);
   else

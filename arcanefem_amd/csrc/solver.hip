@@ -2062,7 +2062,9 @@ static bool resident_usable(afem_system* s, afem_solver_ws* w, const afem_solver
   if (s->block != 1 || o.spmv_lanes != 0 || w->forced_format)
     return false;
   if (!w->pack_valid) {
-    w->pack_usable = resident::pack_pattern(w->pack, s->nb_dof, s->nnz, s->row_index, s->columns, { 0, s->nb_dof });
+    const int32_t* order = s->bsr && s->bsr->border.n == (size_t)s->nb_dof ? s->bsr->border.p : nullptr;
+    w->pack_usable =
+      resident::pack_pattern(w->pack, s->nb_dof, s->nnz, s->row_index, s->columns, { 0, s->nb_dof }, order);
     w->pack_valid = true;
   }
   const bool fp64 = o.method == AFEM_SOLVER_PCG_FP64 || o.method == AFEM_SOLVER_CG_FP64;

@@ -300,3 +300,39 @@ def test_batch_with_entries_outside_its_blocks(afem_gpu):
     assert all(q.converged for q in res)
     assert np.linalg.norm(r[:300]) <= 1.01e-8 * np.linalg.norm(b[:300])
     assert np.linalg.norm(r[300:]) <= 1.01e-8 * np.linalg.norm(b[300:])
+
+
+@pytest.mark.parametrize("cell,n", [("tri", 5), ("tri", 40), ("tet", 4), ("tet", 13)])
+def test_random_numbering(afem_gpu, cell, n):
+    """Rows numbered at random are solved in the Morton order that the
+    assembly left; the solution comes back in the caller's order, for new
+    values too, and for the preconditioner's values."""
+    print(f"[case] resident shuffled {cell} {n}", flush=True)
+    A = afem_gpu
+    dim = 2 if cell == "tri" else 3
+    X, C = A.box_mesh(dim, n, 0.15, seed=3)
+    order = np.random.default_rng(4).permutation(X.shape[0]).astype(np.int32)
+    Y = np.empty_like(X)
+    Y[order] = X
+    C = np.where(C >= 0, order[np.maximum(C, 0)], -1).astype(np.int32)
+    mesh = A.Mesh(dim, Y, C)
+    bsr = A.BSRFormat(mesh, 1, use_csr=True)
+    bsr.compute_sparsity()
+    s = A.DoFLinearSystem(Y.shape[0])
+    on = np.nonzero(Y[:, dim - 1] == 0.0)[0].astype(np.int32)
+    for lam in (1.0, 3.0):
+        bsr.assemble_laplace(A.DeviceArray.from_numpy(np.full(C.shape[0], lam)), 1.0, s.rhs())
+        s.set_bsr(bsr)
+        s.apply_dirichlet(A.DIRICHLET_ROW_ELIMINATION, on, 1, 0, 0.5, 0.0)
+        s.apply_matrix_transformation()
+        s.apply_rhs_transformation()
+        row, col, val, _ = bsr.download()
+        M = sp.csr_matrix((val, col, row), shape=(Y.shape[0],) * 2)
+        b = s.rhs().numpy()
+        d = M.diagonal()
+        rid = np.repeat(np.arange(Y.shape[0]), np.diff(row))
+        s.set_spai(A.DeviceArray.from_numpy(np.where(col == rid, 1.0 / d[rid], 0.0).astype(np.float32)))
+        for kw in (dict(method=0), dict(method=1), dict(method=3, precond_bf16=0), dict(method=3, precond_bf16=1)):
+            r = s.solve(rtol=1e-8, **kw)
+            assert np.linalg.norm(b - M @ s.solution().numpy()) <= 1.01e-8 * np.linalg.norm(b), (lam, kw)
+            assert r.converged and not r.fallback
