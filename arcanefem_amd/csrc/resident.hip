@@ -7,11 +7,11 @@
 // does; larger systems move every vector through memory 11 times an
 // iteration.  Here an iteration is two barriers of 2-3 us and the matrix.
 // FP64 Jacobi-PCG, MI355X, three kernels -> resident: 256 x 256 quads of two
-// triangles (66049 rows) 16.3 -> 6.9 us an iteration; 48 x 52 x 45 nodes of
-// tetrahedra numbered at random (112 thousand rows) 22 -> 15.5 us.  Mixed
+// triangles (66049 rows) 16.3 -> 6.3 us an iteration; 48 x 52 x 45 nodes of
+// tetrahedra numbered at random (112 thousand rows) 22 -> 11.3 us.  Mixed
 // Jacobi-PCG on 128^3 hexes of six tetrahedra (2.15 million rows) to 1e-8
-// 84.9 -> 36.9 ms; flexible PCG with a BF16 sparse preconditioner on 0.89
-// million rows, assembly and inference included, 61.6 -> 27.8 ms.
+// 84.9 -> 34.8 ms; flexible PCG with a BF16 sparse preconditioner on 0.89
+// million rows, assembly and inference included, 61.6 -> 25.3 ms.
 #include "resident_kernel.h"
 
 #include <algorithm>
@@ -437,7 +437,10 @@ k_pair_prec(int32_t nslice, const int32_t* __restrict__ slice_row, const int32_t
 // ---- launch layout ------------------------------------------------------------------------------
 
 constexpr int kMaxRows = kRowSteps[3];
-constexpr int kFewestSlices = kWaves; // per workgroup
+// A workgroup takes a slice for each of its waves before a team gets another:
+// 66 thousand rows on 65 workgroups 6.3 us an iteration, on 130 7.1, on 256 8.0
+// (the barriers).
+constexpr int kFewestSlices = kWaves;
 constexpr int kLaunchIterations = 8192; // iterations of one launch: a second or less at any size
 
 // Workgroups a segment needs at least (kMaxRows slices per wave).

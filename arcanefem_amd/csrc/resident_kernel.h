@@ -7,7 +7,12 @@
 namespace afem {
 namespace resident {
 
-constexpr int kBS = 512; // threads of a workgroup: one workgroup per CU, 256 registers per lane
+// One workgroup per CU, 1024 threads of 128 registers: against 512 threads of
+// 256 registers twice the waves hide the gathers' latency (24 systems of
+// triangles 12.9 -> 10.3 us an iteration, 227 thousand rows of tetrahedra
+// FP64 13.4 -> 11.6, 2.15 million rows mixed 42.8 -> 40.4), at the price of
+// some spills at 9 slices per wave.
+constexpr int kBS = 1024;
 constexpr int kWaves = kBS / kWave;
 constexpr int kSlotWords = 8; // 64 bytes per workgroup and parity
 
@@ -315,7 +320,7 @@ enum StreamKind
 };
 
 template <class T, int R, bool I16, int PREC>
-__global__ void __launch_bounds__(kBS, 2) k_cg(Args a)
+__global__ void __launch_bounds__(kBS, 4) k_cg(Args a)
 {
   using V2 = ValuePair<T>;
   using I2 = IndexPair<I16>;
@@ -323,7 +328,7 @@ __global__ void __launch_bounds__(kBS, 2) k_cg(Args a)
   constexpr bool FLEX = PREC != 0;
   static_assert(!FLEX || MIXED, "the sparse preconditioner is FP32");
   constexpr bool DLDS = !MIXED; // D^-1 in LDS and p in registers, else the other way round
-  constexpr int CP = MIXED ? 8 : 4;
+  constexpr int CP = MIXED ? 4 : (R > 5 ? 2 : 4);
   extern __shared__ __align__(16) unsigned char smem[];
 
   const int wg = (int)xcd_tile(blockIdx.x, gridDim.x);
@@ -765,7 +770,7 @@ void launch_f64(const Args& a, int rows, bool idx16, int grid, size_t lds);
 void launch_f32(const Args& a, int rows, bool idx16, int grid, size_t lds);
 void launch_flex(const Args& a, int rows, bool idx16, bool bf16, int grid, size_t lds);
 
-constexpr int kRowSteps[4] = { 1, 4, 9, 17 };
+constexpr int kRowSteps[4] = { 1, 2, 5, 9 };
 
 template <class T, int PREC, bool I16>
 inline void launch_kernel(const Args& a, int rows, int grid, size_t lds)
@@ -778,9 +783,9 @@ inline void launch_kernel(const Args& a, int rows, int grid, size_t lds)
   };
   switch (rows) {
   case 1: go(std::integral_constant<int, 1>{}); break;
-  case 4: go(std::integral_constant<int, 4>{}); break;
-  case 9: go(std::integral_constant<int, 9>{}); break;
-  default: go(std::integral_constant<int, 17>{}); break;
+  case 2: go(std::integral_constant<int, 2>{}); break;
+  case 5: go(std::integral_constant<int, 5>{}); break;
+  default: go(std::integral_constant<int, 9>{}); break;
   }
   check_launch("resident_cg");
 }

@@ -64,9 +64,9 @@ def check(A, M, method, rtol, norm=0, max_iter=20000):
     return out
 
 
-# rows around one slice, one workgroup (8 slices), one slice per wave on 256
-# CUs (131072 rows), and the first rows that need 4, 9 and 17 slices per wave
-SIZES = [1, 2, 63, 64, 65, 511, 512, 513, 4097, 131072, 131073, 524289, 1179649]
+# rows around one slice, one workgroup (16 slices), one slice per wave on 256
+# CUs (262144 rows), and the first rows that need 2, 5 and 9 slices per wave
+SIZES = [1, 2, 63, 64, 65, 1023, 1024, 1025, 4097, 131073, 262144, 262145, 524289, 1310721]
 
 
 @pytest.mark.parametrize("method", ["fp64", "mixed"])
@@ -201,9 +201,9 @@ def test_changed_values_and_pattern(afem_gpu):
     assert np.linalg.norm(b - M @ s.solution().numpy()) <= 1.01e-10 * np.linalg.norm(b)
 
 
-# the flexible method: one and four slices per wave, 16- and 32-bit offsets,
+# the flexible method: one and two slices per wave, 16- and 32-bit offsets,
 # no off-diagonal pairs in some slices, FP32 and BF16 preconditioner values
-FLEX = {"small": (200, [1, 9]), "wave_edge": (4097, [1, 2, 64]), "rows4": (131073, [1, 2, 70]),
+FLEX = {"small": (200, [1, 9]), "wave_edge": (4097, [1, 2, 64]), "rows2": (262145, [1, 2, 70]),
         "nine_pairs": (3000, list(range(1, 10))), "far": (70001, [1, 33000, 40001]), "diagonal": (130, [])}
 
 
