@@ -202,6 +202,7 @@ struct afem_mesh
   afem::DBuf<int32_t> cells;         // nb_cell * stride
   afem::DBuf<int32_t> nc_offsets;    // nb_node + 1
   afem::DBuf<int32_t> nc_items;      // cell*stride + slot, sorted by cell per node
+  mutable afem::DBuf<double> cell_work; // per-cell terms of a right-hand side
 };
 
 struct afem_bsr
@@ -305,6 +306,18 @@ struct afem_system
 };
 
 namespace afem {
+
+// Sums per-cell terms over the cells of each node (bsr.hip): term
+// nc_items[e] >> shift of the node's list, in a fixed order.
+enum NodeSum
+{
+  kNodeSet = 0,  // rhs[i * nb_dof + dof_index] = sum
+  kNodeAdd = 1,  // += sum
+  kNodeBody = 2, // rhs[3 i + k] += f_k sum
+  kNodeMass = 3  // terms (m sum_j scale u_j, m): += (sum of the first + scale u_i sum of the second) * factor
+};
+void node_sum(const afem_mesh& m, NodeSum mode, int shift, const double* terms, const double* f, const double* field,
+              double scale, double factor, int nb_dof, int dof_index, double* rhs);
 
 // Quad4 / Hexa8 meshes (q1.hip): Laplace values (and the fused constant-source
 // RHS when rhs is given) and the constant-source RHS alone.
