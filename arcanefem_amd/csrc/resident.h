@@ -1,6 +1,7 @@
-// resident.h -- conjugate gradients of scalar systems in one launch: the
-// vectors live in registers and LDS, the matrix in a pair layout read by wide
-// loads, and the workgroups meet at barriers in device memory.
+// resident.h -- conjugate gradients of scalar systems and of systems of 3x3
+// blocks in one launch: the vectors live in registers and LDS, the matrix in a
+// pair layout read by wide loads, and the workgroups meet at barriers in
+// device memory.
 #pragma once
 
 #include "common.h"
@@ -13,9 +14,13 @@ namespace resident {
 // (poff[s] + q) * 64 + l (values as two consecutive numbers, column offsets
 // col - row as two consecutive 16- or 32-bit integers; padding: value 0,
 // offset 0).  The diagonal entries are an array of their own.  Slices start
-// at the first row of every segment.
+// at the first row of every segment.  With block = 3 rows and columns are
+// nodes: a pair is two 3x3 blocks of 9 consecutive values, in pieces that a
+// wave reads 64 x 16 bytes at a time, and the arrays of the diagonal hold
+// blocks in the same kind of pieces, one per slice and lane.
 struct Pack
 {
+  int block = 1;
   int32_t n = 0, nslice = 0, max_len = 0;
   int64_t npair = 0;
   bool idx16 = false;
@@ -27,7 +32,7 @@ struct Pack
   DBuf<int32_t> perm, inv;          // row of the matrix at each place, and back (empty: in order)
   DBuf<int32_t> src;                // with perm: 128 * npair positions in the CSR arrays (-1: padding)
   DBuf<int32_t> idx;                // 64 * npair (16-bit offsets) or 128 * npair words
-  DBuf<double> v64, diag64, dinv64; // 128 * npair values; n
+  DBuf<double> v64, diag64, dinv64; // 128 * npair values; n (blocks: 9 times 128 * npair and 64 * nslice)
   DBuf<float> v32, diag32, dinv32;  // difference form: off-diagonal entries rounded, diag32 the row sum
   bool valid64 = false, valid32 = false;
   DBuf<uint32_t> m;                 // sparse preconditioner: 64 * npair words (BF16) or 128 * npair (FP32)
@@ -39,8 +44,9 @@ struct Pack
 // segment alone does not fit the device, a column leaves its segment, or the
 // layout pads too much.  `order` (device, may be null): a permutation of the
 // rows by locality, used when neighbouring rows have unrelated columns.
+// block 3 (one segment): rows and columns of nodes, nnz blocks.
 bool pack_pattern(Pack& p, int32_t n, int64_t nnz, const int32_t* rp, const int32_t* ci,
-                  const std::vector<int32_t>& seg_rows, const int32_t* order = nullptr);
+                  const std::vector<int32_t>& seg_rows, const int32_t* order = nullptr, int block = 1);
 // Values of the pattern's matrix: FP64, and with want32 the FP32 difference form too.
 void pack_values(Pack& p, const int32_t* rp, const int32_t* ci, const double* v, bool want32);
 

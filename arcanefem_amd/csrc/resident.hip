@@ -436,18 +436,19 @@ k_pair_prec(int32_t nslice, const int32_t* __restrict__ slice_row, const int32_t
 
 // ---- launch layout ------------------------------------------------------------------------------
 
-constexpr int kMaxRows = kRowSteps[3];
 // A workgroup takes a slice for each of its waves before a team gets another:
 // 66 thousand rows on 65 workgroups 6.3 us an iteration, on 130 7.1, on 256 8.0
 // (the barriers).
-constexpr int kFewestSlices = kWaves;
+static int waves_of(const Pack& p) { return p.block == 3 ? kBlockWaves : kWaves; }
+static int max_rows(const Pack& p) { return p.block == 3 ? kBlockRowSteps[2] : kRowSteps[3]; }
 constexpr int kLaunchIterations = 8192; // iterations of one launch: a second or less at any size
 
-// Workgroups a segment needs at least (kMaxRows slices per wave).
+// Workgroups a segment needs at least (max_rows slices per wave).
 static int32_t least_workgroups(const Pack& p, int k)
 {
   const int32_t sl = p.seg_slices[k + 1] - p.seg_slices[k];
-  return (sl + kWaves * kMaxRows - 1) / (kWaves * kMaxRows);
+  const int32_t most = waves_of(p) * max_rows(p);
+  return (sl + most - 1) / most;
 }
 
 // Workgroups per segment of `segs`, `budget` together: at least what it needs,
@@ -456,6 +457,7 @@ static int32_t least_workgroups(const Pack& p, int k)
 static std::vector<int32_t> team_sizes(const Pack& p, const std::vector<int>& segs, int budget)
 {
   const size_t ns = segs.size();
+  const int waves = waves_of(p);
   std::vector<int32_t> m(ns);
   std::vector<double> w(ns);
   double wsum = 0.0;
@@ -468,7 +470,7 @@ static std::vector<int32_t> team_sizes(const Pack& p, const std::vector<int>& se
     for (size_t i = 0; i < ns; ++i) {
       const int32_t sl = p.seg_slices[segs[i] + 1] - p.seg_slices[segs[i]];
       m[i] = std::max(least_workgroups(p, segs[i]),
-                      std::min<int32_t>((sl + kFewestSlices - 1) / kFewestSlices, (int32_t)std::floor(scale * w[i] / wsum)));
+                      std::min<int32_t>((sl + waves - 1) / waves, (int32_t)std::floor(scale * w[i] / wsum)));
       total += m[i];
     }
     if (total <= budget)
@@ -476,12 +478,18 @@ static std::vector<int32_t> team_sizes(const Pack& p, const std::vector<int>& se
   }
 }
 
+static size_t diagonal_values(const Pack& p)
+{
+  return p.block == 3 ? (size_t)p.nslice * 64 * 9 : (size_t)p.n;
+}
+
 // ---- building the pair layout -------------------------------------------------------------------
 
 bool pack_pattern(Pack& p, int32_t n, int64_t nnz, const int32_t* rp, const int32_t* ci,
-                  const std::vector<int32_t>& seg_rows, const int32_t* order)
+                  const std::vector<int32_t>& seg_rows, const int32_t* order, int block)
 {
   p.n = n;
+  p.block = block;
   p.valid64 = p.valid32 = false;
   p.valid_prec = 0;
   p.seg_rows = seg_rows;
@@ -532,15 +540,15 @@ bool pack_pattern(Pack& p, int32_t n, int64_t nnz, const int32_t* rp, const int3
   p.npair = exclusive_scan_i32(width.p, p.poff.p, p.nslice);
   // a segment's buffers end with its rows; a few long rows would pad their slices many times over, and the kernel's
   // stream offsets are 31 bits wide
-  if ((h[2] & 2) || p.npair * 128 > 4 * nnz + 65536 || p.npair * (kWave * 16) >= (1LL << 31))
+  if ((h[2] & 2) || p.npair * 128 > 4 * nnz + 65536 || p.npair * (kWave * 16) * (block * block) >= (1LL << 31))
     return false;
   p.max_len = h[0];
   p.idx16 = h[1] <= 32767;
   p.all_diag = (h[2] & 1) == 0;
   p.idx.reserve((size_t)p.npair * (p.idx16 ? 64 : 128));
-  p.v64.reserve((size_t)p.npair * 128);
-  p.diag64.reserve((size_t)n);
-  p.dinv64.reserve((size_t)n);
+  p.v64.reserve((size_t)p.npair * 128 * (block * block));
+  p.diag64.reserve(diagonal_values(p));
+  p.dinv64.reserve(diagonal_values(p));
   if (p.perm.p) {
     p.src.reserve((size_t)p.npair * 128);
     if (p.idx16)
@@ -568,13 +576,15 @@ void pack_values(Pack& p, const int32_t* rp, const int32_t* ci, const double* v,
   if (p.valid64 && (p.valid32 || !want32))
     return;
   if (want32) {
-    p.v32.reserve((size_t)p.npair * 128);
-    p.diag32.reserve((size_t)p.n);
-    p.dinv32.reserve((size_t)p.n);
+    p.v32.reserve((size_t)p.npair * 128 * (p.block * p.block));
+    p.diag32.reserve(diagonal_values(p));
+    p.dinv32.reserve(diagonal_values(p));
   }
   const int stage = std::min(kStageMax, std::max(1, p.max_len) * 64);
   const size_t lds = (size_t)stage * 12;
-  if (p.perm.p && want32)
+  if (p.block == 3)
+    fill_block_values(p, rp, ci, v, want32);
+  else if (p.perm.p && want32)
     hipLaunchKernelGGL(k_pairp_values<true>, dim3(p.nslice), dim3(64), 0, stream(), p.n, p.perm.p, rp, ci, v, p.poff.p,
                        p.src.p, p.v64.p, p.diag64.p, p.dinv64.p, p.v32.p, p.diag32.p, p.dinv32.p);
   else if (p.perm.p)
@@ -662,13 +672,16 @@ static void layout(const Pack& p, Work& w)
       const int32_t* q = reinterpret_cast<const int32_t*>(&t);
       out.insert(out.end(), q, q + kTeamWords);
       const int per_wg = (sl + m[i] - 1) / m[i];
-      rows = std::max(rows, (per_wg + kWaves - 1) / kWaves);
+      rows = std::max(rows, (per_wg + waves_of(p) - 1) / waves_of(p));
       r.grid += m[i];
     }
     for (size_t i = 0; i < segs.size(); ++i)
       out.insert(out.end(), (size_t)m[i], (int32_t)i);
     out.resize((out.size() + kTeamWords - 1) / kTeamWords * kTeamWords);
-    r.rows_per_wave = *std::find_if(std::begin(kRowSteps), std::end(kRowSteps), [&](int q) { return q >= rows; });
+    const auto at_least = [&](int q) { return q >= rows; };
+    r.rows_per_wave = p.block == 3
+      ? *std::find_if(std::begin(kBlockRowSteps), std::end(kBlockRowSteps), at_least)
+      : *std::find_if(std::begin(kRowSteps), std::end(kRowSteps), at_least);
     slot += (int64_t)2 * r.grid * kSlotWords;
     w.rounds.push_back(r);
   }
@@ -682,8 +695,9 @@ bool solve(const Pack& p, Work& w, const Options& o, double* x, const double* b)
 {
   const int ns = (int)p.seg_rows.size() - 1;
   layout(p, w);
-  w.u.reserve((size_t)p.n);
-  w.keep.reserve((size_t)3 * p.n);
+  const size_t dofs = (size_t)p.n * p.block;
+  w.u.reserve(dofs);
+  w.keep.reserve(3 * dofs);
   if (!w.slots.p || w.epoch > 0x40000000u) {
     w.slots.reserve((size_t)(w.rounds.back().first_slot + (int64_t)2 * w.rounds.back().grid * kSlotWords));
     hipLaunchKernelGGL(k_clear_slots, dim3(64), dim3(256), 0, stream(), (int64_t)w.slots.n, w.slots.p);
@@ -703,11 +717,14 @@ bool solve(const Pack& p, Work& w, const Options& o, double* x, const double* b)
   a.x = x;
   a.b = b;
   if (p.perm.p) {
-    w.xb.reserve((size_t)2 * p.n);
+    w.xb.reserve(2 * dofs);
     a.x = w.xb.p;
-    a.b = w.xb.p + p.n;
-    hipLaunchKernelGGL(k_permute_in, dim3(grid_for(p.n, 256)), dim3(256), 0, stream(), p.n, p.perm.p, x, b, w.xb.p,
-                       w.xb.p + p.n);
+    a.b = w.xb.p + dofs;
+    if (p.block == 3)
+      permute_blocks(p.n, p.perm.p, x, b, w.xb.p, w.xb.p + dofs);
+    else
+      hipLaunchKernelGGL(k_permute_in, dim3(grid_for(p.n, 256)), dim3(256), 0, stream(), p.n, p.perm.p, x, b, w.xb.p,
+                         w.xb.p + dofs);
     check_launch("permute_in");
   }
   a.u = w.u.p;
@@ -735,14 +752,18 @@ bool solve(const Pack& p, Work& w, const Options& o, double* x, const double* b)
       a.slots = w.slots.p + r.first_slot;
       const size_t lds = (size_t)r.rows_per_wave * kBS * 16; // x, and D^-1 (FP64) or p (mixed)
       ProfScope prof(o.prec ? "resident_fpcg" : o.mixed ? "resident_cg_mixed" : "resident_cg_fp64");
-      if (o.prec)
+      if (p.block == 3)
+        launch_block(a, o.mixed, r.rows_per_wave, p.idx16, r.grid);
+      else if (o.prec)
         launch_flex(a, r.rows_per_wave, p.idx16, o.prec == 16, r.grid, lds);
       else if (o.mixed)
         launch_f32(a, r.rows_per_wave, p.idx16, r.grid, lds);
       else
         launch_f64(a, r.rows_per_wave, p.idx16, r.grid, lds);
     }
-    if (p.perm.p) {
+    if (p.perm.p && p.block == 3)
+      unpermute_blocks(p.n, p.perm.p, a.x, x);
+    else if (p.perm.p) {
       hipLaunchKernelGGL(k_permute_out, dim3(grid_for(p.n, 256)), dim3(256), 0, stream(), p.n, p.perm.p, a.x, x);
       check_launch("permute_out");
     }

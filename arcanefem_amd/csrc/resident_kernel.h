@@ -145,11 +145,11 @@ struct Barrier
 // alternate between two sets: a set is written again only after every
 // workgroup has passed the barrier after it.  All workgroups add the slots in
 // the same order and hold the same sums.  False: a wait gave up.
-template <int NV>
+template <int NV, int WAVES = kWaves>
 __device__ __forceinline__ bool team_sum(Barrier& B, double (&v)[NV])
 {
   static_assert(2 * NV <= kSlotWords, "slot too small");
-  __shared__ double s_part[NV][kWaves];
+  __shared__ double s_part[NV][WAVES];
   __shared__ double s_tot[NV];
   __shared__ int s_ok;
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
@@ -169,7 +169,7 @@ __device__ __forceinline__ bool team_sum(Barrier& B, double (&v)[NV])
       const int q = lane >> 1;
       double s = 0.0;
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w)
+      for (int w = 0; w < WAVES; ++w)
         s += s_part[q][w];
       const uint64_t u = (uint64_t)__double_as_longlong(s);
       const uint32_t half = (lane & 1) ? (uint32_t)(u >> 32) : (uint32_t)u;
@@ -771,6 +771,15 @@ void launch_f32(const Args& a, int rows, bool idx16, int grid, size_t lds);
 void launch_flex(const Args& a, int rows, bool idx16, bool bf16, int grid, size_t lds);
 
 constexpr int kRowSteps[4] = { 1, 2, 5, 9 };
+
+// 3x3 blocks (resident_block.hip): 512 threads, for 256 registers each.
+constexpr int kBlockBS = 512;
+constexpr int kBlockWaves = kBlockBS / kWave;
+constexpr int kBlockRowSteps[3] = { 1, 2, 4 };
+void launch_block(const Args& a, bool mixed, int rows, bool idx16, int grid);
+void fill_block_values(const Pack& p, const int32_t* rp, const int32_t* ci, const double* v, bool want32);
+void permute_blocks(int32_t n, const int32_t* perm, const double* x, const double* b, double* xp, double* bp);
+void unpermute_blocks(int32_t n, const int32_t* perm, const double* xp, double* x);
 
 template <class T, int PREC, bool I16>
 inline void launch_kernel(const Args& a, int rows, int grid, size_t lds)

@@ -2054,17 +2054,19 @@ static void launch_flex_iteration(afem_system* s, afem_solver_ws* w, int k, cons
   }
 }
 
-// The resident kernel runs scalar systems whose vectors fit the device's
-// registers and LDS (2.2 million rows on 256 CUs), unless the caller pinned an
-// SpMV format; the mixed solvers' difference form needs every diagonal entry.
+// The resident kernels run systems whose vectors fit the device's registers
+// and LDS (on 256 CUs 2.36 million scalar rows, 524 thousand nodes of 3x3
+// blocks), unless the caller pinned an SpMV format; the mixed solvers'
+// difference form needs every diagonal entry.
 static bool resident_usable(afem_system* s, afem_solver_ws* w, const afem_solver_options& o)
 {
-  if (s->block != 1 || o.spmv_lanes != 0 || w->forced_format)
+  if ((s->block != 1 && s->block != 3) || o.spmv_lanes != 0 || w->forced_format)
     return false;
   if (!w->pack_valid) {
-    const int32_t* order = s->bsr && s->bsr->border.n == (size_t)s->nb_dof ? s->bsr->border.p : nullptr;
-    w->pack_usable =
-      resident::pack_pattern(w->pack, s->nb_dof, s->nnz, s->row_index, s->columns, { 0, s->nb_dof }, order);
+    const int32_t n = s->nb_dof / s->block;
+    const int32_t* order = s->bsr && s->bsr->border.n == (size_t)n ? s->bsr->border.p : nullptr;
+    w->pack_usable = resident::pack_pattern(w->pack, n, s->nnz / (s->block * s->block), s->row_index, s->columns,
+                                            { 0, n }, order, s->block);
     w->pack_valid = true;
   }
   const bool fp64 = o.method == AFEM_SOLVER_PCG_FP64 || o.method == AFEM_SOLVER_CG_FP64;
@@ -2610,7 +2612,7 @@ AFEM_API int afem_system_spmv_format(afem_system_t sys, int* format, int* lanes)
   afem_solver_ws* w = sys->ws;
   // a resident solve alone has tuned nothing: its layout is SELL-64 in pairs
   const bool pairs = w && w->format < 0 && w->pack.valid64;
-  *format = pairs ? (w->pack.idx16 ? kFmtSell16 : kFmtSell) : w ? w->format : -1;
+  *format = pairs ? (w->pack.idx16 && w->block == 1 ? kFmtSell16 : kFmtSell) : w ? w->format : -1;
   *lanes = w ? w->lanes : 0;
   AFEM_GUARD_END
 }

@@ -1,0 +1,138 @@
+"""Solves of 3x3 block systems whose vectors stay on the chip, against host
+residuals and against the kernels that keep every vector in memory (a pinned
+SpMV format selects those).
+
+Both run the same recurrences (the mixed one sums in FP64 here), so the
+iteration counts agree up to rounding in the sums: no more than 5 % (or 3 and
+one for every reliable update, each of which replaces the residual between two
+steps and may cost one) above the streaming kernels', and no less than 25 %
+below.  Residuals are
+checked on the host with the stated tolerance (1.01 x for the host's own
+rounding of b - A x).
+"""
+
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+pytestmark = pytest.mark.gpu
+
+
+def grid_mesh(counts, jitter=0.1, shuffled=False, seed=3):
+    """Tetrahedra of a box of cells with edges of 1 / counts[0]."""
+    rng = np.random.default_rng(seed)
+    nx, ny, nz = (c + 1 for c in counts)
+    z, y, x = np.meshgrid(np.arange(nz), np.arange(ny), np.arange(nx), indexing="ij")
+    X = np.stack([x.ravel(), y.ravel(), z.ravel()], axis=1).astype(np.float64)
+    X += rng.uniform(-jitter, jitter, X.shape) * (X[:, :1] > 0) * (X[:, :1] < counts[0])
+    X /= counts[0]
+    k, j, i = np.meshgrid(np.arange(counts[2]), np.arange(counts[1]), np.arange(counts[0]), indexing="ij")
+    v = (k * ny * nx + j * nx + i).ravel()
+    step = np.array([1, nx, nx * ny])
+    C = []
+    for p in ((0, 1, 2), (1, 2, 0), (2, 0, 1), (0, 2, 1), (2, 1, 0), (1, 0, 2)):
+        a, b, c = v + step[p[0]], v + step[p[0]] + step[p[1]], v + step.sum()
+        even = p in ((0, 1, 2), (1, 2, 0), (2, 0, 1))
+        C.append(np.stack([v, a, b, c] if even else [v, b, a, c], axis=1))
+    C = np.concatenate(C)
+    if shuffled:
+        perm = rng.permutation(len(X))
+        Y = np.empty_like(X)
+        Y[perm] = X
+        X, C = Y, perm[C]
+        C = C[rng.permutation(len(C))]
+    return X, C.astype(np.int32)
+
+
+def elastic_system(A, X, C, load_seed=1):
+    m = A.Mesh(3, X, C)
+    b = A.BSRFormat(m, 3)
+    b.compute_sparsity()
+    b.assemble_elasticity(1.2, 0.8)
+    s = A.DoFLinearSystem(3 * len(X))
+    s.set_bsr(b)
+    s.rhs().upload(np.random.default_rng(load_seed).normal(size=3 * len(X)))
+    fixed = np.nonzero(X[:, 0] == X[:, 0].max())[0]
+    fixed = fixed[fixed > 0]
+    for c in range(3):
+        s.apply_dirichlet(A.DIRICHLET_ROW_COLUMN_ELIMINATION, fixed, 3, c, 0.01 * c)
+    s.apply_matrix_transformation()
+    s.apply_rhs_transformation()
+    row, col, val, _ = b.download()
+    M = sp.bsr_matrix((val.reshape(-1, 3, 3), col, row), shape=(3 * len(X),) * 2)
+    return s, M, (m, b)
+
+
+def check(A, X, C, mixed, rtol, norm=0):
+    s, M, keep = elastic_system(A, X, C)
+    b = s.rhs().numpy()
+    its = {}
+    for lanes in (0, -1):
+        r = s.solve(method=A.SOLVER_PCG_MIXED if mixed else A.SOLVER_PCG_FP64, rtol=rtol, norm=norm, max_iter=20000,
+                    spmv_lanes=lanes)
+        assert r.converged
+        if norm == 0:
+            assert np.linalg.norm(b - M @ s.solution().numpy()) <= 1.01 * rtol * np.linalg.norm(b), lanes
+        its[lanes] = r.iterations
+        updates = r.reliable_updates
+    a, g = its[0], its[-1]
+    print(f"[result] {a} iterations, streaming {g}", flush=True)
+    assert 0.75 * g - 3 <= a <= max(g + 3 + updates, 1.05 * g), its
+
+
+# nodes: 12; 64 (one slice); 60 and 80; 1331 (three workgroups' worth of
+# waves); 129360 (one slice per wave), 132651 (the first that need two),
+# 274625 (four); numbered at random: in Morton order
+SIZES = {"least": (2, 1, 1), "slice": (3, 3, 3), "below": (2, 3, 4), "above": (3, 3, 4), "small": (10, 10, 10),
+         "one": (55, 41, 54), "two": (50, 50, 50), "four": (64, 64, 64)}
+
+
+@pytest.mark.parametrize("mixed", [False, True], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("name", SIZES)
+def test_sizes(afem_gpu, name, mixed):
+    print(f"[case] resident blocks {name} mixed={mixed}", flush=True)
+    X, C = grid_mesh(SIZES[name])
+    check(afem_gpu, X, C, mixed, (1e-8 if mixed else 1e-9) if len(X) < 100000 else 1e-6)
+
+
+@pytest.mark.parametrize("mixed", [False, True], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("counts", [(12, 9, 11), (40, 36, 38)])
+def test_random_numbering(afem_gpu, counts, mixed):
+    print(f"[case] resident blocks shuffled {counts} mixed={mixed}", flush=True)
+    X, C = grid_mesh(counts, shuffled=True)
+    check(afem_gpu, X, C, mixed, 1e-8)
+
+
+@pytest.mark.parametrize("norm", [1, 2])
+def test_norms(afem_gpu, norm):
+    print(f"[case] resident blocks norm {norm}", flush=True)
+    X, C = grid_mesh((7, 9, 8))
+    check(afem_gpu, X, C, False, 1e-9, norm)
+
+
+def test_more_iterations_than_one_launch(afem_gpu):
+    """A long thin bar needs far more than 8192 iterations.  The energy
+    x.Ax/2 - b.x of the iterates falls monotonically, across the launches as
+    well, and as far as the streaming kernels bring it."""
+    print("[case] resident blocks relaunch", flush=True)
+    A = afem_gpu
+    X, C = grid_mesh((1, 1, 900))
+    X = np.ascontiguousarray(X[:, ::-1])  # the bar along x, fixed at its end
+    X[:, 0] = np.round(X[:, 0], 1)
+    C = np.ascontiguousarray(C[:, [0, 2, 1, 3]])
+    s, M, keep = elastic_system(A, X, C)
+    b = s.rhs().numpy()
+
+    def energy(max_iter, lanes):
+        r = s.solve(raise_on_failure=False, method=A.SOLVER_PCG_FP64, rtol=1e-14, max_iter=max_iter, spmv_lanes=lanes)
+        x = s.solution().numpy()
+        assert r.iterations == max_iter and not r.converged
+        rel = np.linalg.norm(b - M @ x) / np.linalg.norm(b)
+        assert abs(r.relres - rel) <= 0.01 * rel
+        return x @ (0.5 * (M @ x) - b)
+
+    e1, e2, g2 = energy(8192, 0), energy(10000, 0), energy(10000, -1)
+    print(f"[result] energies {e1} {e2} streaming {g2}", flush=True)
+    assert e2 < e1 < 0 and g2 < 0
+    # rounding separates the two iterations' paths; both have gone most of the way
+    assert 0.5 <= e2 / g2 <= 2.0
