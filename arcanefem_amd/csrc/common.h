@@ -58,6 +58,12 @@ inline hipStream_t stream()
   return rt().stream;
 }
 
+// Device memory of the buffers below, kept for reuse within bounds
+// (runtime.hip).
+void* pool_alloc(size_t bytes);
+void pool_free(void* p);
+void pool_trim();
+
 // Owning device buffer.
 template <class T>
 struct DBuf
@@ -92,7 +98,7 @@ struct DBuf
     release();
     if (count) {
       ensure_init();
-      AFEM_HIP(hipMalloc(&p, count * sizeof(T)));
+      p = static_cast<T*>(pool_alloc(count * sizeof(T)));
     }
     n = count;
   }
@@ -105,7 +111,7 @@ struct DBuf
   void release()
   {
     if (p)
-      (void)hipFree(p);
+      pool_free(p);
     p = nullptr;
     n = 0;
   }
