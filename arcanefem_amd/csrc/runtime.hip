@@ -65,16 +65,18 @@ void ensure_init()
 // therefore kept, at most kPoolBytes in kPoolBlocks blocks (the oldest go back
 // to the device first; blocks above half of kPoolBytes at once), and serve
 // requests of at least four fifths of their size.  All go back when the device
-// runs out of memory and in afem_finalize.
+// runs out of memory and in afem_finalize.  Flags and short lists, below
+// kPoolLeast, go straight to the runtime, which cuts them from chunks of its
+// own (kept as well, they made gradients of 46^3 systems, 0.52 ms, 0.8 %
+// slower).
 //
 // hipFree waits for the device's work on every stream, and so does the release
 // of a kept block: work that was queued before the release never meets the
-// block's next owner, and a request waits for nothing.  (With the wait in the
-// request that takes the block, gradients of a 64^3 system, which take and
-// release a flag behind queued work, ran up to 4 % slower.)
+// block's next owner, and a request waits for nothing.
 
 constexpr size_t kPoolBytes = size_t(1) << 30;
 constexpr size_t kPoolBlocks = 512;
+constexpr size_t kPoolLeast = size_t(64) << 10;
 
 struct PoolBlock
 {
@@ -107,19 +109,37 @@ static Pool& pool()
   return *p;
 }
 
-static void trim_locked(Pool& q)
+void pool_trim()
 {
+  Pool& q = pool();
+  std::lock_guard<std::mutex> lock(q.mutex);
   while (!q.kept.empty())
     q.give_back(q.kept.begin());
 }
 
+// hipMalloc; out of memory, once more without the kept blocks.
+static void* device_malloc(size_t bytes)
+{
+  void* p = nullptr;
+  hipError_t e = hipMalloc(&p, bytes);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    pool_trim();
+    e = hipMalloc(&p, bytes);
+  }
+  AFEM_HIP(e);
+  return p;
+}
+
 void* pool_alloc(size_t bytes)
 {
+  if (bytes < kPoolLeast)
+    return device_malloc(bytes);
   Pool& q = pool();
   bytes = (bytes + 4095) / 4096 * 4096;
   int device = 0;
   AFEM_HIP(hipGetDevice(&device));
-  std::lock_guard<std::mutex> lock(q.mutex);
+  std::unique_lock<std::mutex> lock(q.mutex);
   PoolBlock b;
   auto it = q.kept.lower_bound(bytes);
   while (it != q.kept.end() && it->first <= bytes + bytes / 4 && it->second.device != device)
@@ -130,13 +150,9 @@ void* pool_alloc(size_t bytes)
     q.kept.erase(it);
   }
   else {
-    hipError_t e = hipMalloc(&b.p, bytes);
-    if (e == hipErrorOutOfMemory && !q.kept.empty()) {
-      (void)hipGetLastError();
-      trim_locked(q);
-      e = hipMalloc(&b.p, bytes);
-    }
-    AFEM_HIP(e);
+    lock.unlock();
+    b.p = device_malloc(bytes);
+    lock.lock();
     b.bytes = bytes;
     b.device = device;
   }
@@ -176,13 +192,6 @@ void pool_free(void* p)
         oldest = k;
     q.give_back(oldest);
   }
-}
-
-void pool_trim()
-{
-  Pool& q = pool();
-  std::lock_guard<std::mutex> lock(q.mutex);
-  trim_locked(q);
 }
 
 // ---- profiling ----------------------------------------------------------------
@@ -419,15 +428,8 @@ AFEM_API int afem_malloc(void** dptr, size_t bytes)
   AFEM_REQUIRE(dptr, AFEM_ERR_ARGUMENT, "null output pointer");
   ensure_init();
   *dptr = nullptr;
-  if (bytes) {
-    hipError_t e = hipMalloc(dptr, bytes);
-    if (e == hipErrorOutOfMemory) {
-      (void)hipGetLastError();
-      pool_trim();
-      e = hipMalloc(dptr, bytes);
-    }
-    AFEM_HIP(e);
-  }
+  if (bytes)
+    *dptr = device_malloc(bytes);
   AFEM_GUARD_END
 }
 
