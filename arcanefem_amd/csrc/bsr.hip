@@ -79,15 +79,21 @@ k_pattern_rows(const int32_t* __restrict__ nc_off, const int32_t* __restrict__ n
 // register slots; the group's 128 keys (padding 0x7fffffff) are sorted by a
 // bitonic network -- key g = 8 lane + slot, exchanges within a lane between
 // registers and across lanes by shuffles -- and every key that differs from
-// its predecessor is a column.  Count pass: the row length; fill pass: the
-// sorted row at row_index[i].  *overflow = 1 when a node's candidates do not
-// fit its 128 slots (the caller then runs the per-thread kernel).
+// its predecessor is a column.  Count pass: the row length, the first
+// kStageRow columns of the row at stage[kStageRow * i], and the longest row in
+// overflow[1]; fill pass: the sorted row at row_index[i].  overflow[0] = 1 when
+// a node's candidates do not fit its 128 slots (the caller then runs the
+// per-thread kernel).  Bound by the network's instructions (1400 per wave):
+// 133 us at 237 thousand nodes of tetrahedra, so the fill pass runs only for
+// rows that the stage does not hold; copying the staged rows takes 14.
 constexpr int kPatternLanes = 16, kPatternSlots = 8;
+constexpr int kStageRow = 32;
 
 __global__ void __launch_bounds__(256)
 k_pattern_rows16(const int32_t* __restrict__ nc_off, const int32_t* __restrict__ nc_items,
                  const int32_t* __restrict__ cells, int npc, int slot_bits, int32_t nb_node,
-                 const int32_t* __restrict__ row_index, int32_t* __restrict__ out, int32_t* __restrict__ overflow)
+                 const int32_t* __restrict__ row_index, int32_t* __restrict__ out, int32_t* __restrict__ stage,
+                 int32_t* __restrict__ overflow)
 {
   constexpr int L = kPatternLanes, S = kPatternSlots;
   const int lane = threadIdx.x & (L - 1);
@@ -175,29 +181,72 @@ k_pattern_rows16(const int32_t* __restrict__ nc_off, const int32_t* __restrict__
     if (lane >= d)
       incl += u;
   }
+  if (row_index == nullptr) {
+    int32_t longest = live && !ovf ? __shfl(incl, L - 1, L) : 0;
+#pragma unroll
+    for (int d = L; d < 64; d <<= 1)
+      longest = max(longest, __shfl_xor(longest, d, 64));
+    // a look first: almost every wave leaves the maximum as it is
+    if ((threadIdx.x & 63) == 0 &&
+        longest > __hip_atomic_load(overflow + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(overflow + 1, longest);
+  }
   if (!live || ovf)
     return;
-  if (row_index == nullptr) {
-    if (lane == L - 1)
-      out[i] = incl;
-  }
-  else {
-    int32_t at = row_index[i] + incl - mine;
+  if (row_index == nullptr && lane == L - 1)
+    out[i] = incl;
+  int32_t* row = row_index ? out + row_index[i] : stage + (int64_t)kStageRow * i;
+  const int32_t room = row_index ? 0x7fffffff : kStageRow;
+  int32_t at = incl - mine;
 #pragma unroll
-    for (int q = 0; q < S; ++q) {
-      const int32_t before = q == 0 ? prev : key[q - 1];
-      if (key[q] != before && key[q] != 0x7fffffff)
-        out[at++] = key[q];
+  for (int q = 0; q < S; ++q) {
+    const int32_t before = q == 0 ? prev : key[q - 1];
+    if (key[q] != before && key[q] != 0x7fffffff) {
+      if (at < room)
+        row[at] = key[q];
+      ++at;
     }
   }
 }
 
+// Staged rows of the count pass to their places, kStageRow lanes per row.
+__global__ void __launch_bounds__(256)
+k_pattern_copy(int32_t nb_node, const int32_t* __restrict__ row_index, const int32_t* __restrict__ stage,
+               int32_t* __restrict__ columns)
+{
+  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int32_t i = (int32_t)(g / kStageRow), q = (int32_t)(g % kStageRow);
+  if (i >= nb_node)
+    return;
+  const int32_t a = row_index[i];
+  if (q < row_index[i + 1] - a)
+    columns[a + q] = stage[g];
+}
+
+__global__ void k_max_row(const int32_t* __restrict__ len, int32_t n, int32_t* __restrict__ out)
+{
+  int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  int32_t v = (i < n) ? len[i] : 0;
+  v = max(v, __shfl_xor(v, 32, 64));
+  v = max(v, __shfl_xor(v, 16, 64));
+  v = max(v, __shfl_xor(v, 8, 64));
+  v = max(v, __shfl_xor(v, 4, 64));
+  v = max(v, __shfl_xor(v, 2, 64));
+  v = max(v, __shfl_xor(v, 1, 64));
+  if ((threadIdx.x & 63) == 0 && v > __hip_atomic_load(out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    atomicMax(out, v);
+}
+
 // Runs one pass (count if row_index == nullptr, fill otherwise) with the
 // smallest LDS capacity that holds every row.  Returns false on overflow at
-// the largest capacity.
-static bool pattern_pass(const afem_mesh& m, const int32_t* row_index, int32_t* out, int cap_hint)
+// the largest capacity.  The count pass gives the longest row, and stage holds
+// the rows afterwards when they all fit it (else it is empty).
+static bool pattern_pass(const afem_mesh& m, const int32_t* row_index, int32_t* out, int cap_hint,
+                         DBuf<int32_t>* stage = nullptr, int32_t* longest = nullptr)
 {
-  DBuf<int32_t> ovf(1);
+  DBuf<int32_t> ovf(2);
+  if (!row_index)
+    stage->alloc((size_t)kStageRow * m.nb_node);
   {
     // sixteen lanes per node when every node's candidates fit 128 slots
     ovf.zero();
@@ -206,14 +255,28 @@ static bool pattern_pass(const afem_mesh& m, const int32_t* row_index, int32_t* 
       const int64_t threads = (int64_t)m.nb_node * kPatternLanes;
       hipLaunchKernelGGL(k_pattern_rows16, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream(),
                          m.nc_offsets.p, m.nc_items.p, m.cells.p, m.npc, m.slot_bits, m.nb_node, row_index, out,
-                         ovf.p);
+                         row_index ? nullptr : stage->p, ovf.p);
     }
     check_launch("pattern_rows16");
-    int32_t flag = 0;
-    ovf.download(&flag, 1);
-    if (flag == 0)
+    int32_t flag[2] = { 0, 0 };
+    ovf.download(flag, 2);
+    if (!row_index && (flag[0] || flag[1] > kStageRow))
+      stage->release();
+    if (flag[0] == 0) {
+      if (longest)
+        *longest = flag[1];
       return true;
+    }
   }
+  auto measure = [&]() {
+    if (!longest)
+      return true;
+    ovf.zero();
+    hipLaunchKernelGGL(k_max_row, dim3(grid_for(m.nb_node, 256)), dim3(256), 0, stream(), out, m.nb_node, ovf.p);
+    check_launch("max_row");
+    ovf.download(longest, 1);
+    return true;
+  };
   auto run = [&](auto cap_tag, auto bs_tag) {
     constexpr int CAP = decltype(cap_tag)::value;
     constexpr int BS = decltype(bs_tag)::value;
@@ -230,10 +293,10 @@ static bool pattern_pass(const afem_mesh& m, const int32_t* row_index, int32_t* 
     return flag == 0;
   };
   if (cap_hint <= 32 && run(std::integral_constant<int, 32>{}, std::integral_constant<int, 256>{}))
-    return true;
+    return measure();
   if (cap_hint <= 128 && run(std::integral_constant<int, 128>{}, std::integral_constant<int, 64>{}))
-    return true;
-  return run(std::integral_constant<int, 512>{}, std::integral_constant<int, 16>{});
+    return measure();
+  return run(std::integral_constant<int, 512>{}, std::integral_constant<int, 16>{}) && measure();
 }
 
 static int row_cap_hint(const afem_mesh& m)
@@ -248,7 +311,7 @@ static void bsr_count_columns(afem_bsr* b)
 {
   const afem_mesh& m = *b->mesh;
   b->nnz_per_row.alloc((size_t)m.nb_node);
-  if (!pattern_pass(m, nullptr, b->nnz_per_row.p, row_cap_hint(m)))
+  if (!pattern_pass(m, nullptr, b->nnz_per_row.p, row_cap_hint(m), &b->row_stage, &b->max_row))
     fail(AFEM_ERR_CAPACITY, "a node has more than 511 neighbours");
   b->row_index.alloc((size_t)m.nb_node + 1);
   int64_t total = exclusive_scan_i32(b->nnz_per_row.p, b->row_index.p, m.nb_node);
@@ -257,32 +320,18 @@ static void bsr_count_columns(afem_bsr* b)
                "matrix too large for 32-bit value offsets");
 }
 
-__global__ void k_max_row(const int32_t* __restrict__ len, int32_t n, int32_t* __restrict__ out)
-{
-  int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  int32_t v = (i < n) ? len[i] : 0;
-  v = max(v, __shfl_xor(v, 32, 64));
-  v = max(v, __shfl_xor(v, 16, 64));
-  v = max(v, __shfl_xor(v, 8, 64));
-  v = max(v, __shfl_xor(v, 4, 64));
-  v = max(v, __shfl_xor(v, 2, 64));
-  v = max(v, __shfl_xor(v, 1, 64));
-  if ((threadIdx.x & 63) == 0)
-    atomicMax(out, v);
-}
-
 static void bsr_compute_sparsity(afem_bsr* b)
 {
   const afem_mesh& m = *b->mesh;
   b->columns.alloc((size_t)b->nb_col);
-  if (!pattern_pass(m, b->row_index.p, b->columns.p, row_cap_hint(m)))
+  if (b->row_stage.p) { // the rows of the count, once
+    hipLaunchKernelGGL(k_pattern_copy, dim3(grid_for((int64_t)kStageRow * m.nb_node, 256)), dim3(256), 0, stream(),
+                       m.nb_node, b->row_index.p, b->row_stage.p, b->columns.p);
+    check_launch("pattern_copy");
+    b->row_stage.release();
+  }
+  else if (!pattern_pass(m, b->row_index.p, b->columns.p, row_cap_hint(m)))
     fail(AFEM_ERR_CAPACITY, "a node has more than 511 neighbours");
-  DBuf<int32_t> mx(1);
-  mx.zero();
-  hipLaunchKernelGGL(k_max_row, dim3(grid_for(m.nb_node, 256)), dim3(256), 0, stream(), b->nnz_per_row.p,
-                     m.nb_node, mx.p);
-  check_launch("max_row");
-  mx.download(&b->max_row, 1);
   b->values.alloc((size_t)b->nb_col * b->nb_dof * b->nb_dof);
   b->values.zero();
   b->has_sparsity = true;
@@ -590,6 +639,10 @@ __device__ __forceinline__ int plan_pos(uint64_t w, int k) { return (int)((w >> 
 // when they fit (8192 entries), so the binary searches of the row positions
 // read LDS instead of re-reading the row from memory for every search.
 constexpr int kPairStage = 8192;
+// A row's cells are far apart in memory: their loads go out four at a time
+// (237 thousand nodes of shuffled tetrahedra: this plan 212 -> 156 us, the
+// brick plan 204 -> 132).
+constexpr int kPlanBatch = 4;
 
 template <class RowPtr>
 __device__ __forceinline__ bool pair_plan_row(RowPtr rc, int len, int32_t i, const int32_t* __restrict__ nc_off,
@@ -599,20 +652,31 @@ __device__ __forceinline__ bool pair_plan_row(RowPtr rc, int len, int32_t i, con
   const int d = find_col(rc, len, i);
   diag_pos[i] = d;
   bool bad = (d >= len || rc[d] != i);
-  for (int32_t e = nc_off[i]; e < nc_off[i + 1]; ++e) {
-    const int32_t it = nc_items[e];
-    const int32_t c = it >> 2;
-    const int s = it & 3;
-    const int4 cq = *reinterpret_cast<const int4*>(cells + 4 * (int64_t)c);
-    const int3 o = other_nodes(cq, s);
-    const int32_t nodes[3] = { o.x, o.y, o.z };
-    uint64_t w = (uint64_t)(uint32_t)c | ((uint64_t)s << 32);
-    for (int k = 0; k < npc - 1; ++k) {
-      const int pos = find_col(rc, len, nodes[k]);
-      bad = bad || pos >= len || rc[pos] != nodes[k] || pos > kPlanMaxRow;
-      w |= (uint64_t)(pos & 0xff) << (34 + 8 * k);
+  const int32_t e1 = nc_off[i + 1];
+  for (int32_t e0 = nc_off[i]; e0 < e1; e0 += kPlanBatch) {
+    int32_t it[kPlanBatch];
+    int4 cq[kPlanBatch];
+#pragma unroll
+    for (int z = 0; z < kPlanBatch; ++z)
+      it[z] = nc_items[min(e0 + z, e1 - 1)];
+#pragma unroll
+    for (int z = 0; z < kPlanBatch; ++z)
+      cq[z] = *reinterpret_cast<const int4*>(cells + 4 * (int64_t)(it[z] >> 2));
+#pragma unroll
+    for (int z = 0; z < kPlanBatch; ++z) {
+      if (e0 + z >= e1)
+        break;
+      const int s = it[z] & 3;
+      const int3 o = other_nodes(cq[z], s);
+      const int32_t nodes[3] = { o.x, o.y, o.z };
+      uint64_t w = (uint64_t)(uint32_t)(it[z] >> 2) | ((uint64_t)s << 32);
+      for (int k = 0; k < npc - 1; ++k) {
+        const int pos = find_col(rc, len, nodes[k]);
+        bad = bad || pos >= len || rc[pos] != nodes[k] || pos > kPlanMaxRow;
+        w |= (uint64_t)(pos & 0xff) << (34 + 8 * k);
+      }
+      plan[e0 + z] = w;
     }
-    plan[e] = w;
   }
   return bad;
 }
@@ -1070,24 +1134,35 @@ k_brick_plan(const int32_t* __restrict__ perm, const int32_t* __restrict__ nc_of
   const int32_t i = perm[slot];
   const int64_t base = slice[blk] + 2 * threadIdx.x;
   bool bad = false;
-  for (int32_t e = nc_off[i]; e < nc_off[i + 1]; ++e) {
-    const uint64_t w = plan[e];
-    const int32_t cell = plan_cell(w);
-    const int4 cq = *reinterpret_cast<const int4*>(cells + 4 * (int64_t)cell);
-    const int3 o = other_nodes(cq, plan_slot(w));
-    const int32_t nodes[3] = { o.x, o.y, o.z };
-    uint64_t lw = 0;
-    for (int k = 0; k < npc - 1; ++k) {
-      const int l = find_node(tab, tn, nodes[k]);
-      const int pos = plan_pos(w, k);
-      bad = bad || l >= tn || tab[l] != nodes[k] || pos >= kCompactMaxRow;
-      lw |= (uint64_t)(l & 2047) << (11 * k);
-      lw |= (uint64_t)(pos & 31) << (33 + 5 * k);
+  const int32_t first = nc_off[i], e1 = nc_off[i + 1];
+  for (int32_t e0 = first; e0 < e1; e0 += kPlanBatch) {
+    uint64_t w[kPlanBatch];
+    int4 cq[kPlanBatch];
+#pragma unroll
+    for (int z = 0; z < kPlanBatch; ++z)
+      w[z] = plan[min(e0 + z, e1 - 1)];
+#pragma unroll
+    for (int z = 0; z < kPlanBatch; ++z)
+      cq[z] = *reinterpret_cast<const int4*>(cells + 4 * (int64_t)plan_cell(w[z]));
+#pragma unroll
+    for (int z = 0; z < kPlanBatch; ++z) {
+      if (e0 + z >= e1)
+        break;
+      const int3 o = other_nodes(cq[z], plan_slot(w[z]));
+      const int32_t nodes[3] = { o.x, o.y, o.z };
+      uint64_t lw = 0;
+      for (int k = 0; k < npc - 1; ++k) {
+        const int l = find_node(tab, tn, nodes[k]);
+        const int pos = plan_pos(w[z], k);
+        bad = bad || l >= tn || tab[l] != nodes[k] || pos >= kCompactMaxRow;
+        lw |= (uint64_t)(l & 2047) << (11 * k);
+        lw |= (uint64_t)(pos & 31) << (33 + 5 * k);
+      }
+      const int32_t j = e0 + z - first;
+      const int64_t at = base + (int64_t)(j >> 1) * (2 * kLocalRows) + (j & 1);
+      out_plan[at] = lw;
+      out_cell[at] = plan_cell(w[z]);
     }
-    const int32_t j = e - nc_off[i];
-    const int64_t at = base + (int64_t)(j >> 1) * (2 * kLocalRows) + (j & 1);
-    out_plan[at] = lw;
-    out_cell[at] = cell;
   }
   if (bad)
     atomicOr(err, 1);

@@ -226,6 +226,7 @@ struct afem_bsr
   afem::DBuf<int32_t> row_index;     // nb_row + 1
   afem::DBuf<int32_t> columns;       // nb_col
   afem::DBuf<int32_t> nnz_per_row;   // nb_row
+  afem::DBuf<int32_t> row_stage;     // rows found by the count, until the first fill (empty: not kept)
   afem::DBuf<double> values;         // nb_col * nb_dof^2
   afem::DBuf<int32_t> csr_row;       // scalar CSR (toCsr), built on demand
   afem::DBuf<int32_t> csr_col;
