@@ -358,18 +358,24 @@ k_gemm_dx(int32_t n, const float* __restrict__ dY, const uint16_t* __restrict__ 
 
 // Partial dW = X^T (dY o [pre > 0]) and db = sum (dY o [pre > 0]) over a
 // contiguous range of nodes per wave; one partial (K*32 + 32 floats) per
-// block.  X as in k_gemm_fwd.
+// block.  X as in k_gemm_fwd.  Bound by the latency of its loads (320 bytes a
+// node at K = 64): 16 waves a block, two steps of 8 nodes in flight per wave,
+// and reads past the range clamped instead of branched around.  275 thousand
+// nodes, K = 64 (88 MB): 87 -> 30 us against four waves and one step.
+constexpr int kDwWaves = 16;
+
 template <int K>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(kDwWaves* kWave)
 k_gemm_dw(int32_t n, int32_t nodes_per_wave, const uint16_t* __restrict__ X1, const uint16_t* __restrict__ X2,
           const float* __restrict__ dY, const uint16_t* __restrict__ pre, float* __restrict__ partial)
 {
   constexpr int LD1 = (K == 64) ? 32 : K;
   constexpr int KT = (K + 31) / 32;
+  constexpr int U = 2; // steps in flight
   __shared__ float red[4][KT * 1024 + 32];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  const int64_t wid = (int64_t)blockIdx.x * 4 + wave;
+  const int64_t wid = (int64_t)blockIdx.x * kDwWaves + wave;
   const int64_t n0 = wid * nodes_per_wave;
   const int64_t n1 = min((int64_t)n, n0 + nodes_per_wave);
   f32x16 acc[KT];
@@ -380,80 +386,97 @@ k_gemm_dw(int32_t n, int32_t nodes_per_wave, const uint16_t* __restrict__ X1, co
       acc[kt][r] = 0.f;
   float dbias = 0.f;
   const int col = lane & 31;
-  for (int64_t base = n0; base < n1; base += 8) {
-    const int64_t nn = base + 4 * (lane >> 5); // 4 nodes per lane half
-    // B[n][j] = dYm[n][j]
-    bf16x4 b;
+  for (int64_t base = n0; base < n1; base += 8 * U) {
+    // B[n][j] = dYm[n][j], A[k][n] = X[n][k] with k = kt*32 + lane%32; 4 nodes per lane half
+    float gv[U][4];
+    uint16_t pv[U][4], xv[U][KT][4];
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int64_t node = nn + v;
-      float g = 0.f;
-      if (node < n1) {
-        g = dY[node * 32 + col];
-        if (pre && !(bf2f(pre[node * 32 + col]) > 0.f))
-          g = 0.f;
-      }
-      dbias += g;
-      b[v] = (short)f2bf(g);
-    }
-#pragma unroll
-    for (int kt = 0; kt < KT; ++kt) {
-      // A[k][n] = X[n][k], k = kt*32 + lane%32
-      const int k = kt * 32 + (lane & 31);
-      bf16x4 a;
+    for (int z = 0; z < U; ++z)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int64_t node = nn + v;
-        uint16_t xv = 0;
-        if (node < n1 && k < K)
-          xv = (K == 64 && k >= 32) ? X2[node * 32 + (k - 32)] : X1[node * LD1 + k];
-        a[v] = (short)xv;
+        const int64_t node = min(base + 8 * z + 4 * (lane >> 5) + v, n1 - 1);
+        gv[z][v] = dY[node * 32 + col];
+        pv[z][v] = pre ? pre[node * 32 + col] : (uint16_t)0;
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) {
+          const int k = kt * 32 + col;
+          xv[z][kt][v] = (K == 64 && kt == 1) ? X2[node * 32 + col] : k < K ? X1[node * LD1 + k] : (uint16_t)0;
+        }
       }
-      acc[kt] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, b, acc[kt], 0, 0, 0);
+#pragma unroll
+    for (int z = 0; z < U; ++z) {
+      bf16x4 b;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const bool live = base + 8 * z + 4 * (lane >> 5) + v < n1 && (!pre || bf2f(pv[z][v]) > 0.f);
+        const float g = live ? gv[z][v] : 0.f;
+        dbias += g;
+        b[v] = (short)f2bf(g);
+      }
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt) {
+        bf16x4 a;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) // a node past the range multiplies b = 0: not even by an infinity
+          a[v] = base + 8 * z + 4 * (lane >> 5) + v < n1 ? (short)xv[z][kt][v] : (short)0;
+        acc[kt] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, b, acc[kt], 0, 0, 0);
+      }
     }
   }
-  // wave partials to LDS: D[k][j] of tile kt
-#pragma unroll
-  for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-    for (int r = 0; r < 16; ++r)
-      red[wave][kt * 1024 + acc_row(r, lane) * 32 + col] = acc[kt][r];
   // the bias gradient: lanes l and l+32 hold halves of column l%32
   dbias += __shfl_xor(dbias, 32, kWave);
-  if (lane < 32)
-    red[wave][KT * 1024 + lane] = dbias;
-  __syncthreads();
+  // wave partials to LDS, four waves at a time: D[k][j] of tile kt
+  for (int turn = 0; turn < kDwWaves / 4; ++turn) {
+    if (wave / 4 == turn) {
+      float* slot = red[wave % 4];
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int q = kt * 1024 + acc_row(r, lane) * 32 + col;
+          slot[q] = turn ? slot[q] + acc[kt][r] : acc[kt][r];
+        }
+      if (lane < 32)
+        slot[KT * 1024 + lane] = turn ? slot[KT * 1024 + lane] + dbias : dbias;
+    }
+    __syncthreads();
+  }
   float* out = partial + (int64_t)blockIdx.x * (K * 32 + 32);
-  for (int q = threadIdx.x; q < K * 32; q += 256)
-    out[q] = red[0][q] + red[1][q] + red[2][q] + red[3][q];
-  if (threadIdx.x < 32) {
-    const int q = KT * 1024 + threadIdx.x;
-    out[K * 32 + threadIdx.x] = red[0][q] + red[1][q] + red[2][q] + red[3][q];
+  for (int q = threadIdx.x; q < K * 32 + 32; q += kDwWaves * kWave) {
+    const int s = q < K * 32 ? q : KT * 1024 + (q - K * 32);
+    out[q] = red[0][s] + red[1][s] + red[2][s] + red[3][s];
   }
 }
 
-// out[q] (+)= sum_b partial[b * stride + q] for q < len: 32 outputs per
-// workgroup, 8 groups of lanes take every 8th partial, and the 8 group sums
-// are added in a fixed order (deterministic).
-__global__ void __launch_bounds__(256)
-k_reduce_partials(int nparts, int stride, int len, const float* __restrict__ partial, float* __restrict__ out,
-                  int accumulate)
+// dW[q] = sum_b partial[b * stride + q] for q < len, the bias behind it to db
+// (null: none).  32 outputs per workgroup; 32 groups of lanes take every 32nd
+// partial and the group sums are added in a fixed order (deterministic).
+// Bound by latency: 8 groups and a launch for each of the two took 20 us a
+// layer, now 4.6.
+constexpr int kRedGroups = 32;
+
+__global__ void __launch_bounds__(kRedGroups * 32)
+k_reduce_partials(int nparts, int stride, int len, const float* __restrict__ partial, float* __restrict__ dW,
+                  float* __restrict__ db)
 {
-  __shared__ double red[8][32];
+  __shared__ double red[kRedGroups][32];
   const int ql = threadIdx.x & 31, g = threadIdx.x >> 5;
   const int q = blockIdx.x * 32 + ql;
   double s = 0.0;
-  if (q < len)
-    for (int b = g; b < nparts; b += 8)
+  if (q < stride)
+    for (int b = g; b < nparts; b += kRedGroups)
       s += partial[(int64_t)b * stride + q];
   red[g][ql] = s;
   __syncthreads();
-  if (g == 0 && q < len) {
+  if (g == 0 && q < stride) {
     double t = 0.0;
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
+    for (int k = 0; k < kRedGroups; ++k)
       t += red[k][ql];
-    out[q] = accumulate ? out[q] + (float)t : (float)t;
+    if (q < len)
+      dW[q] = (float)t;
+    else if (db)
+      db[q - len] = (float)t;
   }
 }
 
@@ -1015,19 +1038,17 @@ template <int K>
 void weight_grad(afem_spai* m, int32_t n, const uint16_t* X1, const uint16_t* X2, const float* dY,
                  const uint16_t* pre, int w_off, int b_off)
 {
-  const int waves = kDwBlocks * 4;
+  const int waves = kDwBlocks * kDwWaves;
   int32_t per = (int32_t)(((int64_t)n + waves - 1) / waves);
   per = (per + 7) / 8 * 8;
   if (per < 8)
     per = 8;
-  hipLaunchKernelGGL(k_gemm_dw<K>, dim3(kDwBlocks), dim3(256), 0, stream(), n, per, X1, X2, dY, pre, m->dwp.p);
+  hipLaunchKernelGGL(k_gemm_dw<K>, dim3(kDwBlocks), dim3(kDwWaves * kWave), 0, stream(), n, per, X1, X2, dY, pre,
+                     m->dwp.p);
   check_launch("spai_gemm_dw");
   const int stride = K * 32 + 32;
-  hipLaunchKernelGGL(k_reduce_partials, dim3((K * 32 + 31) / 32), dim3(256), 0, stream(), kDwBlocks, stride,
-                     K * 32, m->dwp.p, m->grad.p + w_off, 0);
-  if (b_off >= 0)
-    hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(256), 0, stream(), kDwBlocks, stride, 32,
-                       m->dwp.p + K * 32, m->grad.p + b_off, 0);
+  hipLaunchKernelGGL(k_reduce_partials, dim3((stride + 31) / 32), dim3(kRedGroups * 32), 0, stream(), kDwBlocks, stride,
+                     K * 32, m->dwp.p, m->grad.p + w_off, b_off >= 0 ? m->grad.p + b_off : nullptr);
   check_launch("spai_reduce_dw");
 }
 
