@@ -577,21 +577,6 @@ k_aggregate_grad(int32_t n, const int32_t* __restrict__ rp, const int32_t* __res
   *out = o;
 }
 
-__device__ __forceinline__ void load_vec32(const uint16_t* __restrict__ p, float* v)
-{
-  const uint4* q = reinterpret_cast<const uint4*>(p);
-#pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    const uint4 t = q[w];
-    const uint32_t ws[4] = { t.x, t.y, t.z, t.w };
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      v[8 * w + 2 * e] = bf2f((uint16_t)(ws[e] & 0xffffu));
-      v[8 * w + 2 * e + 1] = bf2f((uint16_t)(ws[e] >> 16));
-    }
-  }
-}
-
 // Mh (FP32, pattern of A) and the preconditioner M = D^-1/2 Mh D^-1/2
 // (FP32) that the solver applies; pre_d keeps the diagonal pre-activation.
 // Four lanes per row, eight features per lane (one 16-byte load of u_j);
@@ -733,7 +718,22 @@ k_probe_r(int32_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__
 //   diagonal: dpre_d = G_ii sigmoid(pre_d); dh3_i = dpre_d wd; dwd += dpre_d h3_i; dbd += dpre_d
 //   off-diagonal: dc += G_ij s_ij; du_i = sum_j (G_ij + G_ji) s_ij u_j
 // (Mh_ij and Mh_ji are the same function of the pair, hence G_ij + G_ji).
-// Per-block partials of (dwd[32], dbd, dc) in FP64.
+// Per-block partials of (dwd[32], dbd, dc) in FP64.  Four lanes per row as in
+// k_head, eight features a lane and the probes in each; the entries' gathers
+// go out kBackEntries at a time, every sum of a row keeps its order.  Bound by
+// the gathers; one lane per row read its neighbours' 128 bytes in 16-byte
+// pieces one entry after the other and summed 34 numbers per thread (275
+// thousand rows: 148 us, now 101).  A block takes several rounds of rows,
+// so the partials stay one per 256 rows.
+constexpr int kBackEntries = 2;
+
+__device__ __forceinline__ void load8(const float* __restrict__ p, float (&v)[8])
+{
+  const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
+  v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w;
+  v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+}
+
 __global__ void __launch_bounds__(256)
 k_head_backward(int32_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ ci,
                 const float* __restrict__ shat, const uint8_t* __restrict__ ident, const uint16_t* __restrict__ h3,
@@ -741,67 +741,101 @@ k_head_backward(int32_t n, const int32_t* __restrict__ rp, const int32_t* __rest
                 const float* __restrict__ y, const float* __restrict__ r, float coef, float* __restrict__ du,
                 float* __restrict__ dh3, double* __restrict__ part)
 {
-  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  double pv[kHeadParts] = {};
-  if (i < n) {
-    float dui[32] = {};
-    float dh[32] = {};
-    if (!ident[i]) {
+  static_assert(kP == 8 && kH == 8 * kHeadLanes, "lanes of a row");
+  __shared__ double s_part[4][kHeadParts];
+  const int q = threadIdx.x & (kHeadLanes - 1); // features 8q .. 8q + 7
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x / kHeadLanes;
+  double pv[8] = {}, pb = 0.0, pc = 0.0;
+  for (int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kHeadLanes; i < n; i += stride) {
+    float dui[8] = {}, dh[8] = {};
+    if (!ident[i]) { // the four lanes of a row agree
       float ri[kP], yi[kP];
-#pragma unroll
-      for (int p = 0; p < kP; ++p) {
-        ri[p] = r[(int64_t)i * kP + p];
-        yi[p] = y[(int64_t)i * kP + p];
-      }
-      float hv[32];
-      load_vec32(h3 + (int64_t)i * 32, hv);
+      load8(r + i * kP, ri);
+      load8(y + i * kP, yi);
       float dc = 0.f;
-      for (int32_t k = rp[i]; k < rp[i + 1]; ++k) {
-        const int32_t j = ci[k];
-        const float* yj = y + (int64_t)j * kP;
-        const float* rj = r + (int64_t)j * kP;
-        float gij = 0.f, gji = 0.f;
+      const int32_t e = rp[i + 1];
+      for (int32_t k = rp[i]; k < e; k += kBackEntries) {
+        int32_t j[kBackEntries];
+        float a[kBackEntries];
 #pragma unroll
-        for (int p = 0; p < kP; ++p) {
-          gij += ri[p] * yj[p];
-          gji += rj[p] * yi[p];
+        for (int v = 0; v < kBackEntries; ++v) {
+          j[v] = k + v < e ? ci[k + v] : -1;
+          a[v] = k + v < e ? shat[k + v] : 0.f;
         }
-        gij *= coef;
-        gji *= coef;
-        if (j == i) {
-          const float dpre = gij * sigmoid(pre_d[i]);
+        float rj[kBackEntries][kP], yj[kBackEntries][kP];
+        uint4 w[kBackEntries];
 #pragma unroll
-          for (int q = 0; q < 32; ++q) {
-            dh[q] = dpre * params[oWd + q];
-            pv[q] += (double)dpre * hv[q];
+        for (int v = 0; v < kBackEntries; ++v) {
+          const int64_t at = j[v] >= 0 ? j[v] : i;
+          load8(r + at * kP, rj[v]);
+          load8(y + at * kP, yj[v]);
+          w[v] = *reinterpret_cast<const uint4*>(u + at * 32 + 8 * q);
+        }
+#pragma unroll
+        for (int v = 0; v < kBackEntries; ++v) {
+          float gij = 0.f, gji = 0.f;
+#pragma unroll
+          for (int p = 0; p < kP; ++p) {
+            gij += ri[p] * yj[v][p];
+            gji += rj[v][p] * yi[p];
           }
-          pv[kH] += dpre;
-        }
-        else {
-          const float a = shat[k];
-          if (a != 0.f) {
-            dc += gij * a;
-            float uj[32];
-            load_vec32(u + (int64_t)j * 32, uj);
-            const float w = (gij + gji) * a;
+          gij *= coef;
+          gji *= coef;
+          if (j[v] == i) {
+            const float dpre = gij * sigmoid(pre_d[i]);
+            float hv[8];
+            unpack8(*reinterpret_cast<const uint4*>(h3 + i * 32 + 8 * q), hv);
 #pragma unroll
-            for (int q = 0; q < 32; ++q)
-              dui[q] += w * uj[q];
+            for (int f = 0; f < 8; ++f) {
+              dh[f] = dpre * params[oWd + 8 * q + f];
+              pv[f] += (double)dpre * hv[f];
+            }
+            pb += dpre;
+          }
+          else if (a[v] != 0.f) {
+            dc += gij * a[v];
+            const float g = (gij + gji) * a[v];
+            float uj[8];
+            unpack8(w[v], uj);
+#pragma unroll
+            for (int f = 0; f < 8; ++f)
+              dui[f] += g * uj[f];
           }
         }
       }
-      pv[kH + 1] = dc;
+      pc += dc;
     }
-    // the row's 32 + 32 values as 16-byte stores
-    float4* duo = reinterpret_cast<float4*>(du + (int64_t)i * 32);
-    float4* dho = reinterpret_cast<float4*>(dh3 + (int64_t)i * 32);
+    float4* duo = reinterpret_cast<float4*>(du + i * 32 + 8 * q);
+    float4* dho = reinterpret_cast<float4*>(dh3 + i * 32 + 8 * q);
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      duo[q] = make_float4(dui[4 * q], dui[4 * q + 1], dui[4 * q + 2], dui[4 * q + 3]);
-      dho[q] = make_float4(dh[4 * q], dh[4 * q + 1], dh[4 * q + 2], dh[4 * q + 3]);
+    for (int f = 0; f < 2; ++f) {
+      duo[f] = make_float4(dui[4 * f], dui[4 * f + 1], dui[4 * f + 2], dui[4 * f + 3]);
+      dho[f] = make_float4(dh[4 * f], dh[4 * f + 1], dh[4 * f + 2], dh[4 * f + 3]);
     }
   }
-  block_sum_write<kHeadParts>(pv, part + (int64_t)blockIdx.x * kHeadParts);
+  // over the wave's lanes of the same q, then over the waves
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  auto rows = [](double v) {
+#pragma unroll
+    for (int o = kHeadLanes; o < 64; o <<= 1)
+      v += __shfl_xor(v, o, 64);
+    return v;
+  };
+#pragma unroll
+  for (int f = 0; f < 8; ++f) {
+    const double v = rows(pv[f]);
+    if (lane < kHeadLanes)
+      s_part[wave][8 * q + f] = v;
+  }
+  pb = rows(pb);
+  pc = rows(pc);
+  if (lane == 0) { // all four lanes of a row hold these
+    s_part[wave][kH] = pb;
+    s_part[wave][kH + 1] = pc;
+  }
+  __syncthreads();
+  for (int k = threadIdx.x; k < kHeadParts; k += 256)
+    part[(int64_t)blockIdx.x * kHeadParts + k] = s_part[0][k] + s_part[1][k] + s_part[2][k] + s_part[3][k];
 }
 
 // one workgroup per head parameter q
