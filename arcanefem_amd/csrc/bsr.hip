@@ -325,6 +325,7 @@ static void bsr_compute_sparsity(afem_bsr* b)
   const afem_mesh& m = *b->mesh;
   b->columns.alloc((size_t)b->nb_col);
   if (b->row_stage.p) { // the rows of the count, once
+    ProfScope prof("pattern_copy");
     hipLaunchKernelGGL(k_pattern_copy, dim3(grid_for((int64_t)kStageRow * m.nb_node, 256)), dim3(256), 0, stream(),
                        m.nb_node, b->row_index.p, b->row_stage.p, b->columns.p);
     check_launch("pattern_copy");
