@@ -85,7 +85,7 @@ k_pattern_rows(const int32_t* __restrict__ nc_off, const int32_t* __restrict__ n
 // a node's candidates do not fit its 128 slots (the caller then runs the
 // per-thread kernel).  Bound by the network's instructions (1400 per wave):
 // 133 us at 237 thousand nodes of tetrahedra, so the fill pass runs only for
-// rows that the stage does not hold; copying the staged rows takes 14.
+// rows that the stage does not hold; copying the staged rows takes 23.
 constexpr int kPatternLanes = 16, kPatternSlots = 8;
 constexpr int kStageRow = 32;
 
