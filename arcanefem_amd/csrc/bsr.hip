@@ -83,8 +83,8 @@ k_pattern_rows(const int32_t* __restrict__ nc_off, const int32_t* __restrict__ n
 // kStageRow columns of the row at stage[kStageRow * i], and the longest row in
 // overflow[1]; fill pass: the sorted row at row_index[i].  overflow[0] = 1 when
 // a node's candidates do not fit its 128 slots (the caller then runs the
-// per-thread kernel).  Bound by the network's instructions (1400 per wave):
-// 133 us at 237 thousand nodes of tetrahedra, so the fill pass runs only for
+// per-thread kernel).  Bound by the network's instructions (28 stages of 8
+// keys a lane): 133 us at 237 thousand nodes of tetrahedra, so the fill pass runs only for
 // rows that the stage does not hold; copying the staged rows takes 23.
 constexpr int kPatternLanes = 16, kPatternSlots = 8;
 constexpr int kStageRow = 32;
