@@ -9,6 +9,7 @@
 #include "node_direct.h"
 
 #include <algorithm>
+#include <atomic>
 
 #include <hipcub/hipcub.hpp>
 
@@ -336,7 +337,8 @@ static void bsr_compute_sparsity(afem_bsr* b)
   b->values.alloc((size_t)b->nb_col * b->nb_dof * b->nb_dof);
   b->values.zero();
   b->has_sparsity = true;
-  ++b->pattern_gen;
+  static std::atomic<uint64_t> patterns{ 0 };
+  b->pattern_gen = ++patterns;
 }
 
 static void build_plan(afem_bsr* b);

@@ -219,7 +219,8 @@ struct afem_bsr
   bool use_csr = false;
   bool atomic_free = false;
   bool has_sparsity = false;
-  uint64_t pattern_gen = 0;          // counts computeSparsity calls (linear systems key derived data on it)
+  uint64_t pattern_gen = 0;          // number of the pattern, unique in the process (linear systems key derived
+                                     // data on it: a released matrix's addresses serve the next one)
   int32_t nb_row = 0;
   int64_t nb_col = 0;                // stored blocks
   int32_t max_row = 0;
