@@ -1103,7 +1103,7 @@ struct afem_batch
   DBuf<int32_t> d_list;
   int nlaunch = 0;
   // segment-aligned SELL-64 copy (built with the first solve of a pattern)
-  const int32_t* sell_rp = nullptr;
+  uint64_t sell_pattern = 0; // pattern_count + 1 of the system when it (and the captured graph) was built
   bool sell_ok = false;
   DBuf<int32_t> d_sslice, d_soff, d_slice_row;
   DBuf<int16_t> sdcol;
@@ -1225,7 +1225,7 @@ void shrink_grid(afem_batch* b)
 void build_sell(afem_batch* b)
 {
   afem_system* s = b->sys;
-  b->sell_rp = s->row_index;
+  b->sell_pattern = s->pattern_count + 1;
   b->sell_ok = false;
   std::vector<int32_t> slice_row, sslice(b->nb_seg + 1, 0);
   for (int k = 0; k < b->nb_seg; ++k) {
@@ -1361,7 +1361,7 @@ void prepare(afem_batch* b)
   AFEM_REQUIRE(h == 0, AFEM_ERR_ARGUMENT,
                "the batched solver needs a diagonal entry in every non-empty row (its FP32 product is in "
                "difference form)");
-  if (b->sell_rp != s->row_index) {
+  if (b->sell_pattern != s->pattern_count + 1) { // another view: its addresses say nothing about its columns
     drop_graph(b);
     build_sell(b);
   }
