@@ -125,6 +125,7 @@ def _declare(L):
         "afem_system_solve_noalloc": (ci, [vp, ctypes.POINTER(SolverOptions), ctypes.POINTER(SolveResult)]),
         "afem_system_spmv": (ci, [vp, vp, vp]),
         "afem_system_spmv_fp32": (ci, [vp, vp, vp]),
+        "afem_system_set_spin_limit": (ci, [vp, ctypes.c_longlong]),
         "afem_system_spmv_format": (ci, [vp, ctypes.POINTER(ci), ctypes.POINTER(ci)]),
         "afem_system_spmv_tuning": (ci, [vp] + [ctypes.POINTER(ci)] * 4),
         "afem_system_set_spai": (ci, [vp, vp]),
@@ -479,6 +480,11 @@ class DoFLinearSystem:
         if rc != OK and (raise_on_failure or rc != ERR_NOT_CONVERGED):
             check(rc)
         return r
+
+    def set_spin_limit(self, polls):
+        """Polls after which a barrier wait of a one-launch solve gives up and
+        the solve goes on with the kernels that wait for nothing (0 = default)."""
+        check(lib().afem_system_set_spin_limit(self.h, polls))
 
     def solve_noalloc(self, raise_on_failure=True, **kw):
         """The allocation-free FP64 solve (afem_system_solve_noalloc): at most

@@ -1747,7 +1747,8 @@ bool resident_usable(afem_batch* b, const afem_batch_options& o)
   return b->pack_usable && b->pack.all_diag;
 }
 
-// Solves the segments with want set; false: a barrier wait gave up.
+// Solves the segments with want set; false: a barrier wait gave up (the states
+// hold what led to x, and done for the segments that had ended).
 bool run_resident(afem_batch* b, const afem_batch_options& o, double delta, const std::vector<char>& want,
                   const std::vector<int>& iters)
 {
@@ -1763,8 +1764,8 @@ bool run_resident(afem_batch* b, const afem_batch_options& o, double delta, cons
   }
   resident::Options ro;
   ro.mixed = true;
-  if (!resident::solve(b->pack, b->rwork, ro, s->x.p, s->rhs.p))
-    return false;
+  ro.spin_limit = o.spin_limit;
+  const bool ran = resident::solve(b->pack, b->rwork, ro, s->x.p, s->rhs.p);
   for (int k = 0; k < b->nb_seg; ++k) {
     const resident::Status& st = b->rwork.host[k];
     SegState& z = b->host_st[k];
@@ -1773,8 +1774,9 @@ bool run_resident(afem_batch* b, const afem_batch_options& o, double delta, cons
     z.bb = st.bb;
     z.rr_true = st.rr_true;
     z.converged = st.converged;
+    z.done = st.done;
   }
-  return true;
+  return ran;
 }
 
 // Solves the active segments in one persistent launch.  persistent = 1 uses
@@ -1927,7 +1929,19 @@ AFEM_API int afem_batch_solve(afem_batch_t b, const afem_batch_options* opt, afe
   std::vector<int> iters(b->nb_seg, 0), nru(b->nb_seg, 0), conv(b->nb_seg, 0);
   std::vector<double> relres(b->nb_seg, 0.0);
   std::vector<char> want(b->nb_seg, 1);
-  for (int round = 0; round < 5; ++round) {
+  // a segment's run from its current iterate has ended
+  auto account = [&](int k, const SegState& run, double rr_true) {
+    iters[k] += run.iter;
+    nru[k] += run.nb_ru;
+    const double bn = std::sqrt(run.bb);
+    const double tr = std::sqrt(rr_true);
+    relres[k] = bn > 0.0 ? tr / bn : tr;
+    conv[k] = (relres[k] <= opt->rtol || tr <= opt->atol) ? 1 : 0;
+    // the recursive residual met the tolerance but the true one does not:
+    // run that segment again from its current iterate
+    want[k] = (!conv[k] && run.converged && run.iter > 0 && std::isfinite(relres[k])) ? 1 : 0;
+  };
+  auto start = [&]() {
     bool any = false;
     for (int k = 0; k < b->nb_seg; ++k) {
       SegState z{};
@@ -1939,11 +1953,26 @@ AFEM_API int afem_batch_solve(afem_batch_t b, const afem_batch_options* opt, afe
       any = any || z.active;
       b->host_st[k] = z;
     }
-    if (!any)
-      break;
+    return any;
+  };
+  for (int round = 0; round < 5 && start(); ++round) {
     if (on_chip && !run_resident(b, *opt, delta, want, iters)) {
-      on_chip = false; // another process holds part of the device: the chunked kernels wait for nothing
+      // another process holds part of the device: the chunked kernels wait for
+      // nothing; they solve with this pattern from now on
+      on_chip = b->pack_usable = false;
+      b->pack = resident::Pack();
+      for (int k = 0; k < b->nb_seg; ++k) {
+        const SegState z = b->host_st[k];
+        if (z.active && z.done)
+          account(k, z, z.rr_true);
+        else if (z.active) {
+          iters[k] += z.iter;
+          nru[k] += z.nb_ru;
+        }
+      }
       prepare(b);
+      if (!start())
+        break;
     }
     if (!on_chip) {
       write_states(b);
@@ -1964,15 +1993,7 @@ AFEM_API int afem_batch_solve(afem_batch_t b, const afem_batch_options* opt, afe
     for (int k = 0; k < b->nb_seg; ++k) {
       if (!after[k].active)
         continue;
-      iters[k] += after[k].iter;
-      nru[k] += after[k].nb_ru;
-      const double bn = std::sqrt(after[k].bb);
-      const double tr = std::sqrt(b->host_st[k].rr_true);
-      relres[k] = bn > 0.0 ? tr / bn : tr;
-      conv[k] = (relres[k] <= opt->rtol || tr <= opt->atol) ? 1 : 0;
-      // the recursive residual met the tolerance but the true one does not:
-      // run that segment again from its current iterate
-      want[k] = (!conv[k] && after[k].converged && after[k].iter > 0 && std::isfinite(relres[k])) ? 1 : 0;
+      account(k, after[k], b->host_st[k].rr_true);
       again = again || want[k];
     }
     if (!again)

@@ -307,6 +307,7 @@ struct afem_system
   bool matrix_changed = true;        // invalidates derived data (FP32 copy, diagonal)
   bool pattern_changed = true;       // invalidates pattern-derived data (SELL layouts)
   uint64_t pattern_count = 0;        // counts pattern changes (batched solvers key derived data on it)
+  long long spin_limit = 0;          // polls of a resident solve's barrier wait (0: default)
   bool has_row_column = false;       // row-column eliminations present
   bool dof0_row_column = false;      // DoF 0 is row-column eliminated (column 0 kept: non-symmetric)
   afem::DBuf<double> saved_values;   // values before the row-column elimination

@@ -441,7 +441,10 @@ k_pair_prec(int32_t nslice, const int32_t* __restrict__ slice_row, const int32_t
 // (the barriers).
 static int waves_of(const Pack& p) { return p.block == 3 ? kBlockWaves : kWaves; }
 static int max_rows(const Pack& p) { return p.block == 3 ? kBlockRowSteps[2] : kRowSteps[3]; }
-constexpr int kLaunchIterations = 8192; // iterations of one launch: a second or less at any size
+// Iterations of one launch: 0.05 s for a system of 66 thousand rows, 0.3 s for
+// 2.15 million of tetrahedra, 4 s for the largest layout that is accepted (2.5
+// GiB of FP64 pairs and offsets an iteration).
+constexpr int kLaunchIterations = 8192;
 
 // Workgroups a segment needs at least (max_rows slices per wave).
 static int32_t least_workgroups(const Pack& p, int k)

@@ -2080,7 +2080,8 @@ struct SolveTotals
   double relres = 0.0;
 };
 
-// False: a barrier wait gave up (x is some iterate).
+// False: a barrier wait gave up; x is some iterate, and the totals count what
+// led to it (the vectors of the launch that gave up are lost).
 static bool solve_resident(afem_system* s, afem_solver_ws* w, const afem_solver_options& o, SolveTotals& t)
 {
   const bool flex = o.method == AFEM_SOLVER_FPCG_SPAI;
@@ -2091,6 +2092,7 @@ static bool solve_resident(afem_system* s, afem_solver_ws* w, const afem_solver_
   ro.mixed = mixed;
   ro.precond = o.method != AFEM_SOLVER_CG_FP64 && o.preconditioner != AFEM_PRECOND_NONE;
   ro.norm = o.norm;
+  ro.spin_limit = s->spin_limit;
   if (flex) { // BF16 values come with 16-bit offsets, FP32 otherwise
     ro.prec = o.precond_bf16 && w->pack.idx16 ? 16 : 32;
     resident::pack_prec(w->pack, s->row_index, s->columns, w->spai32.p, ro.prec);
@@ -2103,10 +2105,11 @@ static bool solve_resident(afem_system* s, afem_solver_ws* w, const afem_solver_
     st.delta2 = delta * delta;
     st.max_iter = o.max_iter - t.iterations;
     st.active = 1;
-    if (!resident::solve(w->pack, w->rwork, ro, s->x.p, s->rhs.p))
-      return false;
+    const bool ran = resident::solve(w->pack, w->rwork, ro, s->x.p, s->rhs.p);
     t.iterations += st.iter;
     t.reliable_updates += st.nb_ru;
+    if (!ran)
+      return false;
     t.breakdown = st.breakdown != 0;
     const double bnorm = std::sqrt(st.bb), rnorm = std::sqrt(o.norm == 2 ? st.rr_out : st.rr_true);
     t.relres = bnorm > 0.0 ? rnorm / bnorm : rnorm;
@@ -2123,7 +2126,8 @@ static bool solve_resident(afem_system* s, afem_solver_ws* w, const afem_solver_
   }
 }
 
-// Every vector in memory, three to five kernels an iteration.
+// Every vector in memory, three to five kernels an iteration; adds to the
+// iterations that the totals already count.
 static void solve_streaming(afem_system* s, afem_solver_ws* w, const afem_solver_options& o, SolveTotals& out)
 {
   const bool flex = o.method == AFEM_SOLVER_FPCG_SPAI;
@@ -2148,7 +2152,7 @@ static void solve_streaming(afem_system* s, afem_solver_ws* w, const afem_solver
   init.atol2 = o.atol * o.atol;
   init.delta2 = delta * delta;
   init.natural = o.norm;
-  int total_iter = 0, restarts = 0, nb_ru = 0;
+  int total_iter = out.iterations, restarts = 0, nb_ru = out.reliable_updates;
   bool converged = false, breakdown = false;
   double relres = 0.0;
   double bnorm = 0.0;
@@ -2202,7 +2206,7 @@ static void solve_streaming(afem_system* s, afem_solver_ws* w, const afem_solver
   out = SolveTotals{ total_iter, nb_ru, converged, breakdown, relres };
 }
 
-static int solve(afem_system* s, const afem_solver_options& o, afem_solve_result* res, bool resident_ok = true)
+static int solve(afem_system* s, const afem_solver_options& o, afem_solve_result* res)
 {
   AFEM_REQUIRE(o.method == AFEM_SOLVER_PCG_FP64 || o.method == AFEM_SOLVER_PCG_MIXED ||
                  o.method == AFEM_SOLVER_CG_FP64 || o.method == AFEM_SOLVER_FPCG_SPAI,
@@ -2236,13 +2240,13 @@ static int solve(afem_system* s, const afem_solver_options& o, afem_solve_result
     check_launch("initial_guess");
   }
   SolveTotals t;
-  const bool on_chip = resident_ok && resident_usable(s, w, o);
+  bool on_chip = resident_usable(s, w, o);
   if (on_chip && !solve_resident(s, w, o, t)) {
     // the device could not hold every workgroup at once (another process on
-    // it, say): finish with the kernels that wait for nothing
-    afem_solver_options go = o;
-    go.use_initial_guess = 1;
-    return solve(s, go, res, false);
+    // it, say): the kernels that wait for nothing finish, and solve with this
+    // pattern from now on
+    on_chip = w->pack_usable = false;
+    w->pack = resident::Pack();
   }
   if (!on_chip)
     solve_streaming(s, w, o, t);
@@ -2256,7 +2260,7 @@ static int solve(afem_system* s, const afem_solver_options& o, afem_solve_result
     jo.use_initial_guess = 1;
     jo.max_iter = o.max_iter - t.iterations;
     afem_solve_result jr{};
-    const int rc = solve(s, jo, &jr, resident_ok);
+    const int rc = solve(s, jo, &jr);
     if (rc != AFEM_OK && rc != AFEM_ERR_NOT_CONVERGED)
       return rc;
     t.iterations += jr.iterations;
@@ -2602,6 +2606,14 @@ AFEM_API int afem_system_set_spai(afem_system_t sys, const float* values)
   w->has_spai = true;
   w->spai_sell_valid = false;
   w->pack.valid_prec = 0;
+  AFEM_GUARD_END
+}
+
+AFEM_API int afem_system_set_spin_limit(afem_system_t sys, long long polls)
+{
+  AFEM_GUARD_BEGIN
+  AFEM_REQUIRE(sys && polls >= 0, AFEM_ERR_ARGUMENT, "null handle or negative limit");
+  sys->spin_limit = polls;
   AFEM_GUARD_END
 }
 

@@ -400,9 +400,17 @@ typedef struct afem_solve_result {
 
 AFEM_API void afem_solver_default_options(afem_solver_options* opt);
 /* IDoFLinearSystemImpl::solve.  Synchronous.  Returns AFEM_ERR_NOT_CONVERGED
- * (with the result filled) when max_iter is reached. */
+ * (with the result filled) when max_iter is reached.  With spmv_lanes 0 a
+ * system that fits the chip is solved in one launch whose workgroups wait for
+ * each other; where the device does not run them all at once (it is shared)
+ * the waits end at a limit, and this solve and later ones with the pattern use
+ * the kernels that wait for nothing.  The iterations of the launch that ended
+ * so are lost and not counted. */
 AFEM_API int afem_system_solve(afem_system_t sys, const afem_solver_options* opt,
                                afem_solve_result* result);
+/* Polls after which those waits end (0 = 2^22, seconds).  No counterpart in
+ * the reference. */
+AFEM_API int afem_system_set_spin_limit(afem_system_t sys, long long polls);
 /* No counterpart in the reference.  For callers that cannot allocate device or
  * pinned memory (code under graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): afem_system_solve for the FP64 methods (AFEM_SOLVER_PCG_FP64,
@@ -526,8 +534,10 @@ typedef struct afem_batch_options {
                              vectors exchanged through the device's coherence point */
   int workgroups;         /* persistent: workgroups of the launch (0 = as many as the device holds
                              at once; capped there; at least one per system) */
-  long long spin_limit;   /* persistent: polls before a barrier wait gives up (0 = 2^21); the solve
-                             then fails with AFEM_ERR_DEVICE instead of waiting on */
+  long long spin_limit;   /* polls before a barrier wait gives up.  persistent (0 = 2^21): the solve
+                             then fails with AFEM_ERR_DEVICE instead of waiting on.  Default solve
+                             (0 = 2^22): it goes on with the chunked kernels, as do later ones with
+                             the pattern */
   double timeout_ms;      /* persistent: wall time after which the host raises the cancel flag that
                              every barrier wait polls (0 = 60000) */
 } afem_batch_options;
