@@ -1,8 +1,9 @@
 """GPU tests of the batched solver: independent 2D heat/Poisson systems with
 8x8 checkerboard conductivities on meshes of different sizes, assembled in
 one launch on the disjoint union of the meshes and solved together with
-per-system scalars (segmented mixed-precision PCG: hipGraph chunks of
-ordinary kernels by default, one persistent launch with persistent=1).
+per-system scalars (segmented mixed-precision PCG: teams of resident
+workgroups by default, hipGraph chunks of ordinary kernels once the tiles are
+set, one persistent launch with persistent=1).
 
 Checked against: a direct solve of each diagonal block (scipy), the
 single-system mixed PCG of the same block (iteration counts), the
@@ -76,18 +77,41 @@ def test_batch_matches_direct_solves(afem_gpu):
     assert its[-1] > its[0]
 
 
-def test_batch_graph_equals_plain_launches(afem_gpu):
+def kernel_launches(A, names, run):
+    """(launches of the named kernels, result) of a call, by the library's own timings."""
+    A.profile_enable(True)
+    A.profile_reset()
+    try:
+        r = run()
+        n = sum(A.profile_query(k)[0] for k in names)
+    finally:
+        A.profile_reset()
+        A.profile_enable(False)
+    return n, r
+
+
+@pytest.mark.parametrize("path", ["resident", "chunked", "persistent"])
+def test_batch_graph_equals_plain_launches(afem_gpu, path):
     A = afem_gpu
-    print("[case] batch graph vs plain", flush=True)
+    print(f"[case] batch graph vs plain {path}", flush=True)
     case = build_batch(A, [7, 16, 11], seed=4)
     bs = A.BatchSolver(case["sys"], case["offs"])
-    for persistent in (0, 1):
-        r1, _ = bs.solve(rtol=1e-8, use_graph=1, chunk=8, persistent=persistent)
+    if path == "chunked":
+        bs.set_tiles(1, 1)
+    persistent = 1 if path == "persistent" else 0
+    sols = {}
+    for chunk in (8, 32):
+        n, (r1, _) = kernel_launches(A, ["resident_cg_mixed"], lambda: bs.solve(
+            rtol=1e-8, use_graph=1, chunk=chunk, persistent=persistent))
+        assert n == (1 if path == "resident" else 0)
         x1 = case["sys"].solution().numpy()
-        r2, _ = bs.solve(rtol=1e-8, use_graph=0, chunk=8, persistent=persistent)
+        r2, _ = bs.solve(rtol=1e-8, use_graph=0, chunk=chunk, persistent=persistent)
         x2 = case["sys"].solution().numpy()
         assert [r.iterations for r in r1] == [r.iterations for r in r2]
         assert np.array_equal(x1, x2)
+        sols[chunk] = x1
+    # the chunk sets when the host looks, not what the iterations compute
+    assert np.array_equal(sols[8], sols[32])
 
 
 def test_batch_iterations_match_single_solver(afem_gpu):
@@ -245,9 +269,12 @@ def test_persistent_matches_chunked_and_direct(afem_gpu):
     print("[case] persistent vs chunked", flush=True)
     case = build_batch(A, [40, 6, 7, 8, 9, 6, 7, 8, 9, 25], seed=6)
     bs = A.BatchSolver(case["sys"], case["offs"])
+    bs.set_tiles(1, 1)  # the default solves run the chunked kernels, with the persistent ones' SELL product
     out = {}
     for persistent in (1, 2, 0):
-        res, _ = bs.solve(rtol=1e-10, max_iter=5000, persistent=persistent)
+        n, (res, _) = kernel_launches(A, ["resident_cg_mixed"], lambda: bs.solve(
+            rtol=1e-10, max_iter=5000, persistent=persistent))
+        assert n == 0
         if persistent:
             mode = bs.persistent_mode()
             print(f"[case] persistent={persistent} exchange mode {mode}", flush=True)
