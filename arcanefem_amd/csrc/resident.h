@@ -65,7 +65,7 @@ struct Status // of one segment
 
 struct Options
 {
-  bool mixed = false;   // FP32 vectors and products, FP64 x and reliable updates
+  bool mixed = false;   // FP32 matrix and published vector, reliable updates in FP64
   bool precond = true;  // Jacobi
   int prec = 0;         // flexible CG with the pack's sparse preconditioner (its bits); mixed
   int norm = 0;         // stopping norm of afem_solver_options

@@ -296,20 +296,28 @@ __device__ __forceinline__ IndexPair<I16> load_offsets(Rsrc r, int lane, int q)
 //   -- sum --   beta = r.u / rho; convergence
 //
 // With s kept by its recurrence the product reads u, which was published
-// before the sum that gives beta, so an iteration has two barriers.  FP32
-// vectors (T = float) have x in FP64 and take reliable updates: x is
-// published, r = b - A64 x formed in FP64, u = D r published again.  Their p
-// and s are FP64 and the terms of w are summed in FP64: w is a product with
-// the rough u, not with the smooth p, and FP32 sums would cost 5 % more
-// iterations than forming A p anew (FP64 sums take 6 % fewer).
+// before the sum that gives beta, so an iteration has two barriers.  The mixed
+// solver (T = float) has u and the matrix in FP32 and takes reliable updates:
+// x is published, r = b - A64 x formed, u = D r published again.  Its r, p and
+// s are FP64 and the terms of w exact (FP64 products of the FP32 numbers,
+// summed in FP64): w is a product with the rough u, not with the smooth p, and
+// what it loses stays in s.  With r and the products in FP32 the residual of a
+// late reliable update differed from the recursive one by up to 0.4 %, which
+// cost iterations and left more error at the same residual: checkerboard of
+// 509 x 509 quads 4954 iterations, now 3320; log-normal cube of 128^3 hexes
+// 1724 (x error 1e-9), now 1449 (6e-12; FP64 PCG takes 1448).  The price at 9
+// slices per wave is 40.8 -> 41.2 us an iteration at 2.15 million rows; at 5
+// there is none (16.8, 16.5 at 0.53 million).
 //
 // With a sparse preconditioner (PREC 32 or 16: its values FP32 or BF16) B
 // publishes r, and a third phase forms u = M r, published, and the partials
 // u.r and u.s, whose sum gives the flexible beta = -alpha u.s / rho
 // (Polak-Ribiere; u.r / rho after a reliable update).
 //
-// r, s, the diagonal, FP64's p and FP32's D^-1 (or u = M r) are in registers,
-// x, FP32's p and FP64's D^-1 in LDS.  The matrices are the only streams of an
+// r, s, FP64's p and FP32's D^-1 (or u = M r) are in registers, and the
+// diagonal but for the mixed solvers at 9 slices, which read it with the row's
+// matrix (loaded after the row's sums instead: 42.1 us).  x, FP32's p and
+// FP64's D^-1 are in LDS.  The matrices are the only other streams of an
 // iteration: read a chunk of CP pairs ahead of their use, the first chunk of
 // the next product ahead of the barriers.
 enum StreamKind
@@ -328,6 +336,7 @@ __global__ void __launch_bounds__(kBS, 4) k_cg(Args a)
   constexpr bool FLEX = PREC != 0;
   static_assert(!FLEX || MIXED, "the sparse preconditioner is FP32");
   constexpr bool DLDS = !MIXED; // D^-1 in LDS and p in registers, else the other way round
+  constexpr bool GREG = !MIXED || R <= 5; // the diagonal in registers
   constexpr int CP = MIXED ? 4 : (R > 5 ? 2 : 4);
   extern __shared__ __align__(16) unsigned char smem[];
 
@@ -369,8 +378,8 @@ __global__ void __launch_bounds__(kBS, 4) k_cg(Args a)
 
   double* l_x = reinterpret_cast<double*>(smem) + threadIdx.x;
   double* l_2 = l_x + R * kBS;
-  T r[R], dg[R], di[DLDS ? 1 : R]; // FLEX: di holds u
-  double s[R], pr[DLDS ? R : 1];
+  T dg[GREG ? R : 1], di[DLDS ? 1 : R]; // FLEX: di holds u
+  double r[R], s[R], pr[DLDS ? R : 1];
   auto get_p = [&](int j) -> double {
     if constexpr (DLDS)
       return pr[j];
@@ -389,14 +398,16 @@ __global__ void __launch_bounds__(kBS, 4) k_cg(Args a)
     else
       return di[j];
   };
-  auto get_u = [&](int j) -> T { return FLEX ? di[DLDS ? 0 : j] : get_d(j) * r[j]; };
+  auto get_u = [&](int j) -> T { return FLEX ? di[DLDS ? 0 : j] : get_d(j) * (T)r[j]; };
+  const Rsrc grs = segment_buffer(reinterpret_cast<const T*>(a.diag), team.row0, rows);
+  auto get_g = [&](int j) -> T { return GREG ? dg[GREG ? j : 0] : bload<T, 0>(grs, row_of(j)); };
   {
     const Rsrc drs = segment_buffer(reinterpret_cast<const T*>(a.dinv), team.row0, rows);
-    const Rsrc grs = segment_buffer(reinterpret_cast<const T*>(a.diag), team.row0, rows);
 #pragma unroll
     for (int j = 0; j < R; ++j) {
-      r[j] = dg[j] = (T)0;
-      s[j] = 0.0;
+      r[j] = s[j] = 0.0;
+      if constexpr (GREG)
+        dg[j] = (T)0;
       set_p(j, 0.0);
       if constexpr (!DLDS)
         di[j] = (T)0;
@@ -409,7 +420,8 @@ __global__ void __launch_bounds__(kBS, 4) k_cg(Args a)
           else
             di[j] = d;
         }
-        dg[j] = bload<T, 0>(grs, row_of(j));
+        if constexpr (GREG)
+          dg[j] = bload<T, 0>(grs, row_of(j));
       }
     }
   }
@@ -417,9 +429,9 @@ __global__ void __launch_bounds__(kBS, 4) k_cg(Args a)
   // b - A64 x of row j, x as published; 0 in the lanes past the segment
   auto residual = [&](int j) -> double {
     const Rsrc mrs64 = whole_buffer(a.v64);
-    const Rsrc grs = segment_buffer(a.diag64, team.row0, rows);
+    const Rsrc grs64 = segment_buffer(a.diag64, team.row0, rows);
     const int32_t row = row_of(j);
-    double t0 = bload<double, 0>(grs, row) * l_x[j * kBS], t1 = 0.0;
+    double t0 = bload<double, 0>(grs64, row) * l_x[j * kBS], t1 = 0.0;
     const int q1 = pair0(j + 1);
     for (int q = pair0(j); q < q1; ++q) {
       const ValuePair<double> m = load_values<double>(mrs64, lane, q);
@@ -455,8 +467,8 @@ __global__ void __launch_bounds__(kBS, 4) k_cg(Args a)
   using StreamA = std::integral_constant<int, kStreamA>;
   using StreamM = std::integral_constant<int, PREC>; // A's own when there is none
   // One product: row j's sum of value * (gathered element of `src`, less
-  // `own` in difference form) is handed to finish(j, own, sum).
-  auto product = [&](auto stream, auto next, Rsrc src, auto own, auto finish) {
+  // its own in difference form) is handed to finish(j, own, diagonal, sum).
+  auto product = [&](auto stream, auto next, Rsrc src, auto own, auto diagonal, auto finish) {
     constexpr int S = decltype(stream)::value;
     using Acc = typename std::conditional<S == kStreamA, double, float>::type;
     constexpr bool DIFF = MIXED && S == kStreamA;
@@ -465,7 +477,7 @@ __global__ void __launch_bounds__(kBS, 4) k_cg(Args a)
       if (j < nsl) {
         const int32_t row = row_of(j);
         const int q1 = pair0(j + 1);
-        const T uv = own(j);
+        const T uv = own(j), gv = diagonal(j);
         Acc t0 = 0, t1 = 0;
         int c = pair0(j);
         do {
@@ -497,8 +509,8 @@ __global__ void __launch_bounds__(kBS, 4) k_cg(Args a)
                 t1 += __uint_as_float(w & 0xffff0000u) * x1[z];
               }
               else if constexpr (DIFF) { // padding: value 0, the row itself
-                t0 += (Acc)(m[z].x * (x0[z] - uv));
-                t1 += (Acc)(m[z].y * (x1[z] - uv));
+                t0 += (Acc)m[z].x * ((Acc)x0[z] - (Acc)uv);
+                t1 += (Acc)m[z].y * ((Acc)x1[z] - (Acc)uv);
               }
               else {
                 t0 += m[z].x * x0[z];
@@ -507,19 +519,19 @@ __global__ void __launch_bounds__(kBS, 4) k_cg(Args a)
             }
           c += CP;
         } while (c < q1);
-        finish(j, uv, t0 + t1);
+        finish(j, uv, gv, t0 + t1);
       }
   };
   // u = M r from the published r; partials u.r and u.s
   auto precondition = [&](double (&v)[2]) {
     v[0] = v[1] = 0.0;
     product(
-      StreamM{}, StreamA{}, rrs, [&](int j) { return r[j]; },
-      [&](int j, T rv, float t) {
-        const float u = t + bload<float, 0>(mds, row_of(j)) * (float)rv;
+      StreamM{}, StreamA{}, rrs, [&](int j) { return (T)r[j]; }, [&](int j) { return (T)bload<float, 0>(mds, row_of(j)); },
+      [&](int j, T rv, T g, float t) {
+        const float u = t + (float)g * (float)rv;
         di[DLDS ? 0 : j] = (T)u;
         bstore<float, kSc1>(urs, row_of(j), u);
-        v[0] += (double)u * (double)rv;
+        v[0] += (double)u * r[j];
         v[1] += (double)u * s[j];
       });
   };
@@ -539,16 +551,16 @@ __global__ void __launch_bounds__(kBS, 4) k_cg(Args a)
     for (int j = 0; j < R; ++j)
       if (j < nsl) {
         const double rd = residual(j), bd = bload<double, 0>(brs, row_of(j));
-        r[j] = (T)rd;
+        r[j] = rd;
         if constexpr (FLEX) {
-          bstore<T, kSc1>(rrs, row_of(j), r[j]);
+          bstore<T, kSc1>(rrs, row_of(j), (T)rd);
           v[1] += rd * rd;
           v[2] += bd * bd;
         }
         else {
           const T uv = get_u(j), mb = get_d(j) * (T)bd;
           bstore<T, kSc1>(urs, row_of(j), uv);
-          v[0] += (double)r[j] * (double)uv;
+          v[0] += r[j] * (double)uv;
           v[1] += norm == 2 ? (double)uv * (double)uv : rd * rd;
           v[2] += norm == 2 ? (double)mb * (double)mb : bd * bd;
         }
@@ -574,10 +586,10 @@ __global__ void __launch_bounds__(kBS, 4) k_cg(Args a)
 #pragma unroll
     for (int j = 0; j < R; ++j)
       if (j < nsl) {
-        r[j] = (T)bload<double, 0>(krs, row_of(j));
+        r[j] = bload<double, 0>(krs, row_of(j));
         set_p(j, bload<double, 0>(kps, row_of(j)));
         s[j] = bload<double, 0>(kss, row_of(j));
-        bstore<T, kSc1>(FLEX ? rrs : urs, row_of(j), FLEX ? r[j] : get_u(j));
+        bstore<T, kSc1>(FLEX ? rrs : urs, row_of(j), FLEX ? (T)r[j] : get_u(j));
       }
     double v[1] = { 0.0 };
     if (!team_sum<1>(bar, v))
@@ -595,11 +607,11 @@ __global__ void __launch_bounds__(kBS, 4) k_cg(Args a)
       // A
       double v1[1] = { 0.0 };
       product(
-        StreamA{}, StreamM{}, urs, get_u,
-        [&](int j, T uv, double t) {
+        StreamA{}, StreamM{}, urs, get_u, get_g,
+        [&](int j, T uv, T g, double t) {
           const double pj = (double)uv + beta * get_p(j);
           set_p(j, pj);
-          s[j] = (double)(dg[j] * uv) + t + beta * s[j];
+          s[j] = (double)g * (double)uv + t + beta * s[j];
           v1[0] += pj * s[j];
         });
       if (!team_sum<1>(bar, v1))
@@ -615,16 +627,16 @@ __global__ void __launch_bounds__(kBS, 4) k_cg(Args a)
 #pragma unroll
       for (int j = 0; j < R; ++j)
         if (j < nsl) {
-          r[j] = (T)((double)r[j] - alpha * s[j]);
+          r[j] -= alpha * s[j];
           if constexpr (FLEX) {
-            bstore<T, kSc1>(rrs, row_of(j), r[j]);
-            v2[1] += (double)r[j] * (double)r[j];
+            bstore<T, kSc1>(rrs, row_of(j), (T)r[j]);
+            v2[1] += r[j] * r[j];
           }
           else {
             const T uv = get_u(j);
             bstore<T, kSc1>(urs, row_of(j), uv);
-            v2[0] += (double)r[j] * (double)uv;
-            v2[1] += norm == 2 ? (double)uv * (double)uv : (double)r[j] * (double)r[j];
+            v2[0] += r[j] * (double)uv;
+            v2[1] += norm == 2 ? (double)uv * (double)uv : r[j] * r[j];
           }
           l_x[j * kBS] += alpha * get_p(j);
         }
@@ -643,9 +655,9 @@ __global__ void __launch_bounds__(kBS, 4) k_cg(Args a)
           for (int j = 0; j < R; ++j)
             if (j < nsl) {
               const double rd = residual(j);
-              r[j] = (T)rd;
+              r[j] = rd;
               if constexpr (FLEX)
-                bstore<T, kSc1>(rrs, row_of(j), r[j]);
+                bstore<T, kSc1>(rrs, row_of(j), (T)rd);
               v[0] += rd * rd;
             }
           if (!team_sum<1>(bar, v))
@@ -699,7 +711,7 @@ __global__ void __launch_bounds__(kBS, 4) k_cg(Args a)
           if (j < nsl) {
             const T uv = get_u(j);
             bstore<T, kSc1>(urs, row_of(j), uv);
-            v[0] += (double)r[j] * (double)uv;
+            v[0] += r[j] * (double)uv;
           }
         if (!team_sum<1>(bar, v))
           return;
@@ -748,7 +760,7 @@ __global__ void __launch_bounds__(kBS, 4) k_cg(Args a)
     for (int j = 0; j < R; ++j)
       if (j < nsl) {
         bstore<double, 0>(xrs, row_of(j), l_x[j * kBS]);
-        bstore<double, 0>(krs, row_of(j), (double)r[j]);
+        bstore<double, 0>(krs, row_of(j), r[j]);
         bstore<double, 0>(kps, row_of(j), get_p(j));
         bstore<double, 0>(kss, row_of(j), s[j]);
       }

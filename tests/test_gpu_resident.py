@@ -336,3 +336,60 @@ def test_random_numbering(afem_gpu, cell, n):
             r = s.solve(rtol=1e-8, **kw)
             assert np.linalg.norm(b - M @ s.solution().numpy()) <= 1.01e-8 * np.linalg.norm(b), (lam, kw)
             assert r.converged and not r.fallback
+
+
+def checkerboard_blocks(A, ns):
+    """Plane systems with 8x8 checkerboard conductivities from 0.1 to 10, boundary rows eliminated: one union."""
+    parts, lams, bnd = [], [], []
+    for k, n in enumerate(ns):
+        X, C = A.box_mesh(2, n, 0.2, seed=6 + k)
+        cell = np.minimum((X[C[:, :3]].mean(axis=1)[:, :2] * 8).astype(int), 7)
+        lams.append(np.exp(np.random.default_rng(k).uniform(np.log(0.1), np.log(10.0), 64))[cell[:, 1] * 8 + cell[:, 0]])
+        parts.append((X, C))
+        bnd.append(np.nonzero((X[:, :2] == 0.0).any(axis=1) | (X[:, :2] == 1.0).any(axis=1))[0])
+    X, C, offs = A.union_mesh(parts)
+    mesh = A.Mesh(2, X, C)
+    bsr = A.BSRFormat(mesh, 1, use_csr=True)
+    bsr.compute_sparsity()
+    s = A.DoFLinearSystem(X.shape[0])
+    bsr.assemble_laplace(A.DeviceArray.from_numpy(np.concatenate(lams)), 1.0, s.rhs())
+    s.set_bsr(bsr)
+    nodes = np.concatenate([b + o for b, o in zip(bnd, offs)]).astype(np.int32)
+    s.apply_dirichlet(A.DIRICHLET_ROW_ELIMINATION, nodes, 1, 0, 0.0, 0.0)
+    s.apply_matrix_transformation()
+    s.apply_rhs_transformation()
+    return s, offs, (mesh, bsr)
+
+
+def test_mixed_precision_takes_no_more_iterations_than_fp64(afem_gpu):
+    """Hard coefficients: the mixed solver's rounding neither delays it (2 %,
+    measured 0.4 %) nor leaves more error than FP64 PCG's stopping residual
+    does (ten times it: at the same residual the error moves by a few times
+    with the last iterations' rounding)."""
+    print("[case] mixed against FP64 iterations", flush=True)
+    A = afem_gpu
+    for n in (197, 250, 320):
+        s, offs, keep = checkerboard_blocks(A, [n])
+        s.solve(method=METHODS["fp64"], rtol=1e-11, max_iter=20000)
+        x = s.solution().numpy()
+        err, its = {}, {}
+        for m in ("fp64", "mixed"):
+            its[m] = s.solve(method=METHODS[m], rtol=1e-8, max_iter=20000).iterations
+            err[m] = np.linalg.norm(s.solution().numpy() - x) / np.linalg.norm(x)
+        print(f"[result] n={n} {its} {err}", flush=True)
+        assert its["mixed"] <= 1.02 * its["fp64"] + 3
+        assert err["mixed"] <= 10 * err["fp64"]
+
+
+def test_batch_takes_no_more_iterations_than_the_chunked_kernels(afem_gpu):
+    """What a caller's max_iter allowed them is enough for the default solve."""
+    print("[case] batch against chunked iterations", flush=True)
+    A = afem_gpu
+    s, offs, keep = checkerboard_blocks(A, [60, 197, 320, 250])
+    bs = A.BatchSolver(s, offs)
+    res, _ = bs.solve(rtol=1e-8, max_iter=20000)
+    bs.set_tiles(1, 1)
+    ref, _ = bs.solve(rtol=1e-8, max_iter=20000)
+    its = [(a.iterations, g.iterations) for a, g in zip(res, ref)]
+    print(f"[result] {its}", flush=True)
+    assert all(a <= 1.02 * g + 3 for a, g in its), its
