@@ -1913,12 +1913,29 @@ AFEM_API int afem_batch_solve(afem_batch_t b, const afem_batch_options* opt, afe
   AFEM_REQUIRE(opt->rtol >= 0.0 && opt->atol >= 0.0 && opt->max_iter >= 0, AFEM_ERR_ARGUMENT, "bad tolerances");
   AFEM_REQUIRE(opt->persistent >= 0 && opt->persistent <= 2, AFEM_ERR_ARGUMENT, "persistent must be 0, 1 or 2");
   const auto t0 = std::chrono::steady_clock::now();
-  bool on_chip = resident_usable(b, *opt);
-  if (on_chip) { // the values may have changed in place since the last solve
-    b->pack.valid64 = b->pack.valid32 = false;
-    resident::pack_values(b->pack, s->row_index, s->columns, s->values, true);
-  }
-  else
+  // another process holds part of the device, or the layout does not fit beside
+  // what it holds: the chunked kernels wait for nothing and need less; they
+  // solve with this pattern from now on
+  auto give_up = [&]() {
+    b->pack_pattern = s->pattern_count + 1;
+    b->pack_usable = false;
+    b->pack = resident::Pack();
+    b->rwork.release();
+    prepare(b);
+  };
+  bool tried = false;
+  bool on_chip = resident::unless_out_of_memory([&]() {
+    tried = true;
+    tried = resident_usable(b, *opt);
+    if (tried) { // the values may have changed in place since the last solve
+      b->pack.valid64 = b->pack.valid32 = false;
+      resident::pack_values(b->pack, s->row_index, s->columns, s->values, true);
+    }
+    return tried;
+  });
+  if (tried && !on_chip)
+    give_up();
+  else if (!on_chip)
     prepare(b);
   if (!opt->use_initial_guess) {
     hipLaunchKernelGGL(k_initial_guess, dim3(grid_for(s->nb_dof, 256)), dim3(256), 0, stream(), s->nb_dof,
@@ -1956,11 +1973,9 @@ AFEM_API int afem_batch_solve(afem_batch_t b, const afem_batch_options* opt, afe
     return any;
   };
   for (int round = 0; round < 5 && start(); ++round) {
-    if (on_chip && !run_resident(b, *opt, delta, want, iters)) {
-      // another process holds part of the device: the chunked kernels wait for
-      // nothing; they solve with this pattern from now on
-      on_chip = b->pack_usable = false;
-      b->pack = resident::Pack();
+    if (on_chip &&
+        !resident::unless_out_of_memory([&]() { return run_resident(b, *opt, delta, want, iters); })) {
+      on_chip = false;
       for (int k = 0; k < b->nb_seg; ++k) {
         const SegState z = b->host_st[k];
         if (z.active && z.done)
@@ -1970,7 +1985,7 @@ AFEM_API int afem_batch_solve(afem_batch_t b, const afem_batch_options* opt, afe
           nru[k] += z.nb_ru;
         }
       }
-      prepare(b);
+      give_up();
       if (!start())
         break;
     }

@@ -93,12 +93,34 @@ struct Work
   unsigned epoch = 0;      // largest epoch in the slots
   std::vector<int32_t> layout_rows;
   std::vector<Round> rounds;
+  void release() // the large arrays, when solves go another way
+  {
+    u.release();
+    keep.release();
+    xb.release();
+    slots.release();
+  }
   ~Work()
   {
     if (host)
       (void)hipHostFree(host);
   }
 };
+
+// run(), unless the memory for the layout, its values or the vectors is not
+// there: then false, before anything was launched on x.
+template <class F>
+bool unless_out_of_memory(const F& run)
+{
+  try {
+    return run();
+  }
+  catch (const Error& e) {
+    if (e.status != AFEM_ERR_OUT_OF_MEMORY)
+      throw;
+    return false;
+  }
+}
 
 // Runs the segments of w.host (inputs set, x the starting point) to their end;
 // w.host holds the results.  False: a barrier wait gave up (x is then some

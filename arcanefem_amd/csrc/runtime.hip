@@ -126,6 +126,8 @@ static void* device_malloc(size_t bytes)
     (void)hipGetLastError();
     pool_trim();
     e = hipMalloc(&p, bytes);
+    if (e != hipSuccess)
+      (void)hipGetLastError(); // a caller that does without goes on launching
   }
   AFEM_HIP(e);
   return p;

@@ -2240,13 +2240,20 @@ static int solve(afem_system* s, const afem_solver_options& o, afem_solve_result
     check_launch("initial_guess");
   }
   SolveTotals t;
-  bool on_chip = resident_usable(s, w, o);
-  if (on_chip && !solve_resident(s, w, o, t)) {
+  bool tried = false;
+  const bool on_chip = resident::unless_out_of_memory([&]() {
+    tried = true;
+    tried = resident_usable(s, w, o);
+    return tried && solve_resident(s, w, o, t);
+  });
+  if (tried && !on_chip) {
     // the device could not hold every workgroup at once (another process on
-    // it, say): the kernels that wait for nothing finish, and solve with this
-    // pattern from now on
-    on_chip = w->pack_usable = false;
+    // it, say), or the layout beside what it holds: the kernels that wait for
+    // nothing and need less finish, and solve with this pattern from now on
+    w->pack_valid = true;
+    w->pack_usable = false;
     w->pack = resident::Pack();
+    w->rwork.release();
   }
   if (!on_chip)
     solve_streaming(s, w, o, t);
