@@ -2126,6 +2126,19 @@ static bool solve_resident(afem_system* s, afem_solver_ws* w, const afem_solver_
   }
 }
 
+// The workspace as the format queries report it (null before the first use):
+// a resident solve needs no SpMV format, so it leaves the tuning to them.
+static afem_solver_ws* tuned_workspace(afem_system* s)
+{
+  afem_solver_ws* w = s->ws;
+  if (w && s->has_matrix && w->format < 0 && w->pack.valid64) {
+    w = workspace(s);
+    ensure_derived(s, w, false);
+    choose_format(s, w, 0);
+  }
+  return w;
+}
+
 // Every vector in memory, three to five kernels an iteration; adds to the
 // iterations that the totals already count.
 static void solve_streaming(afem_system* s, afem_solver_ws* w, const afem_solver_options& o, SolveTotals& out)
@@ -2628,10 +2641,8 @@ AFEM_API int afem_system_spmv_format(afem_system_t sys, int* format, int* lanes)
 {
   AFEM_GUARD_BEGIN
   AFEM_REQUIRE(sys && format && lanes, AFEM_ERR_ARGUMENT, "null argument");
-  afem_solver_ws* w = sys->ws;
-  // a resident solve alone has tuned nothing: its layout is SELL-64 in pairs
-  const bool pairs = w && w->format < 0 && w->pack.valid64;
-  *format = pairs ? (w->pack.idx16 && w->block == 1 ? kFmtSell16 : kFmtSell) : w ? w->format : -1;
+  afem_solver_ws* w = tuned_workspace(sys);
+  *format = w ? w->format : -1;
   *lanes = w ? w->lanes : 0;
   AFEM_GUARD_END
 }
@@ -2641,7 +2652,7 @@ AFEM_API int afem_system_spmv_tuning(afem_system_t sys, int* fp64_slots, int* fp
 {
   AFEM_GUARD_BEGIN
   AFEM_REQUIRE(sys && fp64_slots && fp64_block && fp32_slots && fp32_block, AFEM_ERR_ARGUMENT, "null argument");
-  afem_solver_ws* w = sys->ws;
+  afem_solver_ws* w = tuned_workspace(sys);
   const bool sell16 = w && (w->format == kFmtSell16 || w->format == kFmtSell16x8);
   *fp64_slots = sell16 ? (w->format == kFmtSell16x8 ? 8 : 4) : 0;
   *fp64_block = sell16 ? w->bs64 : 0;

@@ -444,7 +444,8 @@ AFEM_API int afem_system_set_spai(afem_system_t sys, const float* values);
 /* SpMV format the autotuner chose for the system's matrix: *format = 0 (CSR,
  * *lanes lanes per row, or per 3x3 block row when the matrix has blocks),
  * 1 (SELL-64), 2 (SELL-64 with 16-bit column offsets) or 3 (the same, 8
- * slots per step); -1 while no SpMV or solve has run on the current matrix. */
+ * slots per step); -1 while no SpMV or solve has run on the current matrix.
+ * A solve in one launch needs no format: the call then runs the autotuner. */
 AFEM_API int afem_system_spmv_format(afem_system_t sys, int* format, int* lanes);
 
 /* Kernel shape of the SELL-64 16-bit-offset SpMV (formats 2 and 3): slots per

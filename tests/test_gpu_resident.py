@@ -393,3 +393,27 @@ def test_batch_takes_no_more_iterations_than_the_chunked_kernels(afem_gpu):
     its = [(a.iterations, g.iterations) for a, g in zip(res, ref)]
     print(f"[result] {its}", flush=True)
     assert all(a <= 1.02 * g + 3 for a, g in its), its
+
+
+@pytest.mark.parametrize("offsets", [[1, 2, 70], [1, 33000, 40001]], ids=["near", "far"])
+def test_spmv_format_after_a_solve(afem_gpu, offsets):
+    """The format that is reported is the one that the products use."""
+    print(f"[case] spmv format after a solve {offsets}", flush=True)
+    A = afem_gpu
+    n = 70001
+    M = band(n, offsets, shift=0.3)
+    s, keep = device_system(A, M)
+    b = np.random.default_rng(1).normal(size=n)
+    s.rhs().upload(b)
+    assert s.spmv_format() is None
+    s.solve(rtol=1e-8)
+    x = s.solution().numpy()
+    fmt, tuning = s.spmv_format(), s.spmv_tuning()
+    assert fmt is not None
+    assert (tuning[0] != (0, 0)) == fmt[0].startswith("sell16"), (fmt, tuning)
+    y = A.DeviceArray(n, np.float64)
+    s.spmv(s.rhs(), y)
+    assert np.abs(y.numpy() - M @ b).max() <= 1e-12 * np.abs(M @ b).max()
+    assert s.spmv_format() == fmt and s.spmv_tuning() == tuning
+    s.solve(rtol=1e-8)
+    assert np.array_equal(s.solution().numpy(), x)
