@@ -42,9 +42,10 @@ struct Pack
 
 // Offsets of a pattern (rows rp, columns ci) cut into segments.  False: a
 // segment alone does not fit the device, a column leaves its segment, or the
-// layout pads too much.  `order` (device, may be null): a permutation of the
-// rows by locality, used when neighbouring rows have unrelated columns.
-// block 3 (one segment): rows and columns of nodes, nnz blocks.
+// layout pads too much.  `order` (device, may be null; one segment of scalar
+// rows): a permutation of the rows by locality, used when neighbouring rows
+// have unrelated columns.  block 3 (one segment): rows and columns of nodes,
+// nnz blocks.
 bool pack_pattern(Pack& p, int32_t n, int64_t nnz, const int32_t* rp, const int32_t* ci,
                   const std::vector<int32_t>& seg_rows, const int32_t* order = nullptr, int block = 1);
 // Values of the pattern's matrix: FP64, and with want32 the FP32 difference form too.

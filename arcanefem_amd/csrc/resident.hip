@@ -526,7 +526,7 @@ bool pack_pattern(Pack& p, int32_t n, int64_t nnz, const int32_t* rp, const int3
   // rows: 16.6 -> 9.9 us an iteration).  Numbered along a grid, the matrix
   // keeps its order: Morton order would read more lines.
   p.perm.release();
-  if (order && nseg == 1 && 2 * h[3] > p.nslice) {
+  if (order && nseg == 1 && block == 1 && 2 * h[3] > p.nslice) {
     p.perm.alloc((size_t)n);
     p.inv.reserve((size_t)n);
     AFEM_HIP(hipMemcpyAsync(p.perm.p, order, sizeof(int32_t) * (size_t)n, hipMemcpyDeviceToDevice, stream()));
@@ -723,11 +723,9 @@ bool solve(const Pack& p, Work& w, const Options& o, double* x, const double* b)
     w.xb.reserve(2 * dofs);
     a.x = w.xb.p;
     a.b = w.xb.p + dofs;
-    if (p.block == 3)
-      permute_blocks(p.n, p.perm.p, x, b, w.xb.p, w.xb.p + dofs);
-    else
-      hipLaunchKernelGGL(k_permute_in, dim3(grid_for(p.n, 256)), dim3(256), 0, stream(), p.n, p.perm.p, x, b, w.xb.p,
-                         w.xb.p + dofs);
+    ProfScope prof("resident_reorder");
+    hipLaunchKernelGGL(k_permute_in, dim3(grid_for(p.n, 256)), dim3(256), 0, stream(), p.n, p.perm.p, x, b, w.xb.p,
+                       w.xb.p + dofs);
     check_launch("permute_in");
   }
   a.u = w.u.p;
@@ -764,9 +762,7 @@ bool solve(const Pack& p, Work& w, const Options& o, double* x, const double* b)
       else
         launch_f64(a, r.rows_per_wave, p.idx16, r.grid, lds);
     }
-    if (p.perm.p && p.block == 3)
-      unpermute_blocks(p.n, p.perm.p, a.x, x);
-    else if (p.perm.p) {
+    if (p.perm.p) {
       hipLaunchKernelGGL(k_permute_out, dim3(grid_for(p.n, 256)), dim3(256), 0, stream(), p.n, p.perm.p, a.x, x);
       check_launch("permute_out");
     }

@@ -574,18 +574,16 @@ constexpr int kFillWaves = 4;
 
 template <bool WANT32>
 __global__ void __launch_bounds__(kFillWaves* kWave)
-k_block_values(int32_t n, const int32_t* __restrict__ perm, const int32_t* __restrict__ rp,
-               const int32_t* __restrict__ ci, const double* __restrict__ v, const int32_t* __restrict__ poff,
-               const int32_t* __restrict__ src, double* __restrict__ v64, double* __restrict__ diag64,
-               double* __restrict__ dinv64, float* __restrict__ v32, float* __restrict__ diag32,
-               float* __restrict__ dinv32)
+k_block_values(int32_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ ci,
+               const double* __restrict__ v, const int32_t* __restrict__ poff, double* __restrict__ v64,
+               double* __restrict__ diag64, double* __restrict__ dinv64, float* __restrict__ v32,
+               float* __restrict__ diag32, float* __restrict__ dinv32)
 {
   __shared__ double s_sum[kFillWaves][9][kWave];
   const int32_t s = blockIdx.x;
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  const int32_t i = s * kWave + lane;
-  const int32_t row = i < n ? (perm ? perm[i] : i) : -1;
-  const int32_t b = row >= 0 ? rp[row] : 0, e = row >= 0 ? rp[row + 1] : 0;
+  const int32_t row = s * kWave + lane;
+  const int32_t b = row < n ? rp[row] : 0, e = row < n ? rp[row + 1] : 0;
   double sum[9] = {};
   int32_t k = b;
   auto next = [&]() -> int32_t { // position of the row's next off-diagonal block
@@ -600,17 +598,10 @@ k_block_values(int32_t n, const int32_t* __restrict__ perm, const int32_t* __res
   const int w = poff[s + 1] - poff[s];
   for (int q = 0; q < w; ++q) {
     int2 f;
-    if (src) {
-      if (q % kFillWaves != wave)
-        continue;
-      f = reinterpret_cast<const int2*>(src)[(at + q) * kWave + lane];
-    }
-    else {
-      f.x = next();
-      f.y = next();
-      if (q % kFillWaves != wave)
-        continue;
-    }
+    f.x = next();
+    f.y = next();
+    if (q % kFillWaves != wave)
+      continue;
     double m[18];
 #pragma unroll
     for (int c = 0; c < 9; ++c) {
@@ -680,46 +671,12 @@ k_block_values(int32_t n, const int32_t* __restrict__ perm, const int32_t* __res
 
 void fill_block_values(const Pack& p, const int32_t* rp, const int32_t* ci, const double* v, bool want32)
 {
-  const int32_t* src = p.perm.p ? p.src.p : nullptr;
   if (want32)
-    hipLaunchKernelGGL(k_block_values<true>, dim3(p.nslice), dim3(kFillWaves * kWave), 0, stream(), p.n, p.perm.p, rp,
-                       ci, v, p.poff.p, src, p.v64.p, p.diag64.p, p.dinv64.p, p.v32.p, p.diag32.p, p.dinv32.p);
+    hipLaunchKernelGGL(k_block_values<true>, dim3(p.nslice), dim3(kFillWaves * kWave), 0, stream(), p.n, rp, ci, v,
+                       p.poff.p, p.v64.p, p.diag64.p, p.dinv64.p, p.v32.p, p.diag32.p, p.dinv32.p);
   else
-    hipLaunchKernelGGL(k_block_values<false>, dim3(p.nslice), dim3(kFillWaves * kWave), 0, stream(), p.n, p.perm.p,
-                       rp, ci, v, p.poff.p, src, p.v64.p, p.diag64.p, p.dinv64.p, (float*)nullptr, (float*)nullptr,
-                       (float*)nullptr);
-}
-
-__global__ void k_permute_blocks(int32_t dofs, const int32_t* __restrict__ perm, const double* __restrict__ x,
-                                 const double* __restrict__ b, double* __restrict__ xp, double* __restrict__ bp)
-{
-  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < dofs) {
-    const int64_t from = 3 * (int64_t)perm[i / 3] + i % 3;
-    xp[i] = x[from];
-    bp[i] = b[from];
-  }
-}
-
-__global__ void k_unpermute_blocks(int32_t dofs, const int32_t* __restrict__ perm, const double* __restrict__ xp,
-                                   double* __restrict__ x)
-{
-  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < dofs)
-    x[3 * (int64_t)perm[i / 3] + i % 3] = xp[i];
-}
-
-void permute_blocks(int32_t n, const int32_t* perm, const double* x, const double* b, double* xp, double* bp)
-{
-  hipLaunchKernelGGL(k_permute_blocks, dim3(grid_for(3 * (int64_t)n, 256)), dim3(256), 0, stream(), 3 * n, perm, x, b,
-                     xp, bp);
-}
-
-void unpermute_blocks(int32_t n, const int32_t* perm, const double* xp, double* x)
-{
-  hipLaunchKernelGGL(k_unpermute_blocks, dim3(grid_for(3 * (int64_t)n, 256)), dim3(256), 0, stream(), 3 * n, perm, xp,
-                     x);
-  check_launch("unpermute_blocks");
+    hipLaunchKernelGGL(k_block_values<false>, dim3(p.nslice), dim3(kFillWaves * kWave), 0, stream(), p.n, rp, ci, v,
+                       p.poff.p, p.v64.p, p.diag64.p, p.dinv64.p, (float*)nullptr, (float*)nullptr, (float*)nullptr);
 }
 
 } // namespace resident

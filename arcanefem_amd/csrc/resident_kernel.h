@@ -790,8 +790,6 @@ constexpr int kBlockWaves = kBlockBS / kWave;
 constexpr int kBlockRowSteps[3] = { 1, 2, 4 };
 void launch_block(const Args& a, bool mixed, int rows, bool idx16, int grid);
 void fill_block_values(const Pack& p, const int32_t* rp, const int32_t* ci, const double* v, bool want32);
-void permute_blocks(int32_t n, const int32_t* perm, const double* x, const double* b, double* xp, double* bp);
-void unpermute_blocks(int32_t n, const int32_t* perm, const double* xp, double* x);
 
 template <class T, int PREC, bool I16>
 inline void launch_kernel(const Args& a, int rows, int grid, size_t lds)

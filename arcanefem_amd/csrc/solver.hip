@@ -2064,7 +2064,10 @@ static bool resident_usable(afem_system* s, afem_solver_ws* w, const afem_solver
     return false;
   if (!w->pack_valid) {
     const int32_t n = s->nb_dof / s->block;
-    const int32_t* order = s->bsr && s->bsr->border.n == (size_t)n ? s->bsr->border.p : nullptr;
+    // an order there is only after an assembly with a brick plan: Laplace and
+    // heat of triangles and tetrahedra
+    const int32_t* order =
+      s->block == 1 && s->bsr && s->bsr->border.n == (size_t)n ? s->bsr->border.p : nullptr;
     w->pack_usable = resident::pack_pattern(w->pack, n, s->nnz / (s->block * s->block), s->row_index, s->columns,
                                             { 0, n }, order, s->block);
     w->pack_valid = true;

@@ -333,7 +333,13 @@ def test_random_numbering(afem_gpu, cell, n):
         rid = np.repeat(np.arange(Y.shape[0]), np.diff(row))
         s.set_spai(A.DeviceArray.from_numpy(np.where(col == rid, 1.0 / d[rid], 0.0).astype(np.float32)))
         for kw in (dict(method=0), dict(method=1), dict(method=3, precond_bf16=0), dict(method=3, precond_bf16=1)):
+            A.profile_enable(True)
+            A.profile_reset()
             r = s.solve(rtol=1e-8, **kw)
+            reordered = A.profile_query("resident_reorder")[0]
+            A.profile_reset()
+            A.profile_enable(False)
+            assert reordered == (1 if Y.shape[0] > 64 else 0), (lam, kw)  # one slice gathers from few lines anyway
             assert np.linalg.norm(b - M @ s.solution().numpy()) <= 1.01e-8 * np.linalg.norm(b), (lam, kw)
             assert r.converged and not r.fallback
 

@@ -82,7 +82,7 @@ def check(A, X, C, mixed, rtol, norm=0):
 
 # nodes: 12; 64 (one slice); 60 and 80; 1331 (three workgroups' worth of
 # waves); 129360 (one slice per wave), 132651 (the first that need two),
-# 274625 (four); numbered at random: in Morton order
+# 274625 (four)
 SIZES = {"least": (2, 1, 1), "slice": (3, 3, 3), "below": (2, 3, 4), "above": (3, 3, 4), "small": (10, 10, 10),
          "one": (55, 41, 54), "two": (50, 50, 50), "four": (64, 64, 64)}
 
@@ -98,6 +98,7 @@ def test_sizes(afem_gpu, name, mixed):
 @pytest.mark.parametrize("mixed", [False, True], ids=["fp64", "mixed"])
 @pytest.mark.parametrize("counts", [(12, 9, 11), (40, 36, 38)])
 def test_random_numbering(afem_gpu, counts, mixed):
+    """Rows of unrelated columns next to each other, solved in the order they have."""
     print(f"[case] resident blocks shuffled {counts} mixed={mixed}", flush=True)
     X, C = grid_mesh(counts, shuffled=True)
     check(afem_gpu, X, C, mixed, 1e-8)
