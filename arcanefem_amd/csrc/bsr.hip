@@ -3140,7 +3140,7 @@ k_node_sum(int32_t nb_node, const int32_t* __restrict__ nc_off, const int32_t* _
       *r = s;
     else if constexpr (MODE == kNodeAdd)
       *r += s;
-    else
+    else if (nc_off[i] < nc_off[i + 1]) // the field of a node without cells counts nowhere, whatever it holds
       *r += (s + field[i] * scale * w) * factor;
   }
 }

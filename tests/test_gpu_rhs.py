@@ -76,3 +76,24 @@ def test_sources_and_mass(afem_gpu, name):
         A.check(A.lib().afem_rhs_body_force(m.h, A._ptr(f), got.c))
         ref = O.rhs_body_force(X, C, f)
         assert np.abs(got.numpy() - ref).max() <= 1e-13 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("name", ["tri_5", "tet_4", "quad_4", "hexa_3"])
+def test_nodes_without_cells(afem_gpu, name):
+    """Unused nodes get nothing, also where the field is not a number."""
+    A = afem_gpu
+    print(f"[case] rhs unused nodes {name}", flush=True)
+    dim, X, C = meshes(A, name)
+    npc = 8 if C.shape[1] == 8 else 3 if name.startswith("tri") else 4
+    N = X.shape[0]
+    Y = np.concatenate([[[9.0, 9.0, 0.0]], X, np.full((2, 3), 7.0) * [1.0, 1.0, 0.0]])
+    m = A.Mesh(dim, Y, np.where(C >= 0, C + 1, -1).astype(np.int32), npc=npc)
+    rng = np.random.default_rng(0)
+    u, r0 = rng.normal(size=N), rng.normal(size=N + 3)
+    field = np.concatenate([[np.nan], u, [np.inf, -np.inf]])
+    got = A.DeviceArray.from_numpy(r0)
+    A.rhs_mass_field(m, A.DeviceArray.from_numpy(field), 3.0, got)
+    ref = O.rhs_mass_field(X, C, npc, u, 3.0, rhs=r0[1:-2].copy(), dim=dim)
+    out = got.numpy()
+    assert np.array_equal(out[[0, -2, -1]], r0[[0, -2, -1]])
+    assert np.abs(out[1:-2] - ref).max() <= 1e-13 * max(1.0, np.abs(ref).max())
