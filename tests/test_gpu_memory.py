@@ -118,3 +118,45 @@ def test_threads(afem_gpu):
     for t in th:
         t.join()
     assert not errors
+
+
+@pytest.mark.parametrize("where", ["same thread, relaxed", "other thread, relaxed", "other thread, thread_local"])
+def test_releases_during_a_capture(afem_gpu, where):
+    """Another stream is being captured in a mode that allows allocations: a
+    released object leaves the capture valid, and the graph replays."""
+    print(f"[case] release during a capture: {where}", flush=True)
+    A = afem_gpu
+    n = 1 << 20
+    x = torch.zeros(n, device="cuda")
+    g = torch.cuda.CUDAGraph()
+    held = []
+
+    def work():
+        held.clear()  # releases blocks that are kept
+        gc.collect()
+        held.append(A.DoFLinearSystem(n))  # and asks for them again
+        held.append(A.DoFLinearSystem(n + 4096))  # these are new
+
+    for _ in range(2):
+        work()
+    A.check(A.lib().afem_synchronize())
+    torch.cuda.synchronize()
+    gc.disable()
+    try:
+        with torch.cuda.graph(g, capture_error_mode=where.split(", ")[1]):
+            x += 1.0
+            if where.startswith("other"):
+                t = threading.Thread(target=work)
+                t.start()
+                t.join()
+            else:
+                work()
+            x += 2.0
+    finally:
+        gc.enable()
+    for k in range(3):
+        g.replay()
+        held[0].rhs().upload(np.full(n, float(k)))
+        torch.cuda.synchronize()
+        assert float(x[0]) == 3.0 * (k + 1) and float(x[-1]) == 3.0 * (k + 1)
+        assert held[0].rhs().numpy()[-1] == k
