@@ -676,6 +676,8 @@ class BatchSolver:
         check(lib().afem_batch_set_tiles(self.h, lanes, tiles))
 
     def autotune(self):
+        """(lanes, tiles, ms per iteration) of the fastest shape of the chunked
+        kernels, kept for the solves that run them (set_tiles makes them do so)."""
         lanes, tiles, ms = ctypes.c_int(), ctypes.c_int(), ctypes.c_double()
         check(lib().afem_batch_autotune(self.h, ctypes.byref(lanes), ctypes.byref(tiles), ctypes.byref(ms)))
         return lanes.value, tiles.value, ms.value

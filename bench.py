@@ -291,8 +291,7 @@ def batch_section(A, args):
 
     variant, _ = bsr.autotune_assembly()  # times the variants with lambda = 1: assemble afterwards
     assemble()
-    lanes, tiles, it_ms = bs.autotune()
-    warm, _ = bs.solve(raise_on_failure=False, rtol=1e-8, max_iter=args.batch_max_iter)  # graph instantiation
+    warm, _ = bs.solve(raise_on_failure=False, rtol=1e-8, max_iter=args.batch_max_iter)  # builds its layout
     for k, r in enumerate(warm):
         if not r.converged:
             log(f"[bench] batch: system {k} (n={ns[k]}) not converged: {r.iterations} it, relres {r.relres:.2e}")
@@ -337,7 +336,6 @@ def batch_section(A, args):
         "iterations_max": int(max(its)), "iterations_mean": float(np.mean(its)),
         "converged": int(sum(r.converged for r in res)),
         "relres_max": float(max(r.relres for r in res)),
-        "tuned": {"lanes": lanes, "tiles": tiles, "ms_per_iteration": it_ms},
         "dofs_per_s": N / ((asm_ms + sol_ms) * 1e-3),
         "solver": "teams of resident workgroups, one launch for as many systems as fit the device together",
         "persistent": {"solve_ms": pers_ms, "iterations_max": int(max(r.iterations for r in pers_res)),

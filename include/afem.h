@@ -559,7 +559,9 @@ AFEM_API int afem_batch_destroy(afem_batch_t batch);
  * 256-row strips per workgroup (1..16).  The batch's default solves use the
  * chunked kernels with this shape from then on. */
 AFEM_API int afem_batch_set_tiles(afem_batch_t batch, int lanes, int tiles);
-/* Times the (lanes, tiles) candidates on one chunk and keeps the fastest. */
+/* Times the (lanes, tiles) candidates on one chunk and keeps the fastest for
+ * the solves that run the chunked kernels.  It does not make them do so:
+ * afem_batch_set_tiles does. */
 AFEM_API int afem_batch_autotune(afem_batch_t batch, int* lanes, int* tiles, double* ms_per_iteration);
 /* Solves every system; results [host] nb_segment entries (may be NULL).
  * AFEM_ERR_NOT_CONVERGED when a system misses the tolerance;
