@@ -9,9 +9,9 @@
 // by the stream (64 MB from the memory-side cache) and two barriers of 2.9 us.
 // Block-Jacobi PCG, three kernels an iteration -> resident: 48 x 45 x 50 hexes
 // of six tetrahedra (115 thousand nodes) mixed to 1e-8 1196 iterations of 30.3
-// us -> 1179 of 16.2, with the copies of the values 36.3 -> 19.1 ms; the same
-// in FP64 25.2 us an iteration; 9261 nodes mixed 8.5; 358 thousand nodes mixed
-// 41, FP64 88 (4.5 TB/s).  Three pairs a chunk (two in FP64) spill at four
+// us -> 1060 of 16.4, with the copies of the values 37.2 -> 17.7 ms; the same
+// in FP64 25.2 us an iteration; 9261 nodes mixed 8.7; 358 thousand nodes mixed
+// 41.5, FP64 88 (4.5 TB/s).  Three pairs a chunk (two in FP64) spill at four
 // nodes a lane: 43 and 127.
 #include "resident_kernel.h"
 
@@ -119,10 +119,10 @@ __device__ __forceinline__ void store3(Rsrc r, int32_t node, const T (&v)[3])
 // ---- the kernel -------------------------------------------------------------------------------------
 
 // Phases A and B and the mixed mode as in k_cg.  r, u, s and up to two nodes'
-// D^-1 are in registers, x and p in LDS; r is FP64 in the mixed mode too (with
-// r in FP32 and exact sums 1273 iterations instead of 1179 at 115 thousand
-// nodes); the diagonal blocks (and D^-1 beyond
-// two nodes a lane) come with the stream.
+// D^-1 are in registers, x and p in LDS; in the mixed mode too r is FP64 and the
+// terms of w are exact, differences and products (115 thousand nodes: FP64's
+// 1060 iterations; differences rounded to FP32 1179, r as well 1273); the
+// diagonal blocks (and D^-1 beyond two nodes a lane) come with the stream.
 template <class T, int R, bool I16>
 __global__ void __launch_bounds__(kBlockBS, 2) k_cg_block(Args a)
 {
@@ -362,19 +362,18 @@ __global__ void __launch_bounds__(kBlockBS, 2) k_cg_block(Args a)
 #pragma unroll
           for (int z = 0; z < CP; ++z)
             if (z < cnt) {
-              if constexpr (MIXED) { // difference form; padding: value 0, the node itself
+              double d0[3], d1[3]; // mixed: difference form; padding: value 0, the node itself
 #pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                  x0[z][c] -= u[j][c];
-                  x1[z][c] -= u[j][c];
-                }
+              for (int c = 0; c < 3; ++c) {
+                d0[c] = MIXED ? (double)x0[z][c] - (double)u[j][c] : (double)x0[z][c];
+                d1[c] = MIXED ? (double)x1[z][c] - (double)u[j][c] : (double)x1[z][c];
               }
 #pragma unroll
               for (int c = 0; c < 3; ++c)
 #pragma unroll
                 for (int e = 0; e < 3; ++e) {
-                  t[c] = fma((double)m[z][3 * c + e], (double)x0[z][e], t[c]);
-                  t[c] = fma((double)m[z][9 + 3 * c + e], (double)x1[z][e], t[c]);
+                  t[c] = fma((double)m[z][3 * c + e], d0[e], t[c]);
+                  t[c] = fma((double)m[z][9 + 3 * c + e], d1[e], t[c]);
                 }
             }
           q += CP;
