@@ -20,7 +20,7 @@
 //
 // By default the solve runs in the resident kernel (resident.hip) instead,
 // every system a team of workgroups of one launch: 24 systems of 2 to 103
-// thousand rows to 1e-8, assembly included, 83.6 -> 20.4 ms.
+// thousand rows to 1e-8, assembly included, 83.6 -> 17.6 ms.
 //
 // Tuning: lanes per row (G) and row tiles per workgroup (T) are timed on
 // the batch and the fastest pair is kept; G = 1 selects a SELL-64 copy of

@@ -11,7 +11,7 @@
 // tetrahedra numbered at random (112 thousand rows) 22 -> 11.3 us.  Mixed
 // Jacobi-PCG on 128^3 hexes of six tetrahedra (2.15 million rows) to 1e-8
 // 84.9 -> 34.8 ms; flexible PCG with a BF16 sparse preconditioner on 0.89
-// million rows, assembly and inference included, 61.6 -> 25.3 ms.
+// million rows, assembly and inference included, 61.7 -> 24.7 ms.
 #include "resident_kernel.h"
 
 #include <algorithm>

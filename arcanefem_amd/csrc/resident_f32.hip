@@ -1,4 +1,4 @@
-// resident_f32.hip -- the resident conjugate-gradient kernels with FP32 vectors.
+// resident_f32.hip -- the resident conjugate-gradient kernels of the mixed solver.
 #include "resident_kernel.h"
 
 namespace afem {

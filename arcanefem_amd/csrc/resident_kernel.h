@@ -10,7 +10,8 @@ namespace resident {
 // One workgroup per CU, 1024 threads of 128 registers: against 512 threads of
 // 256 registers twice the waves hide the gathers' latency (24 systems of
 // triangles 12.9 -> 10.3 us an iteration, 227 thousand rows of tetrahedra
-// FP64 13.4 -> 11.6, 2.15 million rows mixed 42.8 -> 40.4), at the price of
+// FP64 13.4 -> 11.6, 2.15 million rows mixed 42.8 -> 40.4, with the mixed
+// solver's terms still rounded to FP32), at the price of
 // some spills at 9 slices per wave.
 constexpr int kBS = 1024;
 constexpr int kWaves = kBS / kWave;
@@ -304,10 +305,11 @@ __device__ __forceinline__ IndexPair<I16> load_offsets(Rsrc r, int lane, int q)
 // what it loses stays in s.  With r and the products in FP32 the residual of a
 // late reliable update differed from the recursive one by up to 0.4 %, which
 // cost iterations and left more error at the same residual: checkerboard of
-// 509 x 509 quads 4954 iterations, now 3320; log-normal cube of 128^3 hexes
-// 1724 (x error 1e-9), now 1449 (6e-12; FP64 PCG takes 1448).  The price at 9
-// slices per wave is 40.8 -> 41.2 us an iteration at 2.15 million rows; at 5
-// there is none (16.8, 16.5 at 0.53 million).
+// 509 x 509 quads 4994 iterations, now 3320 (FP64 r alone: 4954); log-normal
+// cube of 128^3 hexes 1572 (x error 1e-9; FP64 r alone 1724), now 1449 (6e-12;
+// FP64 PCG takes 1448).  The price at 9 slices per wave is 40.8 -> 41.2 us an
+// iteration at 2.15 million rows; at 5 there is none (16.8, 16.5 at 0.53
+// million).
 //
 // With a sparse preconditioner (PREC 32 or 16: its values FP32 or BF16) B
 // publishes r, and a third phase forms u = M r, published, and the partials
@@ -526,7 +528,8 @@ __global__ void __launch_bounds__(kBS, 4) k_cg(Args a)
   auto precondition = [&](double (&v)[2]) {
     v[0] = v[1] = 0.0;
     product(
-      StreamM{}, StreamA{}, rrs, [&](int j) { return (T)r[j]; }, [&](int j) { return (T)bload<float, 0>(mds, row_of(j)); },
+      StreamM{}, StreamA{}, rrs, [&](int j) { return (T)r[j]; },
+      [&](int j) { return (T)bload<float, 0>(mds, row_of(j)); },
       [&](int j, T rv, T g, float t) {
         const float u = t + (float)g * (float)rv;
         di[DLDS ? 0 : j] = (T)u;

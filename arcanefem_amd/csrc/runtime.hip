@@ -58,7 +58,7 @@ void ensure_init()
 // ---- device memory --------------------------------------------------------------
 //
 // hipMalloc and hipFree of the buffers of a mesh, a matrix or a system take as
-// long as the kernels that fill them: the plans of 61 x 57 x 64 hexes of six
+// long as the kernels that fill them: the plans of 61 x 57 x 66 hexes of six
 // tetrahedra were 10 allocations of 50-75 us and a release of 1 ms, more than
 // a third of the time from a mesh to its assembled matrix (3.7 ms a pass, 1.46
 // without them; the first of a process 2.2 and 1.55).  Released blocks are
