@@ -509,15 +509,16 @@ AFEM_API int afem_spai_inspect(afem_spai_t spai, int what, float* out, int64_t c
  * Independent scalar systems that are the diagonal blocks of one system's
  * matrix (e.g. the Laplace matrix of a disjoint union of meshes, assembled in
  * one launch by afem_bsr_assemble_laplace).  They are solved together by
- * mixed-precision Jacobi PCG with per-system scalars: FP32 matrix and vectors,
- * FP64 x, FP64 reliable-update residual deciding convergence.  By default
+ * mixed-precision Jacobi PCG with per-system scalars: FP32 matrix, FP64
+ * x, FP64 reliable-update residual deciding convergence.  By default
  * every system is a team of workgroups of one launch that keeps its vectors
  * in registers and LDS (further launches for systems that do not fit beside
  * the others).  Systems too large for that, thousands of tiny ones, and
  * batches whose tiles were set run chunks of iterations of ordinary kernels
- * captured in a hipGraph and replayed.  Or one persistent kernel launch (captured in a hipGraph and
- * replayed) in which every system gets a team of resident workgroups that
- * synchronize through bounded barrier waits in device memory. */
+ * captured in a hipGraph and replayed.  Or one persistent kernel launch
+ * (captured in a hipGraph and replayed) in which every system gets a team of
+ * resident workgroups that synchronize through bounded barrier waits in device
+ * memory. */
 typedef struct afem_batch* afem_batch_t;
 typedef struct afem_batch_options {
   double rtol;            /* per system: ||b_s - A_s x_s|| <= max(rtol ||b_s||, atol) */
